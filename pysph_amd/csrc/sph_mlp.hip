@@ -58,21 +58,21 @@ static Layout layout() {
 }
 
 // ---------------------------------------------------------------------------
-// GEMM: C[M x N] = op(A)[M x K] op(B)[K x N], BF16 operands, FP32 accumulate.
-// A(m,k) = TA ? A[k*lda + m] : A[m*lda + k];  B(k,n) = TB ? B[n*ldb + k] : B[k*ldb + n].
-// Block tile 64 x 64 (four 32 x 32 wave tiles), K in steps of 16.  Split-K:
-// block z reduces k in [z*kc, (z+1)*kc) and writes its own partial slab.
+// GEMM: C[M x N] = A[M x K] B[K x N] with B stored transposed ([N x K]), BF16
+// operands, FP32 accumulate.  Block tile 64 x 64 (four 32 x 32 wave tiles).
 // ---------------------------------------------------------------------------
 struct GemmArgs {
-  int M, N, K, kc;
+  int M, N, K;
   const __bf16* A;
   int64_t lda;
   const __bf16* B;
   int64_t ldb;
   float* C;            // FP32 output (may be null)
   int64_t ldc;
-  int64_t c_zstride;   // split-K: slab z at C + z * c_zstride
   int accumulate;      // C += result
+  float* C2;           // K = 128: when set, columns from n2 on are written here instead
+  int64_t ldc2;        // of C (never accumulated)
+  int n2;              // a multiple of 64: no block tile straddles it
   const float* bias;   // [N] or null
   int relu;
   float* U;            // activation before the residual (null: not stored)
@@ -83,65 +83,23 @@ struct GemmArgs {
   int64_t ldcb;
 };
 
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wm = w & 1, wn = w >> 1;
-  const int row = blockIdx.y * 64 + wm * 32 + (lane & 31);   // A row of this lane
-  const int col = blockIdx.x * 64 + wn * 32 + (lane & 31);   // B column of this lane
-  const int kh = 8 * (lane >> 5);
-  const int k_begin = blockIdx.z * g.kc;
-  const int k_end = min(g.K, k_begin + g.kc);
-  f32x16 acc = {};
-  const bool rok = row < g.M, cok = col < g.N;
-  for (int k0 = k_begin; k0 < k_end; k0 += 16) {
-    bf16x8 a, b;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int k = k0 + kh + i;
-      const bool kok = k < k_end;
-      a[i] = (rok && kok) ? (TA ? g.A[(int64_t)k * g.lda + row] : g.A[(int64_t)row * g.lda + k])
-                          : (__bf16)0.f;
-      b[i] = (cok && kok) ? (TB ? g.B[(int64_t)col * g.ldb + k] : g.B[(int64_t)k * g.ldb + col])
-                          : (__bf16)0.f;
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-  }
-  float* C = g.C ? g.C + (int64_t)blockIdx.z * g.c_zstride : nullptr;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int orow = blockIdx.y * 64 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-    const int ocol = col;
-    if (orow >= g.M || ocol >= g.N) continue;
-    float v = acc[r];
-    if (g.bias) v += g.bias[ocol];
-    if (g.relu) v = fmaxf(v, 0.f);
-    if (g.U) g.U[(int64_t)orow * g.ldu + ocol] = v;
-    if (g.res) v += g.res[(int64_t)orow * g.ldr + ocol];
-    if (C) {
-      float* p = C + (int64_t)orow * g.ldc + ocol;
-      if (g.accumulate) v += *p;
-      *p = v;
-    }
-    if (g.Cb) g.Cb[(int64_t)orow * g.ldcb + ocol] = (__bf16)v;
-  }
-}
-
 // Epilogue of the A B^T product with its loads issued ahead: the bias value
 // of the lane's column once, and the residual and accumulated values of all
 // 16 output elements before the first store, so that their latencies overlap
 // (per element, each load would be waited for in turn).  Rows and columns
-// past the matrix read row / column 0 and are not stored.  The arithmetic is
-// that of `gemm_kernel`'s epilogue, in the same order.
+// past the matrix read row / column 0 and are not stored.  (v + bias, ReLU,
+// U, + residual, + accumulated value, C, BF16 copy, in that order.)
 struct EpiIn {
   int rows[16];  // output row of element r, -1 when outside the matrix
   float bv, rv[16], cv[16];
 };
 
+template <bool SPLIT = false>
 __device__ __forceinline__ void epi_load(const GemmArgs& g, int orow0, int col, int lane,
                                          EpiIn& in) {
   const bool cok = col < g.N;
   const int ccol = cok ? col : 0;
+  const bool acc = g.accumulate && !(SPLIT && col >= g.n2);
   in.bv = 0.f;
   if (g.bias) in.bv = g.bias[ccol];
 #pragma unroll
@@ -154,15 +112,19 @@ __device__ __forceinline__ void epi_load(const GemmArgs& g, int orow0, int col, 
     for (int r = 0; r < 16; ++r)
       in.rv[r] = g.res[(int64_t)(in.rows[r] < 0 ? 0 : in.rows[r]) * g.ldr + ccol];
   }
-  if (g.C && g.accumulate) {
+  if (g.C && acc) {
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       in.cv[r] = g.C[(int64_t)(in.rows[r] < 0 ? 0 : in.rows[r]) * g.ldc + ccol];
   }
 }
 
+template <bool SPLIT = false>
 __device__ __forceinline__ void epi_store(const GemmArgs& g, const f32x16& acc, int col,
                                           const EpiIn& in) {
+  const bool second = SPLIT && col >= g.n2;  // uniform over the block
+  float* C = second ? g.C2 - g.n2 : g.C;
+  const int64_t ldc = second ? g.ldc2 : g.ldc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     float v = acc[r];
@@ -171,78 +133,45 @@ __device__ __forceinline__ void epi_store(const GemmArgs& g, const f32x16& acc, 
     const bool ok = in.rows[r] >= 0;
     if (g.U && ok) g.U[(int64_t)in.rows[r] * g.ldu + col] = v;
     if (g.res) v += in.rv[r];
-    if (g.C) {
-      if (g.accumulate) v += in.cv[r];
-      if (ok) g.C[(int64_t)in.rows[r] * g.ldc + col] = v;
+    if (C) {
+      if (g.accumulate && !second) v += in.cv[r];
+      if (ok) C[(int64_t)in.rows[r] * ldc + col] = v;
     }
     if (g.Cb && ok) g.Cb[(int64_t)in.rows[r] * g.ldcb + col] = (__bf16)v;
   }
 }
 
-// k-steps whose fragments are loaded before their MFMAs
-constexpr int kGemmChunk = 8;
-
-// C = A B^T-stored: A [M x K] row-major, B given as B^T [N x K] row-major
-// (k contiguous for both), so every fragment is one 16-byte load from
-// global memory / L2 and no LDS staging is needed.  The forward layers use
-// transposed BF16 copies of the weights; the input gradients use the
-// weights themselves.  Requires lda, ldb % 8 == 0 and K % 16 == 0.
-// KS = K / 16 when the depth is one of the network's (1, 8 or 16 steps):
-// the fragments of kGemmChunk k-steps are loaded before their MFMAs, so
-// their latencies overlap; KS = 0 walks a run-time K one step at a time.
-// Rows (columns) past M (N) load row (column) 0 and their outputs are not
-// stored, so no load is predicated.  The MFMAs run in k order either way.
-template <int KS>
-__global__ __launch_bounds__(256) void gemm_nt_kernel(GemmArgs g) {
+// C = A B^T-stored for K = 16 (the encoder): A [M x 16] row-major, B given as
+// B^T [N x 16] row-major, so every fragment is one 16-byte load from global
+// memory / L2.  Rows (columns) past M (N) load row (column) 0 and their
+// outputs are not stored, so no load is predicated.
+__global__ __launch_bounds__(256) void gemm_nt16_kernel(GemmArgs g) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int wm = w & 1, wn = w >> 1;
   const int row = blockIdx.y * 64 + wm * 32 + (lane & 31);
   const int col = blockIdx.x * 64 + wn * 32 + (lane & 31);
   const int kh = 8 * (lane >> 5);
-  const __bf16* ap = g.A + (int64_t)(row < g.M ? row : 0) * g.lda + kh;
-  const __bf16* bp = g.B + (int64_t)(col < g.N ? col : 0) * g.ldb + kh;
+  const bf16x8 a = *(const bf16x8*)(g.A + (int64_t)(row < g.M ? row : 0) * g.lda + kh);
+  const bf16x8 b = *(const bf16x8*)(g.B + (int64_t)(col < g.N ? col : 0) * g.ldb + kh);
   f32x16 acc = {};
-  if constexpr (KS > 0) {
-    constexpr int kChunk = KS < kGemmChunk ? KS : kGemmChunk;
-#pragma unroll
-    for (int c = 0; c < KS; c += kChunk) {
-      bf16x8 a[kChunk], b[kChunk];
-#pragma unroll
-      for (int s = 0; s < kChunk; ++s) {
-        a[s] = *(const bf16x8*)(ap + 16 * (c + s));
-        b[s] = *(const bf16x8*)(bp + 16 * (c + s));
-      }
-#pragma unroll
-      for (int s = 0; s < kChunk; ++s)
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], b[s], acc, 0, 0, 0);
-    }
-  } else {
-    for (int k0 = 0; k0 < g.K; k0 += 16) {
-      const bf16x8 a = *(const bf16x8*)(ap + k0);
-      const bf16x8 b = *(const bf16x8*)(bp + k0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-  }
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
   EpiIn in;
   epi_load(g, blockIdx.y * 64 + wm * 32, col, lane, in);
   epi_store(g, acc, col, in);
 }
 
-#ifndef SPH_GEMM_LDS
-#define SPH_GEMM_LDS 1
-#endif
-
-// The same product with both 64 x K tiles staged in LDS: the block loads A's
+// The same product for K = 128 and 256 (forward layers with transposed BF16
+// copies of the weights; input gradients with the weights themselves), both
+// 64 x K tiles staged in LDS: the block loads A's
 // 64 rows and B^T's 64 rows with 16-byte loads in which consecutive threads
 // read consecutive bytes of a row (whole cache lines), then each wave reads
 // its MFMA fragments from LDS.  Per-lane fragment loads from global memory
 // touch 32 cache lines per instruction and kept the texture units 73 %
 // busy.  The row pitch is K + 8 elements, so the eight 16-byte reads of a
 // pass start 16 bytes apart modulo 128 (no bank conflicts).  Rows (columns)
-// past M (N) load row (column) 0 and are not stored.  The MFMAs run in k
-// order and the epilogue is `epi_load` / `epi_store`: the results are those
-// of gemm_nt_kernel bit for bit.  K = 16 KS (128 or 256: 35 or 68 KB of LDS).
-template <int KS>
+// past M (N) load row (column) 0 and are not stored.  K = 16 KS (128 or 256:
+// 35 or 68 KB of LDS).  SPLIT: columns from n2 on go to C2.
+template <int KS, bool SPLIT = false>
 __global__ __launch_bounds__(256) void gemm_nt_lds_kernel(GemmArgs g) {
   constexpr int K = 16 * KS;
   constexpr int kPitch = K + 8;
@@ -277,8 +206,8 @@ __global__ __launch_bounds__(256) void gemm_nt_lds_kernel(GemmArgs g) {
   }
   const int col = col0 + wn * 32 + (lane & 31);
   EpiIn in;
-  epi_load(g, row0 + wm * 32, col, lane, in);
-  epi_store(g, acc, col, in);
+  epi_load<SPLIT>(g, row0 + wm * 32, col, lane, in);
+  epi_store<SPLIT>(g, acc, col, in);
 }
 
 // wt[n*K + k] = bf16(w[k*N + n]) for one K x N weight matrix.
@@ -291,18 +220,171 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(int K, int N,
   wt[(int64_t)n * K + k] = (__bf16)w[t];
 }
 
-// Sum of nslab slabs [M x N] (ld) into out (accumulate when acc != 0).
-__global__ __launch_bounds__(256) void slab_sum_kernel(const float* __restrict__ part, int nslab,
-                                                       int64_t zstride, int M, int N,
-                                                       int64_t ld, float* __restrict__ out,
-                                                       int acc) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (int64_t)M * N) return;
-  const int m = (int)(i / N), n = (int)(i % N);
+// out[c] (+)= sum over z of part[z * zstride + c], c < cols: the fixed-order
+// sum of per-block partials.  ZL lanes share a column: lane k sums slabs k,
+// k + ZL, ... and the ZL partials are added as a tree in LDS.  One thread per
+// column walking every slab was one chain of dependent memory waits: 179 us
+// per launch on average over a training step of 33k nodes (up to 4096 slabs
+// of 2176 columns); with the slabs shared out the same sums take 4-6 us.
+template <int ZL>
+__global__ __launch_bounds__(1024) void slab_sum_kernel(const float* __restrict__ part, int nslab,
+                                                        int64_t zstride, int cols,
+                                                        float* __restrict__ out, int acc) {
+  constexpr int kCols = 1024 / ZL;
+  __shared__ float red[ZL][kCols];
+  const int t = threadIdx.x % kCols, k = threadIdx.x / kCols;
+  const int c = blockIdx.x * kCols + t;
   float s = 0.f;
-  for (int z = 0; z < nslab; ++z) s += part[z * zstride + (int64_t)m * ld + n];
-  if (acc) s += out[i];
-  out[i] = s;
+  if (c < cols) {
+#pragma unroll 8
+    for (int z = k; z < nslab; z += ZL) s += part[z * zstride + c];
+  }
+  red[k][t] = s;
+  __syncthreads();
+#pragma unroll
+  for (int h = ZL / 2; h > 0; h >>= 1) {
+    if (k < h) red[k][t] += red[k + h][t];
+    __syncthreads();
+  }
+  if (k == 0 && c < cols) out[c] = acc ? out[c] + red[0][t] : red[0][t];
+}
+
+// Few slabs of many columns: one lane per column keeps every lane busy; many
+// slabs: 16 columns a block, so that 64 lanes read each column's slabs (and
+// a 64-byte segment of a slab at a time).
+static void slab_sum(hipStream_t st, const float* part, int nslab, int64_t zstride, int cols,
+                     float* out, int acc) {
+  const dim3 b(1024);
+  if (nslab <= 4)
+    hipLaunchKernelGGL(slab_sum_kernel<1>, dim3((cols + 1023) / 1024), b, 0, st, part, nslab,
+                       zstride, cols, out, acc);
+  else if (nslab <= 128)
+    hipLaunchKernelGGL(slab_sum_kernel<8>, dim3((cols + 127) / 128), b, 0, st, part, nslab,
+                       zstride, cols, out, acc);
+  else
+    hipLaunchKernelGGL(slab_sum_kernel<64>, dim3((cols + 15) / 16), b, 0, st, part, nslab,
+                       zstride, cols, out, acc);
+}
+
+// ---------------------------------------------------------------------------
+// weight gradients: G[kdim x ncols] = X^T D over the rows (nodes)
+// ---------------------------------------------------------------------------
+struct GradArgs {
+  int rows, kdim, ncols, chunk;  // chunk: rows per blockIdx.z, a multiple of 32
+  const __bf16* X;               // [rows x kdim], leading dimension ldx
+  int64_t ldx;
+  const __bf16* D;               // [rows x ncols]
+  int64_t ldd;
+  float* part;                   // slab z at part + z * kdim * ncols
+};
+
+// Two rows of eight BF16 columns interleaved: out[c] = (row0[c], row1[c]).
+__device__ __forceinline__ void interleave(const uint4 a, const uint4 b, uint32_t (&o)[8]) {
+  const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    o[2 * i] = __builtin_amdgcn_perm(bv[i], av[i], 0x05040100);
+    o[2 * i + 1] = __builtin_amdgcn_perm(bv[i], av[i], 0x07060302);
+  }
+}
+
+// The contraction runs over the rows, so both operands would be read down
+// their columns (the previous kernel: sixteen 2-byte loads per lane and
+// MFMA, 118 us per product of 33k rows).  Here a block owns a TM x TN tile
+// of G and a chunk of rows; it loads 32 rows at a time in whole 16-byte
+// pieces, interleaves pairs of rows in registers, and keeps the pair (rows
+// 2p, 2p + 1) of column c as one dword at lds[p][c]: an MFMA fragment of a
+// column (rows 8h..8h+7 of a 16-row step for half-wave h) is then four
+// conflict-free 4-byte LDS reads.  The next 32 rows are loaded into
+// registers while the current ones are multiplied.  Rows past the chunk are
+// zeros, columns past the matrix are loaded from column 0 and not stored.
+// TM x TN is 128 x 64 (32 x 128 for the 16 node features).
+template <int TM, int TN>
+__global__ __launch_bounds__(256) void grad_kernel(GradArgs g) {
+  constexpr int kRows = 32, kPairs = kRows / 2;
+  constexpr int kCx = TM / 8, kCd = TN / 8;   // 16-byte pieces per row
+  constexpr int WM = TM >= 128 ? 2 : 1, WN = 4 / WM;  // wave grid
+  constexpr int FM = TM / (32 * WM), FN = TN / (32 * WN);
+  constexpr int kTasks = kPairs * (kCx + kCd);
+  constexpr int kPer = (kTasks + 255) / 256;
+  static_assert(FM >= 1 && FN >= 1 && FM * 32 * WM == TM && FN * 32 * WN == TN, "tile");
+  // 16 dwords of padding: the pitch stays a multiple of four dwords for the
+  // 16-byte writes and consecutive pairs start 16 banks apart
+  __shared__ __align__(16) uint32_t lds[kPairs][TM + TN + 16];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
+  const int r_begin = blockIdx.z * g.chunk, r_end = min(g.rows, r_begin + g.chunk);
+  uint4 va[kPer], vb[kPer];
+  auto load = [&](int r0) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int t = tid + 256 * i;
+      va[i] = vb[i] = make_uint4(0, 0, 0, 0);
+      if (t >= kTasks) continue;
+      const int p = t / (kCx + kCd), c = t % (kCx + kCd);
+      const bool x = c < kCx;
+      const int col = x ? m0 + 8 * c : n0 + 8 * (c - kCx);
+      const __bf16* base = x ? g.X : g.D;
+      const int64_t ld = x ? g.ldx : g.ldd;
+      const int cc = col < (x ? g.kdim : g.ncols) ? col : 0;
+      const int r = r0 + 2 * p;
+      if (r < r_end) va[i] = *(const uint4*)(base + (int64_t)r * ld + cc);
+      if (r + 1 < r_end) vb[i] = *(const uint4*)(base + (int64_t)(r + 1) * ld + cc);
+    }
+  };
+  f32x16 acc[FM][FN] = {};
+  load(r_begin);
+  for (int r0 = r_begin; r0 < r_end; r0 += kRows) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int t = tid + 256 * i;
+      if (t >= kTasks) continue;
+      const int p = t / (kCx + kCd), c = t % (kCx + kCd);
+      uint32_t o[8];
+      interleave(va[i], vb[i], o);
+      *(uint4*)&lds[p][8 * c] = make_uint4(o[0], o[1], o[2], o[3]);
+      *(uint4*)&lds[p][8 * c + 4] = make_uint4(o[4], o[5], o[6], o[7]);
+    }
+    __syncthreads();
+    if (r0 + kRows < r_end) load(r0 + kRows);
+    const int wm = w % WM, wn = w / WM;
+#pragma unroll
+    for (int s = 0; s < kRows / 16; ++s) {
+      const int p0 = 8 * s + 4 * (lane >> 5);
+      bf16x8 a[FM], b[FN];
+      auto frag = [&](int col) {
+        union {
+          uint32_t u[4];
+          bf16x8 v;
+        } f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) f.u[k] = lds[p0 + k][col];
+        return f.v;
+      };
+#pragma unroll
+      for (int i = 0; i < FM; ++i) a[i] = frag((wm * FM + i) * 32 + (lane & 31));
+#pragma unroll
+      for (int j = 0; j < FN; ++j) b[j] = frag(TM + (wn * FN + j) * 32 + (lane & 31));
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+  }
+  float* out = g.part + (int64_t)blockIdx.z * g.kdim * g.ncols;
+  const int wm = w % WM, wn = w / WM;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = m0 + (wm * FM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        const int col = n0 + (wn * FN + j) * 32 + (lane & 31);
+        if (row < g.kdim && col < g.ncols) out[(int64_t)row * g.ncols + col] = acc[i][j][r];
+      }
 }
 
 // ---------------------------------------------------------------------------
@@ -802,42 +884,45 @@ __global__ __launch_bounds__(256) void loss_kernel(int n, const int* __restrict_
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-// out = mask(act > 0) * d  (FP32 and BF16 copies); ld strides per array.
-__global__ __launch_bounds__(256) void relu_bwd_kernel(int64_t count, int cols,
-                                                       const float* __restrict__ act,
-                                                       int64_t lda_, const float* __restrict__ d,
-                                                       int64_t ldd, float* __restrict__ out,
-                                                       __bf16* __restrict__ outb) {
-  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= count) return;
-  const int64_t r = t / cols;
-  const int c = (int)(t % cols);
-  const float v = act[r * lda_ + c] > 0.f ? d[r * ldd + c] : 0.f;
-  out[t] = v;
-  outb[t] = (__bf16)v;
-}
-
-// dst[r][c] = a[r][c] + b[r * ldb + c]
-__global__ __launch_bounds__(256) void add_kernel(int64_t count, int cols,
-                                                  const float* __restrict__ a,
-                                                  const float* __restrict__ b, int64_t ldb,
-                                                  float* __restrict__ dst) {
-  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= count) return;
-  const int64_t r = t / cols;
-  const int c = (int)(t % cols);
-  dst[t] = a[t] + b[r * ldb + c];
-}
-
-// Column sums of x [rows x cols] (ld) per block of 256 rows -> part.
-__global__ __launch_bounds__(256) void colsum_part_kernel(int rows, int cols,
-                                                          const float* __restrict__ x,
-                                                          int64_t ld, float* __restrict__ part) {
-  const int r0 = blockIdx.x * 256;
-  for (int c = threadIdx.x; c < cols; c += 256) {
-    float s = 0.f;
-    for (int r = r0; r < min(rows, r0 + 256); ++r) s += x[(int64_t)r * ld + c];
-    part[(int64_t)blockIdx.x * cols + c] = s;
+// outb = BF16(mask(act > 0) * d) and, per block of kReluRows rows, the column
+// sums of the masked FP32 values (the bias gradient's partials): nothing else
+// reads the FP32 values, so they are not stored.  32 lanes x 4 columns cover
+// a row of kH, eight rows at a time.  (Masking and summing in launches of
+// their own took 16 + 61 us for 33k rows; this one 9 us.)
+constexpr int kReluRows = 64;
+__global__ __launch_bounds__(256) void relu_bwd_kernel(int rows, const float* __restrict__ act,
+                                                       const float* __restrict__ d,
+                                                       __bf16* __restrict__ outb,
+                                                       float* __restrict__ part) {
+  __shared__ float4 red[8][32];
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+  const int c = threadIdx.x & 31, k = threadIdx.x >> 5;
+  const int r0 = blockIdx.x * kReluRows;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int i = 0; i < kReluRows / 8; ++i) {
+    const int r = r0 + 8 * i + k;
+    if (r >= rows) break;
+    const int64_t o = (int64_t)r * kH + 4 * c;
+    const float4 a = *(const float4*)(act + o);
+    const float4 v = *(const float4*)(d + o);
+    const float4 z = make_float4(a.x > 0.f ? v.x : 0.f, a.y > 0.f ? v.y : 0.f,
+                                 a.z > 0.f ? v.z : 0.f, a.w > 0.f ? v.w : 0.f);
+    const bf16x4 zb = {(__bf16)z.x, (__bf16)z.y, (__bf16)z.z, (__bf16)z.w};
+    *(bf16x4*)(outb + o) = zb;
+    s.x += z.x;
+    s.y += z.y;
+    s.z += z.z;
+    s.w += z.w;
+  }
+  red[k][c] = s;
+  __syncthreads();
+  if (threadIdx.x < kH) {
+    const int col = threadIdx.x;
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t += ((const float*)red[i])[col];
+    part[(int64_t)blockIdx.x * kH + col] = t;
   }
 }
 
@@ -911,7 +996,7 @@ struct Model {
   double t_ms[4] = {0, 0, 0, 0};
   int64_t t_calls = 0;
   std::vector<hipEvent_t> ev;
-  Buf X, E, N4, H[kR + 1], HA[kR], PQ[kR], U[kR], dH, dZ, dZb, dHA, dPQ, dPQb, part, lossp;
+  Buf X, E, N4, H[kR + 1], HA[kR], PQ[kR], U[kR], dH, dZb, dA, dPQ, dPQb, part, lossp;
   int64_t n_act = -1, e_act = -1;
   bool acts = false;  // the last forward pass stored what the backward pass reads
 };
@@ -980,29 +1065,20 @@ static int edge_fwd_blocks(int64_t n) {
   return (int)std::max<int64_t>(1, (waves + 3) / 4);
 }
 
-static int32_t gemm(hipStream_t st, bool ta, bool tb, GemmArgs a, int splits = 1) {
-  if (!ta && tb && splits == 1 && a.K % 16 == 0 && a.lda % 8 == 0 && a.ldb % 8 == 0 &&
-      ((uintptr_t)a.A & 15) == 0 && ((uintptr_t)a.B & 15) == 0) {
-    a.kc = a.K;
-    dim3 grid((a.N + 63) / 64, (a.M + 63) / 64, 1);
-    if (a.K == 16) hipLaunchKernelGGL(gemm_nt_kernel<1>, grid, dim3(256), 0, st, a);
-    else if (SPH_GEMM_LDS && a.K == 128)
-      hipLaunchKernelGGL(gemm_nt_lds_kernel<8>, grid, dim3(256), 0, st, a);
-    else if (SPH_GEMM_LDS && a.K == 256)
-      hipLaunchKernelGGL(gemm_nt_lds_kernel<16>, grid, dim3(256), 0, st, a);
-    else if (a.K == 128) hipLaunchKernelGGL(gemm_nt_kernel<8>, grid, dim3(256), 0, st, a);
-    else if (a.K == 256) hipLaunchKernelGGL(gemm_nt_kernel<16>, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(gemm_nt_kernel<0>, grid, dim3(256), 0, st, a);
-    return launch_status("sph_mlp/gemm_nt");
+static int32_t gemm(hipStream_t st, const GemmArgs& a) {
+  dim3 grid((a.N + 63) / 64, (a.M + 63) / 64, 1);
+  if (a.K == 16) {
+    hipLaunchKernelGGL(gemm_nt16_kernel, grid, dim3(256), 0, st, a);
+  } else if (a.K == 128 && a.C2 != nullptr) {
+    hipLaunchKernelGGL((gemm_nt_lds_kernel<8, true>), grid, dim3(256), 0, st, a);
+  } else if (a.K == 128) {
+    hipLaunchKernelGGL(gemm_nt_lds_kernel<8>, grid, dim3(256), 0, st, a);
+  } else if (a.K == 256) {
+    hipLaunchKernelGGL(gemm_nt_lds_kernel<16>, grid, dim3(256), 0, st, a);
+  } else {
+    set_error("sph_mlp: no product of depth %d", a.K);
+    return SPH_EUNSUPPORTED;
   }
-  a.kc = (a.K + splits - 1) / splits;
-  a.kc = (a.kc + 15) / 16 * 16;
-  const int z = (a.K + a.kc - 1) / a.kc;
-  dim3 grid((a.N + 63) / 64, (a.M + 63) / 64, z < 1 ? 1 : z);
-  if (!ta && !tb) hipLaunchKernelGGL((gemm_kernel<false, false>), grid, dim3(256), 0, st, a);
-  else if (!ta && tb) hipLaunchKernelGGL((gemm_kernel<false, true>), grid, dim3(256), 0, st, a);
-  else if (ta && !tb) hipLaunchKernelGGL((gemm_kernel<true, false>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((gemm_kernel<true, true>), grid, dim3(256), 0, st, a);
   return launch_status("sph_mlp/gemm");
 }
 
@@ -1019,37 +1095,50 @@ static GemmArgs gargs(int M, int N, int K, const __bf16* A, int64_t lda, const _
   return a;
 }
 
-// Weight gradient G[Kdim x N] += X^T D with X [rows x Kdim] (ldx), D [rows x N]
-// (ldd), reduced over rows in split-K slabs then summed deterministically.
+// Row chunks of a weight gradient: enough blocks for the 256 CUs (four tiles
+// of 128 x 64 per matrix), each with at least 256 rows so that a slab's
+// 128 KB of output stays small against the rows it reads.
+static int grad_splits(int rows) { return std::max(1, std::min(64, (rows + 255) / 256)); }
+
+// Weight gradient G[kdim x ncols] += X^T D with X [rows x kdim] (ldx), D
+// [rows x ncols] (ldd): a slab per chunk of rows, then the fixed-order sum.
 static int32_t weight_grad(Model* M, hipStream_t st, int rows, int kdim, int ncols,
                            const __bf16* X, int64_t ldx, const __bf16* D, int64_t ldd,
                            float* G) {
-  const int splits = rows > 4096 ? std::min(64, rows / 2048) : 1;
+  GradArgs a{};
+  a.rows = rows;
+  a.kdim = kdim;
+  a.ncols = ncols;
+  a.X = X;
+  a.ldx = ldx;
+  a.D = D;
+  a.ldd = ldd;
+  const int splits = grad_splits(rows);
+  a.chunk = ((rows + splits - 1) / splits + 31) / 32 * 32;
+  const int nz = (rows + a.chunk - 1) / a.chunk;
   const int64_t slab = (int64_t)kdim * ncols;
-  SPH_TRY(ensure(M->part, (size_t)splits * slab * 4 + 1024));
-  GemmArgs a = gargs(kdim, ncols, rows, X, ldx, D, ldd);
-  a.C = (float*)M->part.p;
-  a.ldc = ncols;
-  a.c_zstride = slab;
-  SPH_TRY(gemm(st, true, false, a, splits));
-  const int kc = ((rows + splits - 1) / splits + 15) / 16 * 16;
-  const int nz = (rows + kc - 1) / kc;
-  hipLaunchKernelGGL(slab_sum_kernel, dim3(nblk(slab)), dim3(256), 0, st,
-                     (const float*)M->part.p, nz < 1 ? 1 : nz, slab, kdim, ncols,
-                     (int64_t)ncols, G, 1);
+  SPH_TRY(ensure(M->part, (size_t)nz * slab * 4 + 1024));
+  a.part = (float*)M->part.p;
+  if (kdim <= 32)
+    hipLaunchKernelGGL((grad_kernel<32, 128>), dim3((ncols + 127) / 128, 1, nz), dim3(256), 0, st,
+                       a);
+  else
+    hipLaunchKernelGGL((grad_kernel<128, 64>), dim3((ncols + 63) / 64, (kdim + 127) / 128, nz),
+                       dim3(256), 0, st, a);
+  slab_sum(st, (const float*)M->part.p, nz, slab, (int)slab, G, 1);
   return launch_status("sph_mlp/weight_grad");
 }
 
-// bias gradient: G[cols] += column sums of x[rows x cols]
-static int32_t bias_grad(Model* M, hipStream_t st, int rows, int cols, const float* x,
-                         int64_t ld, float* G) {
-  const int nb = (rows + 255) / 256;
-  SPH_TRY(ensure(M->part, (size_t)nb * cols * 4 + 1024));
-  hipLaunchKernelGGL(colsum_part_kernel, dim3(nb), dim3(256), 0, st, rows, cols, x, ld,
+// dZb = BF16(d masked by act > 0) and the bias gradient G[kH] += its column
+// sums.
+static int32_t relu_bias_grad(Model* M, hipStream_t st, int rows, const float* act,
+                              const float* d, __bf16* dZb, float* G) {
+  const int nb = (rows + kReluRows - 1) / kReluRows;
+  SPH_TRY(ensure(M->part, (size_t)nb * kH * 4 + 1024));
+  hipLaunchKernelGGL(relu_bwd_kernel, dim3(nb), dim3(256), 0, st, rows, act, d, dZb,
                      (float*)M->part.p);
-  hipLaunchKernelGGL(slab_sum_kernel, dim3(nblk(cols)), dim3(256), 0, st,
-                     (const float*)M->part.p, nb, (int64_t)cols, 1, cols, (int64_t)cols, G, 1);
-  return launch_status("sph_mlp/bias_grad");
+  slab_sum(st, (const float*)M->part.p, nb, kH, kH, G, 1);
+  return launch_status("sph_mlp/relu_bwd");
 }
 
 static FeatArgs feat_args(const sph_mlp_graph* g) {
@@ -1146,7 +1235,7 @@ int32_t sph_mlp_destroy(void* model) {
                   (void*)M->v})
     (void)hipFree(p);
   for (hipEvent_t e : M->ev) (void)hipEventDestroy(e);
-  for (Buf* b : {&M->X, &M->E, &M->N4, &M->dH, &M->dZ, &M->dZb, &M->dHA, &M->dPQ, &M->dPQb, &M->part,
+  for (Buf* b : {&M->X, &M->E, &M->N4, &M->dH, &M->dZb, &M->dA, &M->dPQ, &M->dPQb, &M->part,
                  &M->lossp})
     (void)hipFree(b->p);
   for (int r = 0; r <= kR; ++r) (void)hipFree(M->H[r].p);
@@ -1272,7 +1361,7 @@ int32_t sph_mlp_forward(void* model, void* stream, const sph_mlp_graph* gr, floa
     a.Cb = (__bf16*)M->HA[0].p;
     a.ldcb = 2 * kH;
     T.begin(1);
-    SPH_TRY(gemm(st, false, true, a));
+    SPH_TRY(gemm(st, a));
     T.end();
   }
   for (int r = 0; r < kR; ++r) {
@@ -1283,7 +1372,7 @@ int32_t sph_mlp_forward(void* model, void* stream, const sph_mlp_graph* gr, floa
       a.C = PQ;
       a.ldc = 2 * kH;
       T.begin(1);
-      SPH_TRY(gemm(st, false, true, a));
+      SPH_TRY(gemm(st, a));
       T.end();
     }
     EdgeArgs e{};
@@ -1319,7 +1408,7 @@ int32_t sph_mlp_forward(void* model, void* stream, const sph_mlp_graph* gr, floa
         a.ldcb = 2 * kH;
       }
       T.begin(1);
-      SPH_TRY(gemm(st, false, true, a));
+      SPH_TRY(gemm(st, a));
       T.end();
     }
   }
@@ -1349,8 +1438,7 @@ int32_t sph_mlp_loss(void* model, void* stream, const sph_mlp_graph* gr, const f
   const float inv_nf = gr->n_fluid > 0 ? 1.f / (float)gr->n_fluid : 0.f;
   hipLaunchKernelGGL(loss_kernel, dim3(nb), dim3(256), 0, st, (int)n, gr->btype, out_dev,
                      target_dev, inv_nf, dout_dev, (float*)M->lossp.p);
-  hipLaunchKernelGGL(slab_sum_kernel, dim3(1), dim3(256), 0, st, (const float*)M->lossp.p, nb,
-                     (int64_t)1, 1, 1, (int64_t)1, loss_dev, 0);
+  slab_sum(st, (const float*)M->lossp.p, nb, 1, 1, loss_dev, 0);
   return launch_status("sph_mlp_loss");
 }
 
@@ -1372,18 +1460,17 @@ int32_t sph_mlp_backward(void* model, void* stream, const sph_mlp_graph* gr,
   hipStream_t st = as_stream(stream);
   const Layout& L = M->L;
   SPH_TRY(ensure(M->dH, (size_t)n * kH * 4));
-  SPH_TRY(ensure(M->dZ, (size_t)n * kH * 4));
-  SPH_TRY(ensure(M->dZb, (size_t)n * 2 * kH * 2));
-  SPH_TRY(ensure(M->dHA, (size_t)n * 2 * kH * 4));
+  SPH_TRY(ensure(M->dZb, (size_t)n * kH * 2));
+  SPH_TRY(ensure(M->dA, (size_t)n * kH * 4));
   SPH_TRY(ensure(M->dPQ, (size_t)n * 2 * kH * 4));
   SPH_TRY(ensure(M->dPQb, (size_t)n * 2 * kH * 2));
   {
     // one scratch buffer serves every partial reduction of this pass: size
     // it once, before any launch reads it
-    const int64_t wg = 64LL * 2 * kH * kH;                       // split-K slabs
+    const int64_t wg = 64LL * 2 * kH * kH;                       // weight-gradient slabs
     const int64_t eg = 1024LL * 4 * (kE + 1) * kH;                // edge partials
     const int64_t dg = ((n + 63) / 64) * (kH * kOut + kOut);      // decoder partials
-    const int64_t bg = ((n + 255) / 256) * kH;                    // bias partials
+    const int64_t bg = ((n + kReluRows - 1) / kReluRows) * kH;    // bias partials
     SPH_TRY(ensure(M->part, (size_t)std::max(std::max(wg, eg), std::max(dg, bg)) * 4 + 1024));
   }
   float* dH = (float*)M->dH.p;
@@ -1396,31 +1483,26 @@ int32_t sph_mlp_backward(void* model, void* stream, const sph_mlp_graph* gr,
                        (const float*)M->H[kR].p, M->w + L.w_out, dout_dev, dH,
                        (float*)M->part.p);
     // W_out and b_out are contiguous: one slab sum over blocks
-    hipLaunchKernelGGL(slab_sum_kernel, dim3(nblk(per)), dim3(256), 0, st,
-                       (const float*)M->part.p, nb, per, 1, (int)per, per, M->g + L.w_out, 1);
+    slab_sum(st, (const float*)M->part.p, nb, per, (int)per, M->g + L.w_out, 1);
     SPH_TRY(launch_status("sph_mlp_backward/decoder"));
   }
   for (int r = kR - 1; r >= 0; --r) {
-    const int64_t cnt = n * kH;
-    float* dZ = (float*)M->dZ.p;
     __bf16* dZb = (__bf16*)M->dZb.p;
-    // dZ = dH' * (U > 0)
-    hipLaunchKernelGGL(relu_bwd_kernel, dim3(nblk(cnt)), dim3(256), 0, st, cnt, kH,
-                       (const float*)M->U[r].p, (int64_t)kH, (const float*)dH, (int64_t)kH, dZ,
-                       dZb);
-    SPH_TRY(bias_grad(M, st, (int)n, kH, dZ, kH, M->g + L.c_u[r]));
+    // dZ = dH' * (U > 0), dc_u
+    SPH_TRY(relu_bias_grad(M, st, (int)n, (const float*)M->U[r].p, dH, dZb, M->g + L.c_u[r]));
     // dW_u += [H | A]^T dZ
     SPH_TRY(weight_grad(M, st, (int)n, 2 * kH, kH, (const __bf16*)M->HA[r].p, 2 * kH, dZb, kH,
                         M->g + L.w_u[r]));
-    {  // d[H | A] = dZ W_u^T
+    {  // d[H | A] = dZ W_u^T: dH_r = dH' + d[H], dA
       GemmArgs a = gargs((int)n, 2 * kH, kH, dZb, kH, M->wb + L.w_u[r], kH);
-      a.C = (float*)M->dHA.p;
-      a.ldc = 2 * kH;
-      SPH_TRY(gemm(st, false, true, a));
+      a.C = dH;
+      a.ldc = kH;
+      a.accumulate = 1;
+      a.C2 = (float*)M->dA.p;
+      a.ldc2 = kH;
+      a.n2 = kH;
+      SPH_TRY(gemm(st, a));
     }
-    // dH_r = dH' + d[H]
-    hipLaunchKernelGGL(add_kernel, dim3(nblk(cnt)), dim3(256), 0, st, cnt, kH, (const float*)dH,
-                       (const float*)M->dHA.p, (int64_t)2 * kH, dH);
     // edges: dP, dQ, dWc, dbe
     EdgeArgs e{};
     e.n = (int)n;
@@ -1430,8 +1512,8 @@ int32_t sph_mlp_backward(void* model, void* stream, const sph_mlp_graph* gr,
     e.PQ = (const float*)M->PQ[r].p;
     e.Wc = M->w + L.w_c[r];
     e.be = M->w + L.b_e[r];
-    e.dA = (const float*)M->dHA.p + kH;
-    e.ldda = 2 * kH;
+    e.dA = (const float*)M->dA.p;
+    e.ldda = kH;
     e.dPQ = (float*)M->dPQ.p;
     e.dPQb = (__bf16*)M->dPQb.p;
     const int nbk = (int)std::min<int64_t>(1024, (n + 3) / 4);
@@ -1440,9 +1522,7 @@ int32_t sph_mlp_backward(void* model, void* stream, const sph_mlp_graph* gr,
     e.part = (float*)M->part.p;
     hipLaunchKernelGGL(edge_bwd_kernel, dim3(nbk), dim3(256), 0, st, e);
     // W_c and b_e are contiguous
-    hipLaunchKernelGGL(slab_sum_kernel, dim3(nblk(per)), dim3(256), 0, st,
-                       (const float*)M->part.p, nbk * 4, per, 1, (int)per, per,
-                       M->g + L.w_c[r], 1);
+    slab_sum(st, (const float*)M->part.p, nbk * 4, per, (int)per, M->g + L.w_c[r], 1);
     SPH_TRY(launch_status("sph_mlp_backward/edges"));
     // dW_ab += H^T dPQ
     SPH_TRY(weight_grad(M, st, (int)n, kH, 2 * kH, (const __bf16*)M->HA[r].p, 2 * kH,
@@ -1453,18 +1533,13 @@ int32_t sph_mlp_backward(void* model, void* stream, const sph_mlp_graph* gr,
       a.C = dH;
       a.ldc = kH;
       a.accumulate = 1;
-      SPH_TRY(gemm(st, false, true, a));
+      SPH_TRY(gemm(st, a));
     }
   }
   // encoder: dZ0 = dH * (H0 > 0); dW_in += X^T dZ0; db_in
   {
-    const int64_t cnt = n * kH;
-    float* dZ = (float*)M->dZ.p;
     __bf16* dZb = (__bf16*)M->dZb.p;
-    hipLaunchKernelGGL(relu_bwd_kernel, dim3(nblk(cnt)), dim3(256), 0, st, cnt, kH,
-                       (const float*)M->H[0].p, (int64_t)kH, (const float*)dH, (int64_t)kH, dZ,
-                       dZb);
-    SPH_TRY(bias_grad(M, st, (int)n, kH, dZ, kH, M->g + L.b_in));
+    SPH_TRY(relu_bias_grad(M, st, (int)n, (const float*)M->H[0].p, dH, dZb, M->g + L.b_in));
     SPH_TRY(weight_grad(M, st, (int)n, kIn, kH, (const __bf16*)M->X.p, kIn, dZb, kH,
                         M->g + L.w_in));
   }

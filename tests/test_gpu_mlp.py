@@ -191,3 +191,40 @@ def test_adam_steps_reduce_the_loss():
         model.adam(stream, lr=3e-3)
     print("loss %.3e -> %.3e" % (losses[0], losses[-1]))
     assert losses[-1] < 0.7 * losses[0]
+
+
+@pytest.mark.parametrize("width,height", [(0.01, 0.01), (0.02, 0.03), (0.05, 0.07), (0.3, 0.43)])
+def test_gradients_at_chunk_remainders(width, height):
+    """Weight and bias gradients where the node count leaves remainders of
+    the 32-row steps, the 64-row bias blocks and the 256-row chunks (one
+    chunk of a few rows up to several chunks), each tensor against the
+    BF16-rounded oracle.  Biases and non-negative H x H weights keep every ReLU
+    active, so that no unit near zero is masked on one side only (one such unit of one node is worth
+    up to 1/nodes of a gradient).  What is left: FP32 sums of at most 2e3
+    terms in another order (2e3 * 2^-24 = 1e-4), the aggregation's split
+    products (2^-16) and BF16 copies of H, A and dZ that round the other way
+    (2^-8 of a value, on a small share of them): below 1e-3."""
+    g, _ = _graph(width=width, height=height)
+    p = M.unflatten(_params(2).astype(np.float64))
+    for k in p:
+        if k.startswith(("b_in", "b_e", "c_u")):
+            p[k] = np.full(p[k].shape, 200.0)
+        elif k.startswith(("w_ab", "w_u")):
+            p[k] = np.abs(p[k])
+    theta = M.flatten(p).astype(np.float32)
+    p = M.unflatten(theta.astype(np.float64))
+    model = EdgeMLP(params=theta)
+    pos4, vel4, rho, bt, off, nbr, c = _host(g)
+    rng = np.random.Generator(np.random.PCG64(9))
+    T = rng.normal(0, 1, (g.n, 2)).astype(np.float32)
+    X, E, dst, src = M.features(pos4, vel4, rho, bt, off, nbr, c)
+    Y, cache = M.forward(p, X, E, dst, src, g.n, round_bf16=True)
+    assert cache["H0"].min() > 0
+    for r in range(M.ROUNDS):
+        assert cache["r%d" % r]["S"].min() > 0 and cache["r%d" % r]["U"].min() > 0
+    ref = M.backward(p, cache, M.loss(Y, T, bt)[1])
+    model.zero_grad(torch.cuda.current_stream().cuda_stream)
+    model.loss_backward(g, torch.from_numpy(T).cuda())
+    got = M.unflatten(model.grads().astype(np.float64))
+    for k in ref:
+        assert _rel(got[k], ref[k]) < 3e-3, (k, g.n)
