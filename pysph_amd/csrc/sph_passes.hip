@@ -6,85 +6,167 @@
 //   * the same pass fused with the Euler / RK2 stage update of the particle
 //     (integrator.py:472-514, :534-551, :597-619).
 //
-// One thread per destination particle.  Destinations are visited in the
-// cell-sorted layout, so the 64 lanes of a wave share the same few stencil
-// rows and their source reads hit in L1/L2.  Each stencil (dy,dz) row is a
-// single contiguous source range.  Candidates are screened in the storage
-// precision and accepted by the reference's exact FP64 test.
+// These are the passes over the SoA fields: FP64 storage, variable-h
+// symmetric pairs, periodic axes, density rates and FP32 arrays without
+// packed copies.  A group of 4 to 32 lanes serves one destination
+// (sph_group.h).  Destinations are visited in the cell-sorted layout, so the
+// groups of a wave share stencil rows and their source reads hit in L1/L2.
+// Candidates are screened in the storage precision and accepted by the
+// reference's exact FP64 test.
 #include <math.h>
 
+#include "sph_group.h"
 #include "sph_passes.h"
 
 namespace sph {
 
-// Every accepted source j of destination (xd,yd,zd) in cell (cx,cy,cz):
-// the stencil rows of the destination and of its periodic images (one ring
-// wider, their cells come from FP64 image points), each pair through
-// pair_geom; body(j, d2, rx, ry, rz).
-template <typename T, typename CT, class F>
-__device__ __forceinline__ void scan_pairs(const Grid& g, const PassArgs<T>& a, const View<T>& S,
-                                           T xd, T yd, T zd, int cx, int cy, int cz, int ring,
-                                           float r2f, double r2d, F&& body) {
-  for_each_image(g, (double)xd, (double)yd, (double)zd, cx, cy, cz, ring * g.cs,
-                 [&](double ox, double oy, double oz, int icx, int icy, int icz, bool image) {
-                   for_each_row(g, S.cstart, icx, icy, icz, image ? ring + 1 : ring,
-                                [&](int j0, int j1) {
-                                  for (int j = j0; j < j1; ++j) {
-                                    CT d2, rx, ry, rz;
-                                    if (!pair_geom<T, CT>(a, S, j, xd, yd, zd, r2f, r2d, image,
-                                                          ox, oy, oz, d2, rx, ry, rz))
-                                      continue;
-                                    body(j, d2, rx, ry, rz);
-                                  }
-                                });
-                 });
+// Accepted sources waiting for their pair arithmetic, per wave, shared by
+// its groups.
+constexpr int kGroupQueue = 1024;
+struct GroupQueue {
+  int j[kGroupQueue];
+  uint8_t image[kGroupQueue];
+};
+
+// Offset of a periodic image's sources: x_j + s L.
+__device__ __forceinline__ double image_offset(int code, int axis, double period) {
+  const int d = axis == 0 ? code % 3 : (axis == 1 ? (code / 3) % 3 : code / 9);
+  return image_shift(d, period);
 }
 
-template <typename T, typename CT, bool TAIT>
-__global__ __launch_bounds__(kBlock) void density_kernel(Grid g, PassArgs<T> a) {
-  const int bid = xcd_block(blockIdx.x, gridDim.x);
-  const int i = bid * kBlock + threadIdx.x;
-  if (i >= a.dst.n) return;
-  if (a.dst.tag != nullptr && a.dst.tag[i] != 0) {
-    a.rho[i] = T(0);
-    if (TAIT) {
-      a.p[i] = T(0);
-      a.cs[i] = T(0);
+// The destination of a lane's group: i = its particle, whether it exists and
+// is LocalReal, its position, cell and search radius.
+template <typename T>
+struct GroupDst {
+  int i;
+  bool valid, local;
+  T x, y, z, h;
+  double r2d, rc;
+  float r2f;
+  int cx, cy, cz, ring;
+  __device__ __forceinline__ GroupDst(const Grid& g, const PassArgs<T>& a, const Group& gr,
+                                      int log2) {
+    const int bid = xcd_block(blockIdx.x, gridDim.x);
+    const int wave = bid * (kBlock / 64) + (threadIdx.x >> 6);
+    i = wave * (64 >> log2) + gr.index;
+    valid = i < a.dst.n;
+    local = valid && (a.dst.tag == nullptr || a.dst.tag[i] == 0);
+    x = y = z = h = T(0);
+    cx = cy = cz = 0;
+    if (local) {
+      x = a.dst.x[i];
+      y = a.dst.y[i];
+      z = a.dst.z[i];
+      h = a.dst.h[i];
+      cell_xyz(a.dst.cell[i], g, cx, cy, cz);
     }
-    return;
+    const double r = (double)h * a.rs;
+    r2d = r * r;
+    r2f = (float)r2d;
+    ring = ring_of(g, a.disp);
+    // symmetric pairs reach as far as the largest radius
+    const double reach = a.symmetric && g.rmax > fabs(r) ? g.rmax : fabs(r);
+    rc = reach + (a.disp ? (double)*a.disp : 0.0);
   }
-  const T xd = a.dst.x[i], yd = a.dst.y[i], zd = a.dst.z[i];
-  const T hd = a.dst.h[i];
-  const double r = (double)hd * a.rs;
-  const double r2d = r * r;
-  const float r2f = (float)r2d;
-  int cx, cy, cz;
-  cell_xyz(a.dst.cell[i], g, cx, cy, cz);
-  const int ring = ring_of(g, a.disp);
+};
+
+// Every accepted source of source array S: body(j, d2, rx, ry, rz), each lane
+// of the group its share of them.  QUEUED: accepted candidates are collected
+// in LDS per group and body runs on G of them at a time, so that the pair
+// arithmetic keeps the lanes busy (about 60 % of the candidates are accepted
+// with bins of half the search radius, 20 % with bins of the radius).  Not
+// queued: body runs on each candidate as it is found, for bodies that cost
+// less than the second gather.
+template <typename T, typename CT, bool PERIODIC, bool QUEUED, class F>
+__device__ __forceinline__ void scan_pairs(const Grid& g, const PassArgs<T>& a, const View<T>& S,
+                                           const Group& gr, const GroupDst<T>& D, GroupRows& rows,
+                                           GroupQueue* queue, F&& body) {
+  const int cap = kGroupQueue / (64 / gr.size);
+  int* qj = QUEUED ? queue->j + gr.index * cap : nullptr;
+  uint8_t* qi = QUEUED ? queue->image + gr.index * cap : nullptr;
+  int count = 0;
+  auto geom = [&](int j, int code, CT& d2, CT& rx, CT& ry, CT& rz) {
+    if (PERIODIC && code != 0)
+      return pair_geom<T, CT>(a, S, j, D.x, D.y, D.z, D.r2f, D.r2d, true,
+                              image_offset(code, 0, g.per[0]), image_offset(code, 1, g.per[1]),
+                              image_offset(code, 2, g.per[2]), d2, rx, ry, rz);
+    return pair_geom<T, CT>(a, S, j, D.x, D.y, D.z, D.r2f, D.r2d, false, 0.0, 0.0, 0.0, d2, rx,
+                            ry, rz);
+  };
+  auto drain = [&]() {
+    wave_lds_fence();
+    for (int k = gr.rank; __any(k - gr.rank < count); k += gr.size) {
+      if (k < count) {
+        CT d2, rx, ry, rz;
+        const int j = qj[k];
+        if (geom(j, PERIODIC ? qi[k] : 0, d2, rx, ry, rz)) body(j, d2, rx, ry, rz);
+      }
+    }
+    count = 0;
+    wave_lds_fence();
+  };
+  group_scan<PERIODIC>(g, S.cstart, gr, rows, D.local, (double)D.x, (double)D.y, (double)D.z, D.cx,
+                       D.cy, D.cz, D.ring, D.rc, [&](bool valid, int j, int code) {
+    CT d2, rx, ry, rz;
+    const bool ok = valid && geom(j, code, d2, rx, ry, rz);
+    if constexpr (QUEUED) {
+      const unsigned m = gr.mine(__ballot(ok));
+      if (ok) {
+        const int at = count + gr.before(m);
+        qj[at] = j;
+        if (PERIODIC) qi[at] = (uint8_t)code;
+      }
+      count += __popc(m);
+      if (__any(count > cap - gr.size)) drain();
+    } else {
+      if (ok) body(j, d2, rx, ry, rz);
+    }
+  });
+  if constexpr (QUEUED) drain();
+}
+
+template <typename T, typename CT, bool TAIT, bool PERIODIC>
+__global__ __launch_bounds__(kBlock) void density_kernel(Grid g, PassArgs<T> a, int log2) {
+  __shared__ GroupRows rows[kBlock / 64];
+  const Group gr(log2);
+  const GroupDst<T> D(g, a, gr, log2);
+  const int i = D.i, wid = threadIdx.x >> 6;
   const int dim = a.dim;
   CT rho = CT(0);
   for (int s = 0; s < a.nsrc; ++s) {
     const View<T> S = a.src[s];
     CT nr = CT(0);
     if (s == a.cache_src && a.cache_mode == 2) {
-      nr = (CT)a.cache_sums[i];  // stored partial sum of a static source
+      // stored partial sum of a static source
+      if (D.local) nr = (CT)a.cache_sums[i];
     } else {
-      scan_pairs<T, CT>(g, a, S, xd, yd, zd, cx, cy, cz, ring, r2f, r2d,
-                        [&](int j, CT d2, CT, CT, CT) {
-                          const CT hab = CT(0.5) * ((CT)hd + (CT)S.h[j]);
-                          const CT inv = CT(1) / hab;
-                          const CT q = sqrt(d2) * inv;
-                          nr += (CT)S.m[j] * (w_shape<CT>(q) * h_dim_inv<CT>(inv, dim));
-                        });
-      if (s == a.cache_src && a.cache_mode == 1) a.cache_sums[i] = (double)nr;
+      scan_pairs<T, CT, PERIODIC, false>(g, a, S, gr, D, rows[wid], nullptr,
+                                         [&](int j, CT d2, CT, CT, CT) {
+        const CT hab = CT(0.5) * ((CT)D.h + (CT)S.h[j]);
+        const CT inv = CT(1) / hab;
+        const CT q = sqrt(d2) * inv;
+        nr += (CT)S.m[j] * (w_shape<CT>(q) * h_dim_inv<CT>(inv, dim));
+      });
+      nr = gr.sum(nr);
+      if (s == a.cache_src && a.cache_mode == 1 && D.local && gr.rank == 0)
+        a.cache_sums[i] = (double)nr;
     }
-    if ((a.excl_self >> s) & 1u) {
+    if (((a.excl_self >> s) & 1u) && D.local) {
       // the self pair (d2 = 0, h_ab = h_a) as the scan added it
-      const CT hab = CT(0.5) * ((CT)hd + (CT)hd);
+      const CT hab = CT(0.5) * ((CT)D.h + (CT)D.h);
       const CT inv = CT(1) / hab;
       nr -= (CT)S.m[i] * (w_shape<CT>(sqrt(CT(0)) * inv) * h_dim_inv<CT>(inv, dim));
     }
     rho += nr;
+  }
+  if (!D.valid || gr.rank != 0) return;
+  if (!D.local) {
+    a.rho[i] = T(0);
+    if (TAIT) {
+      a.p[i] = T(0);
+      a.cs[i] = T(0);
+    }
+    return;
   }
   rho *= (CT)a.fac1;
   a.rho[i] = (T)rho;
@@ -98,43 +180,38 @@ __global__ __launch_bounds__(kBlock) void density_kernel(Grid g, PassArgs<T> a) 
 
 // SPHDensityRate (density_funcs.pyx:89-158): sum_b m_b (v_a - v_b) .
 // grad_a W_ab with h_ab = (h_a + h_b)/2; non-LocalReal destinations get 0.
-template <typename T, typename CT>
-__global__ __launch_bounds__(kBlock) void density_rate_kernel(Grid g, PassArgs<T> a) {
-  const int bid = xcd_block(blockIdx.x, gridDim.x);
-  const int i = bid * kBlock + threadIdx.x;
-  if (i >= a.dst.n) return;
-  if (a.dst.tag != nullptr && a.dst.tag[i] != 0) {
-    a.rate[i] = T(0);
-    return;
+template <typename T, typename CT, bool PERIODIC>
+__global__ __launch_bounds__(kBlock) void density_rate_kernel(Grid g, PassArgs<T> a, int log2) {
+  __shared__ GroupRows rows[kBlock / 64];
+  __shared__ GroupQueue queue[kBlock / 64];
+  const Group gr(log2);
+  const GroupDst<T> D(g, a, gr, log2);
+  const int i = D.i, wid = threadIdx.x >> 6;
+  T ud = T(0), vd = T(0), wd = T(0);
+  if (D.local) {
+    ud = a.dst.u[i];
+    vd = a.dst.v[i];
+    wd = a.dst.w[i];
   }
-  const T xd = a.dst.x[i], yd = a.dst.y[i], zd = a.dst.z[i];
-  const T ud = a.dst.u[i], vd = a.dst.v[i], wd = a.dst.w[i];
-  const CT ha = (CT)a.dst.h[i];
-  const double r = (double)a.dst.h[i] * a.rs;
-  const double r2d = r * r;
-  const float r2f = (float)r2d;
-  int cx, cy, cz;
-  cell_xyz(a.dst.cell[i], g, cx, cy, cz);
-  const int ring = ring_of(g, a.disp);
+  const CT ha = (CT)D.h;
   const int dim = a.dim;
   CT rate = CT(0);
   for (int s = 0; s < a.nsrc; ++s) {
     const View<T> S = a.src[s];
     CT nr = CT(0);
-    scan_pairs<T, CT>(g, a, S, xd, yd, zd, cx, cy, cz, ring, r2f, r2d,
-                      [&](int j, CT d2, CT rx, CT ry, CT rz) {
-                        const CT hab = CT(0.5) * (ha + (CT)S.h[j]);
-                        const CT inv = CT(1) / hab;
-                        const CT rr = sqrt(d2);
-                        const CT q = rr * inv;
-                        const CT gf = grad_shape<CT>(q, rr, hab, inv) * h_dim_inv<CT>(inv, dim);
-                        const CT vx = (CT)ud - (CT)S.u[j], vy = (CT)vd - (CT)S.v[j],
-                                 vz = (CT)wd - (CT)S.w[j];
-                        nr += (vx * rx + vy * ry + vz * rz) * gf * (CT)S.m[j];
-                      });
-    rate += nr;
+    scan_pairs<T, CT, PERIODIC, true>(g, a, S, gr, D, rows[wid], &queue[wid],
+                                      [&](int j, CT d2, CT rx, CT ry, CT rz) {
+      const CT hab = CT(0.5) * (ha + (CT)S.h[j]);
+      const CT inv = CT(1) / hab;
+      const CT rr = sqrt(d2);
+      const CT q = rr * inv;
+      const CT gf = grad_shape<CT>(q, rr, hab, inv) * h_dim_inv<CT>(inv, dim);
+      const CT vx = (CT)ud - (CT)S.u[j], vy = (CT)vd - (CT)S.v[j], vz = (CT)wd - (CT)S.w[j];
+      nr += (vx * rx + vy * ry + vz * rz) * gf * (CT)S.m[j];
+    });
+    rate += gr.sum(nr);
   }
-  a.rate[i] = (T)(rate * (CT)a.fac1);
+  if (D.valid && gr.rank == 0) a.rate[i] = D.local ? (T)(rate * (CT)a.fac1) : T(0);
 }
 
 template <typename T>
@@ -158,85 +235,87 @@ __global__ __launch_bounds__(kBlock) void tait_kernel(int n, const T* __restrict
 
 // MODE 0: write acc / dv.  MODE 1: RK2 predictor.  MODE 2: RK2 final.
 // MODE 3: Euler.
-template <typename T, typename CT, int MODE>
-__global__ __launch_bounds__(kBlock) void momentum_kernel(Grid g, PassArgs<T> a) {
-  const int bid = xcd_block(blockIdx.x, gridDim.x);
-  const int i = bid * kBlock + threadIdx.x;
-  if (i >= a.dst.n) return;
+template <typename T, typename CT, int MODE, bool PERIODIC>
+__global__ __launch_bounds__(kBlock) void momentum_kernel(Grid g, PassArgs<T> a, int log2) {
+  __shared__ GroupRows rows[kBlock / 64];
+  __shared__ GroupQueue queue[kBlock / 64];
+  const Group gr(log2);
+  const GroupDst<T> D(g, a, gr, log2);
+  const int i = D.i, wid = threadIdx.x >> 6;
   const int dim = a.dim;
-  const bool local = a.dst.tag == nullptr || a.dst.tag[i] == 0;
+  const bool local = D.local;
   CT acc[3] = {CT(0), CT(0), CT(0)};
   CT dv[3] = {CT(0), CT(0), CT(0)};
-  const T xd = a.dst.x[i], yd = a.dst.y[i], zd = a.dst.z[i];
-  const T ud = a.dst.u[i], vd = a.dst.v[i], wd = a.dst.w[i];
+  T ud = T(0), vd = T(0), wd = T(0);
+  CT rhoa = CT(0), ca = CT(0), Aa = CT(0);
+  if (D.valid) {
+    ud = a.dst.u[i];
+    vd = a.dst.v[i];
+    wd = a.dst.w[i];
+  }
   if (local) {
-    const CT ha = (CT)a.dst.h[i];
-    const CT rhoa = (CT)a.dst.rho[i];
-    const CT Pa = (CT)a.dst.p[i];
-    const CT ca = (CT)a.dst.cs[i];
-    const CT Aa = Pa / (rhoa * rhoa);
-    const double r = (double)a.dst.h[i] * a.rs;
-    const double r2d = r * r;
-    const float r2f = (float)r2d;
-    int cx, cy, cz;
-    cell_xyz(a.dst.cell[i], g, cx, cy, cz);
-    const int ring = ring_of(g, a.disp);
-    const CT alpha = (CT)a.alpha, beta = (CT)a.beta, eta2 = (CT)(a.eta * a.eta);
-    for (int s = 0; s < a.nsrc; ++s) {
-      const View<T> S = a.src[s];
-      const bool do_m = (a.flags[s] & SPH_SRC_MOMENTUM) != 0 && a.do_mom;
-      const bool do_x = (a.flags[s] & SPH_SRC_XSPH) != 0 && a.do_xsph;
-      if (!do_m && !do_x) continue;
-      CT am[3] = {CT(0), CT(0), CT(0)};
-      CT ax[3] = {CT(0), CT(0), CT(0)};
-      scan_pairs<T, CT>(g, a, S, xd, yd, zd, cx, cy, cz, ring, r2f, r2d,
-                        [&](int j, CT d2, CT rx, CT ry, CT rz) {
-          const CT hab = CT(0.5) * (ha + (CT)S.h[j]);
-          const CT inv = CT(1) / hab;
-          const CT rr = sqrt(d2);
-          const CT q = rr * inv;
-          const CT fac = h_dim_inv<CT>(inv, dim);
-          const CT mb = (CT)S.m[j];
-          const CT rhob = (CT)S.rho[j];
-          if (do_m) {
-            const CT vx = (CT)ud - (CT)S.u[j], vy = (CT)vd - (CT)S.v[j],
-                     vz = (CT)wd - (CT)S.w[j];
-            const CT dot = vx * rx + vy * ry + vz * rz;
-            const CT Pb = (CT)S.p[j];
-            CT tmp = Aa + Pb / (rhob * rhob);
-            if (dot < CT(0)) {
-              const CT cab = CT(0.5) * (ca + (CT)S.cs[j]);
-              const CT rhoab = CT(0.5) * (rhoa + rhob);
-              const CT mu = hab * dot / (d2 + eta2 * hab * hab);
-              tmp += (-alpha * cab * mu + beta * mu * mu) / rhoab;
-            }
-            const CT gf = -mb * tmp * (grad_shape<CT>(q, rr, hab, inv) * fac);
-            am[0] += gf * rx;
-            am[1] += gf * ry;
-            am[2] += gf * rz;
-          }
-          if (do_x) {
-            const CT rhoab = CT(0.5) * (rhob + rhoa);
-            const CT temp = mb * (w_shape<CT>(q) * fac) / rhoab;
-            ax[0] += temp * ((CT)S.u[j] - (CT)ud);
-            ax[1] += temp * ((CT)S.v[j] - (CT)vd);
-            ax[2] += temp * ((CT)S.w[j] - (CT)wd);
-          }
-      });
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        acc[c] += am[c];
-        dv[c] += ax[c];
+    rhoa = (CT)a.dst.rho[i];
+    ca = (CT)a.dst.cs[i];
+    Aa = (CT)a.dst.p[i] / (rhoa * rhoa);
+  }
+  const CT ha = (CT)D.h;
+  const CT alpha = (CT)a.alpha, beta = (CT)a.beta, eta2 = (CT)(a.eta * a.eta);
+  for (int s = 0; s < a.nsrc; ++s) {
+    const View<T> S = a.src[s];
+    const bool do_m = (a.flags[s] & SPH_SRC_MOMENTUM) != 0 && a.do_mom;
+    const bool do_x = (a.flags[s] & SPH_SRC_XSPH) != 0 && a.do_xsph;
+    if (!do_m && !do_x) continue;
+    CT am[3] = {CT(0), CT(0), CT(0)};
+    CT ax[3] = {CT(0), CT(0), CT(0)};
+    scan_pairs<T, CT, PERIODIC, true>(g, a, S, gr, D, rows[wid], &queue[wid],
+                                      [&](int j, CT d2, CT rx, CT ry, CT rz) {
+      const CT hab = CT(0.5) * (ha + (CT)S.h[j]);
+      const CT inv = CT(1) / hab;
+      const CT rr = sqrt(d2);
+      const CT q = rr * inv;
+      const CT fac = h_dim_inv<CT>(inv, dim);
+      const CT mb = (CT)S.m[j];
+      const CT rhob = (CT)S.rho[j];
+      const CT rhoab = CT(0.5) * (rhoa + rhob);
+      // v_b - v_a = -(v_a - v_b) exactly: one difference serves both sums
+      const CT vx = (CT)ud - (CT)S.u[j], vy = (CT)vd - (CT)S.v[j], vz = (CT)wd - (CT)S.w[j];
+      if (do_m) {
+        const CT dot = vx * rx + vy * ry + vz * rz;
+        const CT Pb = (CT)S.p[j];
+        CT tmp = Aa + Pb / (rhob * rhob);
+        if (dot < CT(0)) {
+          const CT cab = CT(0.5) * (ca + (CT)S.cs[j]);
+          const CT mu = hab * dot / (d2 + eta2 * hab * hab);
+          tmp += (-alpha * cab * mu + beta * mu * mu) / rhoab;
+        }
+        const CT gf = -mb * tmp * (grad_shape<CT>(q, rr, hab, inv) * fac);
+        am[0] += gf * rx;
+        am[1] += gf * ry;
+        am[2] += gf * rz;
       }
-    }
-    const CT f1 = (CT)a.fac1, fe = (CT)(a.fac1 * a.eps);
+      if (do_x) {
+        const CT temp = mb * (w_shape<CT>(q) * fac) / rhoab;
+        ax[0] += temp * -vx;
+        ax[1] += temp * -vy;
+        ax[2] += temp * -vz;
+      }
+    });
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      acc[c] *= f1;
-      dv[c] *= fe;
+      acc[c] += gr.sum(am[c]);
+      dv[c] += gr.sum(ax[c]);
     }
   }
+  const CT f1 = (CT)a.fac1, fe = (CT)(a.fac1 * a.eps);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    acc[c] *= f1;
+    dv[c] *= fe;
+  }
+  // one lane of the group writes (the others stay for the wave reduction)
+  const bool writer = D.valid && gr.rank == 0;
   if (MODE == 0) {
+    if (!writer) return;
     // components >= dim are written (as 0) when the caller passes them,
     // like the reference's num_outputs = 3 in a 2D run
     for (int c = 0; c < 3; ++c) {
@@ -252,7 +331,7 @@ __global__ __launch_bounds__(kBlock) void momentum_kernel(Grid g, PassArgs<T> a)
   const T hdt = (T)(0.5 * a.dt);
   const T vel[3] = {ud, vd, wd};
   double mv2 = 0.0;
-  for (int c = 0; c < dim; ++c) {
+  for (int c = 0; writer && c < dim; ++c) {
     const T x0 = a.s0[c][i];
     const T u0 = a.s0[3 + c][i];
     const T km = (T)acc[c];
@@ -332,32 +411,75 @@ static int32_t check_common(const sph_grid* g, const sph_params* prm, const sph_
 }
 
 
+// Lanes per destination (log2).  Eight is the best split from 16k particles
+// on (FP64 momentum of 40k particles in 2D: 82 / 68 / 77 us with 4 / 8 / 16
+// lanes, FP32 periodic in 3D, 100k: 231 / 197 / 220 us, FP64 density of 300k:
+// 349 us with 8, 375 with 4); smaller sets have too few waves and take 16
+// (5k: 18.8 / 13.3 / 12.1 us).  Two sources cull every row twice, which
+// fewer groups per wave make dearer: 4 lanes once the waves suffice (dam
+// break of 60k + 15k, FP64 momentum: 146 / 171 / 213 us; density 66 / 68 / 76).
+static int group_log2(int64_t n, int nsrc) {
+  if (n < (1 << 14)) return 4;
+  return nsrc >= 2 && n >= (1 << 15) ? 2 : 3;
+}
+
+static int group_blocks(int64_t n, int log2) {
+  return (int)((n + (kBlock >> log2) - 1) / (kBlock >> log2));
+}
+
 template <typename T, typename CT>
 static void launch_density(hipStream_t st, const Grid& G, const PassArgs<T>& a, bool tait) {
-  const int nb = nblocks_for(a.dst.n);
-  if (tait)
-    hipLaunchKernelGGL((density_kernel<T, CT, true>), dim3(nb), dim3(kBlock), 0, st, G, a);
+  const int k = group_log2(a.dst.n, a.nsrc);
+  const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
+  if (G.periodic) {
+    if (tait)
+      hipLaunchKernelGGL((density_kernel<T, CT, true, true>), nb, th, 0, st, G, a, k);
+    else
+      hipLaunchKernelGGL((density_kernel<T, CT, false, true>), nb, th, 0, st, G, a, k);
+  } else {
+    if (tait)
+      hipLaunchKernelGGL((density_kernel<T, CT, true, false>), nb, th, 0, st, G, a, k);
+    else
+      hipLaunchKernelGGL((density_kernel<T, CT, false, false>), nb, th, 0, st, G, a, k);
+  }
+}
+
+template <typename T, typename CT>
+static void launch_rate(hipStream_t st, const Grid& G, const PassArgs<T>& a) {
+  const int k = group_log2(a.dst.n, a.nsrc);
+  const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
+  if (G.periodic)
+    hipLaunchKernelGGL((density_rate_kernel<T, CT, true>), nb, th, 0, st, G, a, k);
   else
-    hipLaunchKernelGGL((density_kernel<T, CT, false>), dim3(nb), dim3(kBlock), 0, st, G, a);
+    hipLaunchKernelGGL((density_rate_kernel<T, CT, false>), nb, th, 0, st, G, a, k);
+}
+
+template <typename T, typename CT, bool PERIODIC>
+static void launch_momentum_p(hipStream_t st, const Grid& G, const PassArgs<T>& a, int mode) {
+  const int k = group_log2(a.dst.n, a.nsrc);
+  const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
+  switch (mode) {
+    case 0:
+      hipLaunchKernelGGL((momentum_kernel<T, CT, 0, PERIODIC>), nb, th, 0, st, G, a, k);
+      break;
+    case 1:
+      hipLaunchKernelGGL((momentum_kernel<T, CT, 1, PERIODIC>), nb, th, 0, st, G, a, k);
+      break;
+    case 2:
+      hipLaunchKernelGGL((momentum_kernel<T, CT, 2, PERIODIC>), nb, th, 0, st, G, a, k);
+      break;
+    default:
+      hipLaunchKernelGGL((momentum_kernel<T, CT, 3, PERIODIC>), nb, th, 0, st, G, a, k);
+      break;
+  }
 }
 
 template <typename T, typename CT>
 static void launch_momentum(hipStream_t st, const Grid& G, const PassArgs<T>& a, int mode) {
-  const int nb = nblocks_for(a.dst.n);
-  switch (mode) {
-    case 0:
-      hipLaunchKernelGGL((momentum_kernel<T, CT, 0>), dim3(nb), dim3(kBlock), 0, st, G, a);
-      break;
-    case 1:
-      hipLaunchKernelGGL((momentum_kernel<T, CT, 1>), dim3(nb), dim3(kBlock), 0, st, G, a);
-      break;
-    case 2:
-      hipLaunchKernelGGL((momentum_kernel<T, CT, 2>), dim3(nb), dim3(kBlock), 0, st, G, a);
-      break;
-    default:
-      hipLaunchKernelGGL((momentum_kernel<T, CT, 3>), dim3(nb), dim3(kBlock), 0, st, G, a);
-      break;
-  }
+  if (G.periodic)
+    launch_momentum_p<T, CT, true>(st, G, a, mode);
+  else
+    launch_momentum_p<T, CT, false>(st, G, a, mode);
 }
 
 template <typename T>
@@ -504,11 +626,10 @@ static int32_t density_rate_impl(hipStream_t st, const sph_grid* g, const sph_pa
   Grid G = make_grid(*g, rmax);
   if (dst->n == 0) return SPH_OK;
   SPH_TRY(check_period(g, rmax, "sph_density_rate"));
-  const int nb = nblocks_for(a.dst.n);
   if (sizeof(T) == 4 && prm->pair_prec == SPH_PAIR_F64)
-    hipLaunchKernelGGL((density_rate_kernel<T, double>), dim3(nb), dim3(kBlock), 0, st, G, a);
+    launch_rate<T, double>(st, G, a);
   else
-    hipLaunchKernelGGL((density_rate_kernel<T, T>), dim3(nb), dim3(kBlock), 0, st, G, a);
+    launch_rate<T, T>(st, G, a);
   return launch_status("sph_density_rate");
 }
 

@@ -1,0 +1,123 @@
+"""The SoA passes' group scan (4, 8 or 16 lanes per destination) at the sizes
+where it can go wrong, against the FP64 oracle on the same stored bits.
+
+The lanes of a group share a list of stencil rows and a queue of accepted
+sources in LDS, both flushed when nearly full: particle counts around whole
+waves and around the sizes where the lane count changes, more rows than the
+list holds (bins much smaller than the search radius), more neighbours than
+the queue holds (dense points), one and two sources, far coordinates that the
+FP32 cull cannot represent.  FP64 storage within 1e-12 (sums of at most 1e3
+terms of one sign per particle: 1e3 * 2^-53 = 1.1e-13 relative; accelerations
+normwise)."""
+import numpy as np
+import pytest
+
+import pysph_amd.base.api as base
+import pysph_amd.solver.api as solver
+import pysph_amd.sph.api as sph
+from oracle import oracle as O
+from tests.util import max_rel, rel_norm, to_oracle
+
+pytestmark = pytest.mark.gpu
+Fluid = base.ParticleType.Fluid
+Solid = base.ParticleType.Solid
+
+
+def _points(n, dim, h, seed, ptype, spread=1.0, at=0.0):
+    rng = np.random.Generator(np.random.PCG64(seed))
+    pos = at + spread * rng.random((3, n))
+    pos[dim:] = 0.0
+    vel = rng.normal(size=(3, n))
+    vel[dim:] = 0.0
+    return base.get_particle_array(
+        name="p%d" % seed, type=ptype, x=pos[0], y=pos[1], z=pos[2], u=vel[0], v=vel[1],
+        w=vel[2], h=np.full(n, h), m=0.5 + rng.random(n), rho=1000.0 + 10 * rng.random(n),
+        p=1e3 * rng.random(n), cs=10.0 + rng.random(n))
+
+
+def _check(arrays, dim, min_cell_size=-1, varh=False):
+    f = arrays[0]
+    particles = base.Particles(arrays, min_cell_size=min_cell_size, variable_h=varh)
+    cs = particles.cell_manager.cell_size
+    kernel = base.CubicSplineKernel(dim=dim)
+    for nm in ("o0", "o1", "o2"):
+        f.add_property({"name": nm})
+    types = [Fluid, Solid][:len(arrays)]
+    refs = [to_oracle(a, k) for k, a in enumerate(arrays)]
+    op = solver.SPHOperation(sph.SPHRho.withargs(), on_types=[Fluid], from_types=types,
+                             updates=["rho"], id="rho")
+    op.get_calcs(particles, kernel)[0].sph("o0")
+    ref = O.sphrho(dim, refs[0], refs, cell_size=cs)
+    assert max_rel(f.get("o0"), ref) < 1e-12
+    ups = ["u", "v", "w"][:dim]
+    op = solver.SPHIntegration(sph.MomentumEquation.withargs(alpha=0.5, beta=0.5, eta=0.1,
+                                                             dim=dim),
+                               on_types=[Fluid], from_types=types, updates=ups, id="mom")
+    op.get_calcs(particles, kernel)[0].sph(*["o0", "o1", "o2"][:dim])
+    got = np.stack([f.get(nm) for nm in ["o0", "o1", "o2"][:dim]])
+    ref = O.momentum(dim, refs[0], refs, alpha=0.5, beta=0.5, eta=0.1, cell_size=cs)[:dim]
+    if np.linalg.norm(ref) > 0:
+        assert rel_norm(got, ref) < 1e-12
+    else:
+        assert not got.any()
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 63, 64, 65, 255, 257])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_small_counts(n, dim):
+    _check([_points(n, dim, 0.1, n, Fluid)], dim)
+
+
+@pytest.mark.parametrize("n", [(1 << 14) - 1, 1 << 14, (1 << 15) - 1, 1 << 15])
+def test_counts_where_the_lanes_change(n):
+    h = 0.5 * (20 / (np.pi * n)) ** 0.5
+    _check([_points(n, 2, h, 1, Fluid), _points(n // 3, 2, h, 2, Solid)], 2)
+
+
+@pytest.mark.parametrize("n,dim,h", [(3000, 2, 0.15), (3000, 3, 0.25), (17000, 2, 0.05)])
+def test_more_neighbours_than_the_queue_holds(n, dim, h):
+    # 200 to 700 neighbours per particle; the queues hold 256 (128 from 16k
+    # particles on)
+    _check([_points(n, dim, h, 5, Fluid)], dim)
+
+
+@pytest.mark.parametrize("n", [700, 17000])
+def test_more_rows_than_the_list_holds(n):
+    # search radius of 7 cells, 14 bins: up to 29 x 29 rows, lists of 128 / 64
+    h = 0.14 if n < 1000 else 0.035
+    _check([_points(n, 3, h, 6, Fluid)], 3, min_cell_size=2 * h / 7)
+
+
+def test_points_beyond_the_cull_take_the_whole_ring():
+    # 1e31: outside the range the FP32 cull is used in; the cells, the test
+    # and the sums are FP64
+    a = _points(200, 2, 1e30, 7, Fluid, spread=1e31)
+    a.set(m=np.full(200, 1e60))
+    particles = base.Particles([a])
+    kernel = base.CubicSplineKernel(dim=2)
+    op = solver.SPHOperation(sph.SPHRho.withargs(), on_types=[Fluid], from_types=[Fluid],
+                             updates=["rho"], id="rho")
+    op.get_calcs(particles, kernel)[0].sph("rho")
+    ref = O.sphrho(2, to_oracle(a), [to_oracle(a)],
+                   cell_size=particles.cell_manager.cell_size)
+    assert max_rel(a.get("rho"), ref) < 1e-12
+
+
+def test_mixed_radii_symmetric():
+    a = _points(5000, 2, 0.01, 8, Fluid)
+    rng = np.random.Generator(np.random.PCG64(9))
+    a.set(h=0.01 * (1 + 4 * rng.random(5000) ** 4))
+    particles = base.Particles([a], variable_h=True)
+    kernel = base.CubicSplineKernel(dim=2)
+    op = solver.SPHOperation(sph.SPHRho.withargs(), on_types=[Fluid], from_types=[Fluid],
+                             updates=["rho"], id="rho")
+    op.get_calcs(particles, kernel)[0].sph("rho")
+    # every pair within the larger of the two radii, brute force
+    x, y, h, m = (a.get(c) for c in ("x", "y", "h", "m"))
+    r = np.sqrt((x[:, None] - x) ** 2 + (y[:, None] - y) ** 2)
+    hab = 0.5 * (h[:, None] + h)
+    q = r / hab
+    w = 10.0 / (7.0 * np.pi * hab ** 2) * np.where(
+        q > 2, 0.0, np.where(q > 1, 0.25 * (2 - q) ** 3, 1 - 1.5 * q * q * (1 - 0.5 * q)))
+    w[r >= 2 * np.maximum(h[:, None], h)] = 0.0
+    assert max_rel(a.get("rho"), (m * w).sum(1)) < 1e-12
