@@ -54,6 +54,15 @@ __device__ __forceinline__ float move_bound(double mv2) {
   return (float)(sqrt(mv2) * (1.0 + 1e-6));
 }
 
+// *out = max(*out, v) for non-negative floats and NaN, ordered as integers
+// (NaN last).  The value is read first: it only grows, so a stale value costs
+// an atomic and skips none, and most callers find a larger one there already.
+__device__ __forceinline__ void raise_max(float* out, float v) {
+  int* p = (int*)out;
+  if (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < __float_as_int(v))
+    atomicMax(p, __float_as_int(v));
+}
+
 // Stencil ring: ceil(r/cs) cells (cell.pyx:1127-1129) widened by the largest
 // displacement since binning, so that a binning stays exact when reused.
 __device__ __forceinline__ int ring_of(const Grid& g, const float* disp) {

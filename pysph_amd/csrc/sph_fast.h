@@ -921,7 +921,7 @@ __device__ __forceinline__ void mom_epilogue(const PassArgs<float>& a, int i, bo
   if (a.disp_out != nullptr) {
     float disp = move_bound(mv2);
     for (int off = 32; off > 0; off >>= 1) disp = fmaxf(disp, __shfl_xor(disp, off, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax((int*)a.disp_out, __float_as_int(disp));
+    if ((threadIdx.x & 63) == 0) raise_max(a.disp_out, disp);
   }
 }
 
