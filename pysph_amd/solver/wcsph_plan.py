@@ -11,7 +11,8 @@ density):
     PositionStepping on F                      (integrates x, y[, z])
     XSPHCorrection   on F, optional            (integrates x, y[, z])
 
-Per RK2 step the plan issues, on one stream (FP32 storage, the defaults):
+Per RK2 step the plan issues, on one stream (FP32 storage, the defaults;
+FP64 storage the same without the packs, one density launch per array):
 
     re-bin F (counting sort + permutation)          sph_bin / sph_permute
     pack F's float4 copies                          sph_pack
@@ -105,8 +106,7 @@ class WCSPHPlan:
         self.list_skin = 0.0
         # stage2_rebin: re-bin the moving array by X1 before stage 2 (the
         # reference rebuilds its caches after the predictor).  Off, stage 2
-        # keeps the stage-1 binning and the packed passes widen their
-        # stencil by the predictor's largest displacement (measured on the
+        # keeps the stage-1 binning and the passes widen their stencil by the predictor's largest displacement (measured on the
         # device by the stage-1 kernel), which skips one binning and
         # permutation per step; the neighbour sets are the same.
         self.stage2_rebin = False
@@ -492,9 +492,11 @@ class WCSPHPlan:
         self._pack_all()
         ov = self._override()
         # lists built anew in stage 2 need the X1 binning (their validity
-        # check reads the same displacement as the widened stencil)
+        # check reads the same displacement as the widened stencil); periodic
+        # positions are wrapped at a binning, so X1 gets one there
         keep_binning = (self.use_list and self.list_reuse) or (
-            self.use_packed and not self.stage2_rebin and not self.use_list)
+            not self.stage2_rebin and not self.use_list and
+            self.cm.periodic_domain is None)
         if keep_binning:
             # stage 2 keeps the binning: the stage-1 kernel records the
             # predictor's largest displacement on the device, and the stage-2
@@ -504,11 +506,18 @@ class WCSPHPlan:
             # displacement stays within the list skin
             stream = require_gpu(b["disp"])
             _abi.call("sph_fill_i32", stream, b["disp"].data_ptr(), 1, 0)
-            self._density(override=ov, list_mode=0)
+            # the SoA passes get the (zero) displacement in stage 1 too, so
+            # that both stages sum the same way (source caches keep the bits)
+            d1 = None if self.use_packed else b["disp"]
+            self._density(disp=d1, override=ov, list_mode=0)
             probe("density1", b, ov)
             self._stage(1, dt, b, override=ov, disp_out=b["disp"])
             probe("stage1", b, ov)
             s1 = self._s1_fields(b)
+            if not self.use_packed:
+                # the SoA passes' stage 2 still counts jumps at X1, as their
+                # re-binning did
+                self.cm.check_moved(self.fluid, [s1[c] for c in ("x", "y", "z")])
             self._pack(self.fluid, fields=s1, force=True)
             ov = self._override(s1)
             self._density(disp=b["disp"], override=ov, list_mode=1)
