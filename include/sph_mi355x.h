@@ -284,6 +284,22 @@ int32_t sph_varh_neighbor_fill(void *stream, const sph_grid *g, const sph_view *
                                int64_t *nbrs_dev, int64_t cap, int64_t total,
                                int64_t *needed_host);
 
+/* ---- the same sets with rows in the callers' own numbering: row
+ *      dst_ids_dev[i] belongs to destination slot i (NULL: row i), entries
+ *      are src_ids_dev[j] (NULL: j) sorted ascending.  rmax > 0 selects the
+ *      symmetric variable-h sets, as above.  counts_dev[row] is written for
+ *      every row; offsets_dev is its exclusive scan.  With self_last (src is
+ *      dst, equal ids) a row's own id then changes places with the row's
+ *      last entry (nnps.pyx:612-618).  cap < total -> SPH_ECAPACITY. --------------- */
+int32_t sph_neighbor_row_counts(void *stream, const sph_grid *g, const sph_view *dst,
+                                const sph_view *src, double radius_scale, double rmax,
+                                const int64_t *dst_ids_dev, int64_t *counts_dev);
+int32_t sph_neighbor_row_fill(void *stream, const sph_grid *g, const sph_view *dst,
+                              const sph_view *src, double radius_scale, double rmax,
+                              const int64_t *dst_ids_dev, const int64_t *src_ids_dev,
+                              const int64_t *offsets_dev, int64_t *nbrs_dev, int64_t cap,
+                              int64_t total, int32_t self_last);
+
 /* ---- neighbour passes -------------------------------------------------- */
 
 /* Optional neighbour list of one destination array, built by a density

@@ -166,6 +166,12 @@ _SIGS = {
                                                 ctypes.c_double, ctypes.c_double, _vp, _vp,
                                                 _vp, ctypes.c_int64, ctypes.c_int64,
                                                 _P(ctypes.c_int64)]),
+    "sph_neighbor_row_counts": (ctypes.c_int32, [_vp, _P(SphGrid), _P(SphView), _P(SphView),
+                                                 ctypes.c_double, ctypes.c_double, _vp, _vp]),
+    "sph_neighbor_row_fill": (ctypes.c_int32, [_vp, _P(SphGrid), _P(SphView), _P(SphView),
+                                               ctypes.c_double, ctypes.c_double, _vp, _vp, _vp,
+                                               _vp, ctypes.c_int64, ctypes.c_int64,
+                                               ctypes.c_int32]),
     "sph_density_rate": (ctypes.c_int32, [_vp, _P(SphGrid), _P(SphParams), _P(SphView),
                                           ctypes.c_int32, _P(SphView), ctypes.c_double, _vp,
                                           _vp]),

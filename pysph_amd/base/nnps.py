@@ -17,7 +17,7 @@ import numpy as np
 import torch
 
 from .. import _abi
-from .._device import require_gpu
+from .._device import ptr, require_gpu
 from .carray import LongArray
 from .particle_array import ParticleArray
 
@@ -28,41 +28,13 @@ class NeighborLocatorType:
     NSquareNeighborLocator = 2
 
 
-def _csr_user_order(pa_dst, off_slot, nbr, n):
-    """Reorder CSR rows from destination slot order to user order."""
-    order = pa_dst._order_np()
-    counts = np.diff(off_slot)
-    if order is None:
-        return off_slot, nbr
-    ucounts = np.empty_like(counts)
-    ucounts[order] = counts
-    uoff = np.zeros(n + 1, dtype=np.int64)
-    np.cumsum(ucounts, out=uoff[1:])
-    # entry e of slot row s moves to uoff[order[s]] + (e - off_slot[s])
-    row = np.repeat(np.arange(n, dtype=np.int64), counts)
-    dest = uoff[order[row]] + (np.arange(len(nbr), dtype=np.int64) - off_slot[row])
-    out = np.empty_like(nbr)
-    out[dest] = nbr
-    return uoff, out
-
-
-def _self_last(off, nb):
-    """Move each row's own index to the row's last slot (nnps.pyx:612-618);
-    rows hold an index at most once."""
-    n = len(off) - 1
-    row = np.repeat(np.arange(n, dtype=np.int64), np.diff(off))
-    pos = np.nonzero(nb == row)[0]
-    last = off[row[pos] + 1] - 1
-    nb[pos] = nb[last]
-    nb[last] = row[pos]
-    return nb
-
-
-def neighbor_csr(cell_manager, src, dst, radius_scale, symmetric=False):
+def neighbor_csr(cell_manager, src, dst, radius_scale, symmetric=False, self_last=False):
     """All neighbour lists of dst from src on the GPU: (offsets, nbrs) in user
     index space, rows in user order, each row sorted ascending.  With
     `symmetric` the rows are the variable-h sets of VarHNbrParticleLocator
-    (nnps.pyx:654-749): d2 < (h_dst rs)^2 or d2 < (h_src rs)^2."""
+    (nnps.pyx:654-749): d2 < (h_dst rs)^2 or d2 < (h_src rs)^2.  `self_last`
+    (src is dst) lets each row's own index change places with its last entry
+    (nnps.pyx:612-618).  The arrays are host copies in page-locked memory."""
     cm = cell_manager
     cm.update()
     n = dst.get_number_of_particles()
@@ -70,36 +42,32 @@ def neighbor_csr(cell_manager, src, dst, radius_scale, symmetric=False):
         return np.zeros(1, dtype=np.int64), np.zeros(0, dtype=np.int64)
     stream = require_gpu(dst.get_carray("x"))
     dev = dst.device
-    counts = torch.empty(n, dtype=torch.int64, device=dev)
     vd = dst.view()
     vs = src.view()
-    if symmetric:
-        rmax = float(radius_scale) * cm.max_h
-        _abi.call("sph_varh_neighbor_counts", stream, cm.grid, vd, vs, float(radius_scale),
-                  rmax, counts.data_ptr())
-    else:
-        _abi.call("sph_neighbor_counts", stream, cm.grid, vd, vs, float(radius_scale),
-                  counts.data_ptr())
+    rs = float(radius_scale)
+    rmax = rs * cm.max_h if symmetric else 0.0
+    if symmetric and not rmax > 0:
+        raise _abi.SphError("neighbor_csr", _abi.SPH_EINVAL,
+                            "variable-h sets need a positive smoothing length")
+    counts = torch.empty(n, dtype=torch.int64, device=dev)
     offsets = torch.empty(n + 1, dtype=torch.int64, device=dev)
+    _abi.call("sph_neighbor_row_counts", stream, cm.grid, vd, vs, rs, rmax, ptr(dst._order),
+              counts.data_ptr())
     total = _abi.ctypes.c_int64(0)
     _abi.call("sph_scan_counts", stream, n, counts.data_ptr(), offsets.data_ptr(),
               _abi.ctypes.byref(total))
     total = int(total.value)
-    nbrs = torch.empty(max(total, 1), dtype=torch.int64, device=dev)
-    ids = src._order if src._order is not None else torch.arange(
-        src.get_number_of_particles(), dtype=torch.int64, device=dev)
-    needed = _abi.ctypes.c_int64(0)
-    if symmetric:
-        _abi.call("sph_varh_neighbor_fill", stream, cm.grid, vd, vs, float(radius_scale),
-                  rmax, ids.data_ptr(), offsets.data_ptr(), nbrs.data_ptr(), total, total,
-                  _abi.ctypes.byref(needed))
-    else:
-        _abi.call("sph_neighbor_fill", stream, cm.grid, vd, vs, float(radius_scale),
-                  ids.data_ptr(), offsets.data_ptr(), nbrs.data_ptr(), total, total,
-                  _abi.ctypes.byref(needed))
-    off = offsets.cpu().numpy()
-    nb = nbrs[:total].cpu().numpy()
-    return _csr_user_order(dst, off, nb, n)
+    off = torch.empty(n + 1, dtype=torch.int64, pin_memory=True)
+    off.copy_(offsets, non_blocking=True)
+    nb = torch.empty(total, dtype=torch.int64, pin_memory=True)
+    if total:
+        nbrs = torch.empty(total, dtype=torch.int64, device=dev)
+        _abi.call("sph_neighbor_row_fill", stream, cm.grid, vd, vs, rs, rmax, ptr(dst._order),
+                  ptr(src._order), offsets.data_ptr(), nbrs.data_ptr(), total, total,
+                  int(bool(self_last)))
+        nb.copy_(nbrs, non_blocking=True)
+    torch.cuda.current_stream(dev).synchronize()
+    return off.numpy(), nb.numpy()
 
 
 class NbrParticleLocatorBase:
@@ -162,10 +130,8 @@ class FixedDestNbrParticleLocator(NbrParticleLocatorBase):
                 self.is_dirty = True
         if self.is_dirty or self._off is None:
             off, nb = neighbor_csr(self.cell_manager, self.source, self.dest,
-                                   self.radius_scale, symmetric=self.symmetric)
-            if self.source is self.dest:
-                # keep the particle itself in the last slot (nnps.pyx:612-618)
-                nb = _self_last(off, nb)
+                                   self.radius_scale, symmetric=self.symmetric,
+                                   self_last=self.source is self.dest)
             self._off, self._nbr = off, nb
             self.is_dirty = False
         return 0

@@ -22,6 +22,22 @@
 
 namespace sph {
 
+// Lanes per destination (log2).  Eight is the best split from 16k particles
+// on (FP64 momentum of 40k particles in 2D: 82 / 68 / 77 us with 4 / 8 / 16
+// lanes, FP32 periodic in 3D, 100k: 231 / 197 / 220 us, FP64 density of 300k:
+// 349 us with 8, 375 with 4); smaller sets have too few waves and take 16
+// (5k: 18.8 / 13.3 / 12.1 us).  Two sources cull every row twice, which
+// fewer groups per wave make dearer: 4 lanes once the waves suffice (dam
+// break of 60k + 15k, FP64 momentum: 146 / 171 / 213 us; density 66 / 68 / 76).
+inline int group_log2(int64_t n, int nsrc) {
+  if (n < (1 << 14)) return 4;
+  return nsrc >= 2 && n >= (1 << 15) ? 2 : 3;
+}
+
+inline int group_blocks(int64_t n, int log2) {
+  return (int)((n + (kBlock >> log2) - 1) / (kBlock >> log2));
+}
+
 constexpr int kGroupRows = 512;  // row entries per wave, shared by its groups
 
 // LDS of one wave.
@@ -68,6 +84,12 @@ struct Group {
 // for 0, +1 and -1 periods.
 __device__ __forceinline__ double image_shift(int digit, double period) {
   return digit == 0 ? 0.0 : (digit == 1 ? period : -period);
+}
+
+// Offset of a periodic image's sources: x_j + s L.
+__device__ __forceinline__ double image_offset(int code, int axis, double period) {
+  const int d = axis == 0 ? code % 3 : (axis == 1 ? (code / 3) % 3 : code / 9);
+  return image_shift(d, period);
 }
 
 // Walk every candidate source of the group's destination at (px, py, pz) in

@@ -28,12 +28,6 @@ struct GroupQueue {
   uint8_t image[kGroupQueue];
 };
 
-// Offset of a periodic image's sources: x_j + s L.
-__device__ __forceinline__ double image_offset(int code, int axis, double period) {
-  const int d = axis == 0 ? code % 3 : (axis == 1 ? (code / 3) % 3 : code / 9);
-  return image_shift(d, period);
-}
-
 // The destination of a lane's group: i = its particle, whether it exists and
 // is LocalReal, its position, cell and search radius.
 template <typename T>
@@ -426,22 +420,6 @@ static int32_t check_common(const sph_grid* g, const sph_params* prm, const sph_
   return SPH_OK;
 }
 
-
-// Lanes per destination (log2).  Eight is the best split from 16k particles
-// on (FP64 momentum of 40k particles in 2D: 82 / 68 / 77 us with 4 / 8 / 16
-// lanes, FP32 periodic in 3D, 100k: 231 / 197 / 220 us, FP64 density of 300k:
-// 349 us with 8, 375 with 4); smaller sets have too few waves and take 16
-// (5k: 18.8 / 13.3 / 12.1 us).  Two sources cull every row twice, which
-// fewer groups per wave make dearer: 4 lanes once the waves suffice (dam
-// break of 60k + 15k, FP64 momentum: 146 / 171 / 213 us; density 66 / 68 / 76).
-static int group_log2(int64_t n, int nsrc) {
-  if (n < (1 << 14)) return 4;
-  return nsrc >= 2 && n >= (1 << 15) ? 2 : 3;
-}
-
-static int group_blocks(int64_t n, int log2) {
-  return (int)((n + (kBlock >> log2) - 1) / (kBlock >> log2));
-}
 
 template <typename T, typename CT, bool TAIT, bool QUEUED>
 static void launch_density_q(hipStream_t st, const Grid& G, const PassArgs<T>& a) {
