@@ -34,7 +34,7 @@
 #pragma once
 #include <math.h>
 
-#include "sph_cull.h"
+#include "sph_group.h"
 #include "sph_passes.h"
 
 namespace sph {
@@ -113,12 +113,22 @@ __device__ __forceinline__ bool accept_exact(const float4& s, const float4& d, f
   return Within32::test(s.x, s.y, s.z, d.x, d.y, d.z, d2f, r2f, r2d);
 }
 
+// The pair arithmetic below spells out its fused multiply-adds and forbids
+// the compiler others, so that a pair gives the same bits in every kernel it
+// is inlined into (the scan of one lane per destination, the groups of lanes
+// that share one, the batched scenes).
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) {
+  return __builtin_fma(a, b, c);
+}
+
 template <typename CT>
 __device__ __forceinline__ CT pair_d2(const float4& d, const float4& s, CT& rx, CT& ry, CT& rz) {
+#pragma clang fp contract(off)
   rx = (CT)d.x - (CT)s.x;
   ry = (CT)d.y - (CT)s.y;
   rz = (CT)d.z - (CT)s.z;
-  return rx * rx + ry * ry + rz * rz;
+  return fma_(rz, rz, fma_(ry, ry, rx * rx));
 }
 
 // Reciprocal and square root: hardware 1-ulp instructions for FP32 pair
@@ -143,18 +153,20 @@ __device__ __forceinline__ float fsqrt<float>(float x) {
 // Branch-free cubic spline shape W(q) (kernels.pyx:367-374).
 template <typename CT>
 __device__ __forceinline__ CT w_sel(CT q) {
+#pragma clang fp contract(off)
   const CT t = CT(2) - q;
   const CT outer = CT(0.25) * t * t * t;
-  const CT inner = CT(1) - CT(1.5) * (q * q) * (CT(1) - CT(0.5) * q);
+  const CT inner = fma_(CT(-1.5) * (q * q), fma_(CT(-0.5), q, CT(1)), CT(1));
   return q > CT(2) ? CT(0) : (q > CT(1) ? outer : inner);
 }
 
 // Branch-free gradient factor (kernels.pyx:403-412): grad W = r_ab * g.
 template <typename CT>
 __device__ __forceinline__ CT g_sel(CT q, CT r, CT h, CT inv) {
+#pragma clang fp contract(off)
   const CT t = CT(2) - q;
   const CT outer = CT(-0.75) * t * t * frcp<CT>(h * r);
-  const CT inner = CT(3) * (CT(0.75) * q - CT(1)) * (inv * inv);
+  const CT inner = CT(3) * fma_(CT(0.75), q, CT(-1)) * (inv * inv);
   return q > CT(2) ? CT(0) : (q >= CT(1) ? outer : (q > CT(1e-14) ? inner : CT(0)));
 }
 
@@ -252,6 +264,15 @@ __device__ __forceinline__ void screen_block(const View<float>& S, __amdgpu_buff
 // 4^(1/3): with v = 4^(1/3) max(1 - q, 0), v^3 = 4 max(1 - q, 0)^3.
 constexpr float kCbrt4 = 1.5874010519681994f;
 
+// 4 w(q) of a pair at squared distance d2, see density_direct_block.
+__device__ __forceinline__ float direct_w4(float d2, float ninv, float nkinv) {
+  const float s = __builtin_amdgcn_sqrtf(d2);
+  // t = max(2 - q, 0) makes w exactly 0 from q = 2 on
+  const float t = fmaxf(fmaf(ninv, s, 2.f), 0.f);
+  const float v = fmaxf(fmaf(nkinv, s, kCbrt4), 0.f);
+  return fmaf(-(v * v), v, t * t * t);
+}
+
 // records a wave stages for density_lds_row: its 4 KB LDS region (the
 // queue area the queue-free density path does not use)
 constexpr int kStage = 256;
@@ -329,7 +350,7 @@ __device__ __forceinline__ void density_direct_block(__amdgpu_buffer_rsrc_t rs, 
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const float dx = c[u].x - pd.x, dy = c[u].y - pd.y, dz = c[u].z - pd.z;
-    d2[u] = dx * dx + dy * dy + dz * dz;
+    d2[u] = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
     const bool in = kStride * u < rem;
     const bool lo = d2[u] < r2lo;
     const bool hi = d2[u] <= r2hi;
@@ -346,14 +367,7 @@ __device__ __forceinline__ void density_direct_block(__amdgpu_buffer_rsrc_t rs, 
                              (double)pd.y, (double)pd.z, r2d);
   }
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const float s = __builtin_amdgcn_sqrtf(d2[u]);
-    // t = max(2 - q, 0) makes w exactly 0 from q = 2 on
-    const float t = fmaxf(fmaf(ninv, s, 2.f), 0.f);
-    const float v = fmaxf(fmaf(nkinv, s, kCbrt4), 0.f);
-    const float w4 = fmaf(-(v * v), v, t * t * t);
-    nr = fmaf(ok[u] ? c[u].w : 0.f, w4, nr);
-  }
+  for (int u = 0; u < U; ++u) nr = fmaf(ok[u] ? c[u].w : 0.f, direct_w4(d2[u], ninv, nkinv), nr);
 }
 
 // The candidate records of a density source of uniform h for
@@ -489,21 +503,16 @@ __device__ __forceinline__ bool list_valid(const float* disp, float skin, double
 // ---------------------------------------------------------------------------
 // density
 // ---------------------------------------------------------------------------
-// m W(r_a - r_b, (h_a + h_b) / 2); ps carries the source position.
+// W(r_a - r_b, (h_a + h_b) / 2) without fac(1); ps carries the source
+// position.
 template <typename CT>
-__device__ __forceinline__ CT w_term_hb(const float4& pd, const float4& ps, CT hd, CT hb, CT m,
-                                        int dim) {
+__device__ __forceinline__ CT w_value(const float4& pd, const float4& ps, CT hd, CT hb, int dim) {
   CT rx, ry, rz;
   const CT d2 = pair_d2<CT>(pd, ps, rx, ry, rz);
   const CT hab = CT(0.5) * (hd + hb);
   const CT inv = frcp<CT>(hab);
   const CT qq = fsqrt<CT>(d2) * inv;
-  return m * (w_sel<CT>(qq) * h_dim_inv<CT>(inv, dim));
-}
-
-template <typename CT>
-__device__ __forceinline__ CT w_term(const float4& pd, const float4& ps, CT hd, CT m, int dim) {
-  return w_term_hb<CT>(pd, ps, hd, (CT)ps.w, m, dim);
+  return w_sel<CT>(qq) * h_dim_inv<CT>(inv, dim);
 }
 
 template <bool TAIT>
@@ -540,6 +549,7 @@ __device__ __forceinline__ void density_epilogue(const PassArgs<float>& a, int i
 template <typename CT, bool TAIT, bool BUILD, int DIM = 0, bool LDS = false>
 __device__ __forceinline__ void density_scan_body(const Grid& g, const PassArgs<float>& a,
                                                   int i, int* q) {
+#pragma clang fp contract(off)
   const bool valid = i < a.dst.n;
   const bool local = valid && (a.dst.tag == nullptr || a.dst.tag[i] == 0);
   const float4 pd = valid ? a.dst.pos4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -681,7 +691,7 @@ __device__ __forceinline__ void density_scan_body(const Grid& g, const PassArgs<
           if (k < cnt) {
             const int j = q[k * 64];
             const float4 pm = ld4(S.pm4, j);
-            nr += w_term_hb<CT>(pd, pm, hd, h_src, (CT)pm.w, dim);
+            nr = fma_((CT)pm.w, w_value<CT>(pd, pm, hd, h_src, dim), nr);
             if (write_list && lpos + k < a.nl_max) a.nl_idx[(int64_t)(lpos + k) * ndst + i] = j;
           }
         }
@@ -691,7 +701,7 @@ __device__ __forceinline__ void density_scan_body(const Grid& g, const PassArgs<
             const int j = q[k * 64];
             const float4 ps = ld4(S.pos4, j);
             if (exact_list || accept_exact(ps, pd, r2f, r2d))
-              nr += w_term<CT>(pd, ps, hd, (CT)ld4(S.vel4, j).w, dim);
+              nr = fma_((CT)ld4(S.vel4, j).w, w_value<CT>(pd, ps, hd, (CT)ps.w, dim), nr);
             if (write_list && lpos + k < a.nl_max) a.nl_idx[(int64_t)(lpos + k) * ndst + i] = j;
           }
         }
@@ -734,15 +744,38 @@ struct MomDst {
   int dim;
 };
 
+// What a pair adds to the sums of its destination: gf * (rx, ry, rz) to the
+// momentum sum, temp * -(vx, vy, vz) to the XSPH sum (v_b - v_a = -(v_a - v_b)
+// exactly).
+template <typename CT>
+struct PairTerms {
+  CT gf, rx, ry, rz, temp, vx, vy, vz;
+};
+
+template <typename CT, bool DM, bool DX>
+__device__ __forceinline__ void mom_add(const PairTerms<CT>& t, CT* am, CT* ax) {
+  if (DM) {
+    am[0] = fma_(t.gf, t.rx, am[0]);
+    am[1] = fma_(t.gf, t.ry, am[1]);
+    am[2] = fma_(t.gf, t.rz, am[2]);
+  }
+  if (DX) {
+    ax[0] = fma_(t.temp, -t.vx, ax[0]);
+    ax[1] = fma_(t.temp, -t.vy, ax[1]);
+    ax[2] = fma_(t.temp, -t.vz, ax[2]);
+  }
+}
+
 // One pair of the momentum (DM) and XSPH (DX) sums.  The roles are fixed
 // at compile time, so no branch separates a pair's gathers: the compiler
 // would otherwise sink the loads that only one role uses behind that
 // role's branch, and wait for memory twice per pair.
 template <typename CT, bool DM, bool DX>
-__device__ __forceinline__ void mom_pair_r(const MomDst<CT>& D, const float4& ps,
-                                           const float4& vs, const float4& as, CT* am, CT* ax) {
-  CT rx, ry, rz;
-  const CT d2 = pair_d2<CT>(D.pd, ps, rx, ry, rz);
+__device__ __forceinline__ PairTerms<CT> mom_terms_r(const MomDst<CT>& D, const float4& ps,
+                                                     const float4& vs, const float4& as) {
+#pragma clang fp contract(off)
+  PairTerms<CT> T{};
+  const CT d2 = pair_d2<CT>(D.pd, ps, T.rx, T.ry, T.rz);
   const CT hab = CT(0.5) * (D.ha + (CT)ps.w);
   const CT inv = frcp<CT>(hab);
   const CT rr = fsqrt<CT>(d2);
@@ -751,28 +784,22 @@ __device__ __forceinline__ void mom_pair_r(const MomDst<CT>& D, const float4& ps
   const CT mb = (CT)vs.w;
   const CT rhob = (CT)as.x;
   const CT irhoab = frcp<CT>(CT(0.5) * (D.rhoa + rhob));
-  // the velocity difference serves both sums (v_b - v_a = -(v_a - v_b)
-  // exactly), and every source field is read before the branches, so the
-  // three gathers of a pair go out together
-  const CT vx = (CT)D.vd.x - (CT)vs.x, vy = (CT)D.vd.y - (CT)vs.y, vz = (CT)D.vd.z - (CT)vs.z;
+  // every source field is read before the branches, so the three gathers of
+  // a pair go out together
+  T.vx = (CT)D.vd.x - (CT)vs.x;
+  T.vy = (CT)D.vd.y - (CT)vs.y;
+  T.vz = (CT)D.vd.z - (CT)vs.z;
   const CT Ab = sizeof(CT) == 8 ? (CT)as.w / (rhob * rhob) : (CT)as.z;
   const CT cab = CT(0.5) * (D.ca + (CT)as.y);
   if (DM) {
-    const CT dot = vx * rx + vy * ry + vz * rz;
-    const CT mu = hab * dot * frcp<CT>(d2 + D.eta2 * hab * hab);
-    const CT piab = (-D.alpha * cab * mu + D.beta * mu * mu) * irhoab;
+    const CT dot = fma_(T.vz, T.rz, fma_(T.vy, T.ry, T.vx * T.rx));
+    const CT mu = hab * dot * frcp<CT>(fma_(D.eta2 * hab, hab, d2));
+    const CT piab = fma_(D.beta * mu, mu, -D.alpha * cab * mu) * irhoab;
     const CT tmp = D.Aa + Ab + (dot < CT(0) ? piab : CT(0));
-    const CT gf = -mb * tmp * (g_sel<CT>(qq, rr, hab, inv) * fac);
-    am[0] += gf * rx;
-    am[1] += gf * ry;
-    am[2] += gf * rz;
+    T.gf = -mb * tmp * (g_sel<CT>(qq, rr, hab, inv) * fac);
   }
-  if (DX) {
-    const CT temp = mb * (w_sel<CT>(qq) * fac) * irhoab;
-    ax[0] += temp * -vx;
-    ax[1] += temp * -vy;
-    ax[2] += temp * -vz;
-  }
+  if (DX) T.temp = mb * (w_sel<CT>(qq) * fac) * irhoab;
+  return T;
 }
 
 // Constants of the pairs of one destination with a source whose h is
@@ -793,46 +820,42 @@ __device__ __forceinline__ MomUni mom_uni(float ha, float hb, float eta2, int di
   return u;
 }
 
-// mom_pair_r<float, DM, DX> for a source of uniform h: the per-pair
+// mom_terms_r<float, DM, DX> for a source of uniform h: the per-pair
 // reciprocal of h_ab and the normalisation come from MomUni, and one
 // reciprocal square root gives both |r_ab| and the 1/|r_ab| of the outer
 // gradient branch (kernels.pyx:403-412), so a pair costs three
 // quarter-rate transcendental instructions instead of five.
 template <bool DM, bool DX>
-__device__ __forceinline__ void mom_pair_u(const MomDst<float>& D, const MomUni& U,
-                                           const float4& ps, const float4& vs,
-                                           const float4& as, float* am, float* ax) {
-  float rx, ry, rz;
-  const float d2 = pair_d2<float>(D.pd, ps, rx, ry, rz);
+__device__ __forceinline__ PairTerms<float> mom_terms_u(const MomDst<float>& D, const MomUni& U,
+                                                        const float4& ps, const float4& vs,
+                                                        const float4& as) {
+#pragma clang fp contract(off)
+  PairTerms<float> T{};
+  const float d2 = pair_d2<float>(D.pd, ps, T.rx, T.ry, T.rz);
   const float rs = __builtin_amdgcn_rsqf(d2);
   const float rr = d2 > 0.f ? d2 * rs : 0.f;  // the self pair: r = 0, not 0 * inf
   const float qq = rr * U.inv;
   const float mb = vs.w;
   const float rhob = as.x;
   const float irhoab = frcp<float>(0.5f * (D.rhoa + rhob));
-  const float vx = D.vd.x - vs.x, vy = D.vd.y - vs.y, vz = D.vd.z - vs.z;
+  T.vx = D.vd.x - vs.x;
+  T.vy = D.vd.y - vs.y;
+  T.vz = D.vd.z - vs.z;
   const float Ab = as.z;
   const float cab = 0.5f * (D.ca + as.y);
   if (DM) {
-    const float dot = vx * rx + vy * ry + vz * rz;
+    const float dot = fma_(T.vz, T.rz, fma_(T.vy, T.ry, T.vx * T.rx));
     const float mu = U.hab * dot * frcp<float>(d2 + U.eta2hh);
-    const float piab = (-D.alpha * cab * mu + D.beta * mu * mu) * irhoab;
+    const float piab = fma_(D.beta * mu, mu, -D.alpha * cab * mu) * irhoab;
     const float tmp = D.Aa + Ab + (dot < 0.f ? piab : 0.f);
     const float t = 2.f - qq;
     const float outer = U.kout * (t * t) * rs;
-    const float inner = U.kin * (0.75f * qq - 1.f);
+    const float inner = U.kin * fma_(0.75f, qq, -1.f);
     const float gfac = qq > 2.f ? 0.f : (qq >= 1.f ? outer : (qq > 1e-14f ? inner : 0.f));
-    const float gf = -mb * tmp * gfac;
-    am[0] += gf * rx;
-    am[1] += gf * ry;
-    am[2] += gf * rz;
+    T.gf = -mb * tmp * gfac;
   }
-  if (DX) {
-    const float temp = mb * (w_sel<float>(qq) * U.fac) * irhoab;
-    ax[0] += temp * -vx;
-    ax[1] += temp * -vy;
-    ax[2] += temp * -vz;
-  }
+  if (DX) T.temp = mb * (w_sel<float>(qq) * U.fac) * irhoab;
+  return T;
 }
 
 // The same pair with the roles chosen at run time (list passes).
@@ -841,11 +864,11 @@ __device__ __forceinline__ void mom_pair(const MomDst<CT>& D, const float4& ps, 
                                          const float4& as, bool do_m, bool do_x, CT* am,
                                          CT* ax) {
   if (do_m && do_x)
-    mom_pair_r<CT, true, true>(D, ps, vs, as, am, ax);
+    mom_add<CT, true, true>(mom_terms_r<CT, true, true>(D, ps, vs, as), am, ax);
   else if (do_m)
-    mom_pair_r<CT, true, false>(D, ps, vs, as, am, ax);
+    mom_add<CT, true, false>(mom_terms_r<CT, true, false>(D, ps, vs, as), am, ax);
   else if (do_x)
-    mom_pair_r<CT, false, true>(D, ps, vs, as, am, ax);
+    mom_add<CT, false, true>(mom_terms_r<CT, false, true>(D, ps, vs, as), am, ax);
 }
 
 template <typename CT, int DIM = 0>
@@ -869,9 +892,11 @@ __device__ __forceinline__ MomDst<CT> mom_dst(const PassArgs<float>& a, int i, b
 // Outputs of the plain pass (MODE 0) or the integrator update of one
 // particle in the reference's per-calc order mom, gravity, step, xsph
 // (MODE 1 RK2 predictor, 2 RK2 final, 3 Euler); see momentum_kernel.
+// Returns the bound of the particle's move (modes 1 to 3; 0 for mode 0).
 template <typename CT, int MODE>
-__device__ __forceinline__ void mom_epilogue(const PassArgs<float>& a, int i, bool local,
-                                             CT* acc, CT* dv, const float4& vd) {
+__device__ __forceinline__ float mom_epilogue(const PassArgs<float>& a, int i, bool local,
+                                              CT* acc, CT* dv, const float4& vd) {
+#pragma clang fp contract(off)
   const CT f1 = (CT)a.fac1, fe = (CT)(a.fac1 * a.eps);
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
@@ -883,7 +908,7 @@ __device__ __forceinline__ void mom_epilogue(const PassArgs<float>& a, int i, bo
       if (a.do_mom && a.acc[c] != nullptr) a.acc[c][i] = (float)acc[c];
       if (a.do_xsph && a.dv[c] != nullptr) a.dv[c][i] = (float)dv[c];
     }
-    return;
+    return 0.f;
   }
   const float dt = (float)a.dt;
   const float hdt = (float)(0.5 * a.dt);
@@ -898,31 +923,33 @@ __device__ __forceinline__ void mom_epilogue(const PassArgs<float>& a, int i, bo
     const float ks = local ? vel[c] : 0.f;
     float xn, un;
     if (MODE == 1 || MODE == 3) {
-      un = u0 + km * dt;
-      if (a.has_gravity) un = un + kg * dt;
-      xn = x0 + ks * dt;
-      if (a.do_xsph) xn = xn + kx * dt;
+      un = fma_(km, dt, u0);
+      if (a.has_gravity) un = fma_(kg, dt, un);
+      xn = fma_(ks, dt, x0);
+      if (a.do_xsph) xn = fma_(kx, dt, xn);
       if (MODE == 1) {
         a.k1[c][i] = km;
         a.k1[3 + c][i] = kx;
       }
     } else {
       const float k1m = a.k1[c][i], k1x = a.k1[3 + c][i];
-      un = u0 + hdt * (k1m + km);
-      if (a.has_gravity) un = un + hdt * (kg + kg);
-      xn = x0 + hdt * (u0 + ks);
-      if (a.do_xsph) xn = xn + hdt * (k1x + kx);
+      un = fma_(hdt, k1m + km, u0);
+      if (a.has_gravity) un = fma_(hdt, kg + kg, un);
+      xn = fma_(hdt, u0 + ks, x0);
+      if (a.do_xsph) xn = fma_(hdt, k1x + kx, xn);
     }
     a.out[c][i] = xn;
     a.out[3 + c][i] = un;
     const double mv = (double)xn - (double)x0;  // exact for two floats this close
     mv2 += mv * mv;
   }
-  if (a.disp_out != nullptr) {
-    float disp = move_bound(mv2);
-    for (int off = 32; off > 0; off >>= 1) disp = fmaxf(disp, __shfl_xor(disp, off, 64));
-    if ((threadIdx.x & 63) == 0) raise_max(a.disp_out, disp);
-  }
+  return move_bound(mv2);
+}
+
+// The largest of a wave's move bounds into *disp_out.
+__device__ __forceinline__ void wave_raise_max(float* disp_out, float disp) {
+  for (int off = 32; off > 0; off >>= 1) disp = fmaxf(disp, __shfl_xor(disp, off, 64));
+  if ((threadIdx.x & 63) == 0) raise_max(disp_out, disp);
 }
 
 // Cell scan with LDS queues (no list) for destination i; q as in
@@ -969,8 +996,10 @@ __device__ __forceinline__ void momentum_scan_body(const Grid& g, const PassArgs
           for (int k = 0; __any(k < cnt); ++k) {
             if (k < cnt) {
               const int j = q[k * 64];
-              mom_pair_u<M, X>(reinterpret_cast<const MomDst<float>&>(D), U, ld4(S.pos4, j),
-                               ld4(S.vel4, j), ld4(S.aux4, j), (float*)am, (float*)ax);
+              mom_add<float, M, X>(
+                  mom_terms_u<M, X>(reinterpret_cast<const MomDst<float>&>(D), U, ld4(S.pos4, j),
+                                    ld4(S.vel4, j), ld4(S.aux4, j)),
+                  (float*)am, (float*)ax);
             }
           }
           cnt = 0;
@@ -980,7 +1009,8 @@ __device__ __forceinline__ void momentum_scan_body(const Grid& g, const PassArgs
       for (int k = 0; __any(k < cnt); ++k) {
         if (k < cnt) {
           const int j = q[k * 64];
-          mom_pair_r<CT, M, X>(D, ld4(S.pos4, j), ld4(S.vel4, j), ld4(S.aux4, j), am, ax);
+          mom_add<CT, M, X>(
+              mom_terms_r<CT, M, X>(D, ld4(S.pos4, j), ld4(S.vel4, j), ld4(S.aux4, j)), am, ax);
         }
       }
       cnt = 0;
@@ -1016,7 +1046,228 @@ __device__ __forceinline__ void momentum_scan_body(const Grid& g, const PassArgs
     }
   }
   if (!valid) return;
-  mom_epilogue<CT, MODE>(a, i, local, acc, dv, D.vd);
+  const float disp = mom_epilogue<CT, MODE>(a, i, local, acc, dv, D.vd);
+  if (MODE != 0 && a.disp_out != nullptr) wave_raise_max(a.disp_out, disp);
+}
+
+// ---------------------------------------------------------------------------
+// groups of lanes sharing a destination (sph_group.h), packed FP32 inputs
+// ---------------------------------------------------------------------------
+// Small sets leave most SIMDs idle at one lane per destination, and each
+// lane then pays its rows' and pairs' latencies one after another (2D dam
+// break of 1.5k + 0.8k particles: density 18, stage 31 us a launch; with 16
+// lanes 12 and 12; the lines are at small_log2).  The
+// groups below give the same bits as the scans above: they visit the same
+// accepted sources in the same order, each lane works out the terms of one
+// pair (the arithmetic spells out its roundings), and the terms are added
+// one after another in that order, a sum per lane of the group.
+constexpr int kSmallQueue = 1024;  // queued sources per wave, shared by its groups
+constexpr int kTermPitch = 9;      // floats per lane: the groups of a wave use other banks
+
+struct SmallLds {
+  GroupRows rows;
+  int queue[kSmallQueue];
+  float terms[64 * kTermPitch];
+};
+
+// Ordered accepted sources of S: drain(queue, count) is called with the
+// group's queue, in pieces, by all lanes of the wave.
+template <class Drain>
+__device__ __forceinline__ void small_scan(const Grid& g, const View<float>& S, const Group& gr,
+                                           SmallLds& L, bool local, const float4& pd, int cx,
+                                           int cy, int cz, int ring, double rc, float r2lo,
+                                           float r2hi, double r2d, Drain&& drain) {
+  const int cap = kSmallQueue / (64 / gr.size);
+  int* q = L.queue + gr.index * cap;
+  int count = 0;
+  auto empty = [&]() {
+    wave_lds_fence();
+    drain(q, count);
+    count = 0;
+    wave_lds_fence();
+  };
+  group_scan<false>(g, S.cstart, gr, L.rows, local, (double)pd.x, (double)pd.y, (double)pd.z, cx,
+                    cy, cz, ring, rc, [&](bool valid, int j, int) {
+    bool ok = false;
+    if (valid) {
+      float x, y, z;
+      if (S.pos3 != nullptr) {
+        const float* c = S.pos3 + 3 * (int64_t)j;
+        x = c[0];
+        y = c[1];
+        z = c[2];
+      } else {
+        const float4 c = ld4(S.pos4, j);
+        x = c.x;
+        y = c.y;
+        z = c.z;
+      }
+      const float dx = x - pd.x, dy = y - pd.y, dz = z - pd.z;
+      const float d2f = dx * dx + dy * dy + dz * dz;
+      ok = d2f < r2lo;
+      if (!ok && d2f <= r2hi)
+        ok = exact_within((double)x, (double)y, (double)z, (double)pd.x, (double)pd.y,
+                          (double)pd.z, r2d);
+    }
+    const unsigned m = gr.mine(__ballot(ok));
+    if (ok) q[count + gr.before(m)] = j;
+    count += __popc(m);
+    if (__any(count > cap - gr.size)) empty();
+  });
+  empty();
+}
+
+// density_scan_body<float> (no list, no source cache) for the group of
+// destination i.
+template <bool TAIT, int DIM>
+__device__ __forceinline__ void density_small_body(const Grid& g, const PassArgs<float>& a,
+                                                   const Group& gr, int i, SmallLds& L) {
+#pragma clang fp contract(off)
+  const bool valid = i < a.dst.n;
+  const bool local = valid && (a.dst.tag == nullptr || a.dst.tag[i] == 0);
+  const float4 pd = valid ? a.dst.pos4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  const double r = (double)pd.w * a.rs;
+  const double r2d = r * r;
+  const float r2f = (float)r2d;
+  const float r2lo = r2f * 0.999998f, r2hi = r2f * 1.000002f;
+  int cx = 0, cy = 0, cz = 0;
+  if (local) cell_xyz(a.dst.cell[i], g, cx, cy, cz);
+  const int ring = ring_of(g, a.disp);
+  const double rc = r + (a.disp ? (double)*a.disp : 0.0);
+  const int dim = DIM ? DIM : a.dim;
+  float* terms = L.terms + gr.base * kTermPitch;
+  float rho = 0.f;
+  for (int s = 0; s < a.nsrc; ++s) {
+    const View<float> S = a.src[s];
+    const bool uni = kDensDirect && S.pm4 != nullptr && S.hrange != nullptr &&
+                     S.hrange[0] == S.hrange[1];
+    const float hb = uni ? __int_as_float(S.hrange[0]) : 1.f;
+    const float inv = frcp<float>(0.5f * (pd.w + hb));
+    const float fac = h_dim_inv<float>(inv, dim);
+    float nr = 0.f;
+    small_scan(g, S, gr, L, local, pd, cx, cy, cz, ring, rc, r2lo, r2hi, r2d,
+               [&](const int* q, int count) {
+      for (int b = 0; __any(b < count); b += gr.size) {
+        const int k = b + gr.rank;
+        float m = 0.f, w = 0.f;
+        if (k < count) {
+          const int j = q[k];
+          if (uni) {
+            const float4 c = ld4(S.pm4, j);
+            const float dx = c.x - pd.x, dy = c.y - pd.y, dz = c.z - pd.z;
+            const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+            m = c.w;
+            w = direct_w4(d2, -inv, -kCbrt4 * inv);
+          } else {
+            const float4 c = ld4(S.pos4, j);
+            m = ld4(S.vel4, j).w;
+            w = w_value<float>(pd, c, pd.w, c.w, dim);
+          }
+        }
+        terms[gr.rank * kTermPitch] = m;
+        terms[gr.rank * kTermPitch + 1] = w;
+        wave_lds_fence();
+        // lanes without a pair left zeros, which add nothing
+        if (gr.rank == 0) {
+          for (int t0 = 0; t0 < gr.size; t0 += 8)
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+              nr = fmaf(terms[(t0 + t) * kTermPitch], terms[(t0 + t) * kTermPitch + 1], nr);
+        }
+        wave_lds_fence();
+      }
+    });
+    rho += uni ? nr * (0.25f * fac) : nr;
+  }
+  if (!valid || gr.rank != 0) return;
+  density_epilogue<TAIT>(a, i, local, (double)(rho * (float)a.fac1));
+}
+
+// momentum_scan_body<float, MODE> for the group of destination i (groups of
+// at least eight lanes: one sum component per lane).
+template <int MODE, int DIM>
+__device__ __forceinline__ void momentum_small_body(const Grid& g, const PassArgs<float>& a,
+                                                    const Group& gr, int i, SmallLds& L) {
+  const bool valid = i < a.dst.n;
+  const bool local = valid && (a.dst.tag == nullptr || a.dst.tag[i] == 0);
+  const MomDst<float> D = mom_dst<float, DIM>(a, i, valid);
+  const double r = (double)D.pd.w * a.rs;
+  const double r2d = r * r;
+  const float r2f = (float)r2d;
+  const float r2lo = r2f * 0.999998f, r2hi = r2f * 1.000002f;
+  int cx = 0, cy = 0, cz = 0;
+  if (local) cell_xyz(a.dst.cell[i], g, cx, cy, cz);
+  const int ring = ring_of(g, a.disp);
+  const double rc = r + (a.disp ? (double)*a.disp : 0.0);
+  float* terms = L.terms + gr.base * kTermPitch;
+  // lane c of the group holds component c of (momentum, XSPH)
+  const int comp = gr.rank;
+  const float sign = comp < 3 ? 1.f : -1.f;
+  const int fa = comp < 3 ? 0 : 4, fb = comp < 3 ? 1 + comp : 2 + comp;
+  float total = 0.f;
+  for (int s = 0; s < a.nsrc; ++s) {
+    const View<float> S = a.src[s];
+    const bool do_m = (a.flags[s] & SPH_SRC_MOMENTUM) != 0 && a.do_mom;
+    const bool do_x = (a.flags[s] & SPH_SRC_XSPH) != 0 && a.do_xsph;
+    if (!do_m && !do_x) continue;
+    const bool uni = kMomUni && S.hrange != nullptr && S.hrange[0] == S.hrange[1];
+    const MomUni U = mom_uni(D.ha, uni ? __int_as_float(S.hrange[0]) : 1.f, D.eta2, D.dim);
+    const bool mine = comp < 6 && (comp < 3 ? do_m : do_x);
+    float sum = 0.f;
+    small_scan(g, S, gr, L, local, D.pd, cx, cy, cz, ring, rc, r2lo, r2hi, r2d,
+               [&](const int* q, int count) {
+      for (int b = 0; __any(b < count); b += gr.size) {
+        const int k = b + gr.rank;
+        PairTerms<float> T{};
+        if (k < count) {
+          const int j = q[k];
+          const float4 ps = ld4(S.pos4, j), vs = ld4(S.vel4, j), as = ld4(S.aux4, j);
+          T = uni ? mom_terms_u<true, true>(D, U, ps, vs, as)
+                  : mom_terms_r<float, true, true>(D, ps, vs, as);
+        }
+        float* tp = terms + gr.rank * kTermPitch;
+        tp[0] = T.gf;
+        tp[1] = T.rx;
+        tp[2] = T.ry;
+        tp[3] = T.rz;
+        tp[4] = T.temp;
+        tp[5] = T.vx;
+        tp[6] = T.vy;
+        tp[7] = T.vz;
+        wave_lds_fence();
+        // lanes without a pair left zeros, which add nothing
+        if (mine) {
+          for (int t0 = 0; t0 < gr.size; t0 += 8)
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+              const float* p = terms + (t0 + t) * kTermPitch;
+              sum = fmaf(p[fa], sign * p[fb], sum);
+            }
+        }
+        wave_lds_fence();
+      }
+    });
+    total += sum;
+  }
+  float acc[3], dv[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    acc[c] = __shfl(total, gr.base + c, 64);
+    dv[c] = __shfl(total, gr.base + 3 + c, 64);
+  }
+  float disp = 0.f;
+  if (valid && gr.rank == 0) disp = mom_epilogue<float, MODE>(a, i, local, acc, dv, D.vd);
+  if (MODE != 0 && a.disp_out != nullptr) {
+    // one atomic per block at most
+    for (int off = 32; off > 0; off >>= 1) disp = fmaxf(disp, __shfl_xor(disp, off, 64));
+    __shared__ float bmax[kBlock / 64];
+    if ((threadIdx.x & 63) == 0) bmax[threadIdx.x >> 6] = disp;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int k = 1; k < kBlock / 64; ++k) disp = fmaxf(disp, bmax[k]);
+      raise_max(a.disp_out, disp);
+    }
+  }
 }
 
 }  // namespace sph

@@ -112,8 +112,10 @@ __global__ __launch_bounds__(kBlock) void density_list(Grid g, PassArgs<float> a
       const float4 p0 = e0 ? S.pos4[j0] : kFar4;
       const float4 p1 = e1 ? S.pos4[j1] : kFar4;
       const float m0 = e0 ? S.vel4[j0].w : 0.f, m1 = e1 ? S.vel4[j1].w : 0.f;
-      if (e0 && accept_exact(p0, pd, r2f, r2d)) nr += w_term<CT>(pd, p0, hd, (CT)m0, dim);
-      if (e1 && accept_exact(p1, pd, r2f, r2d)) nr += w_term<CT>(pd, p1, hd, (CT)m1, dim);
+      if (e0 && accept_exact(p0, pd, r2f, r2d))
+        nr = fma_((CT)m0, w_value<CT>(pd, p0, hd, (CT)p0.w, dim), nr);
+      if (e1 && accept_exact(p1, pd, r2f, r2d))
+        nr = fma_((CT)m1, w_value<CT>(pd, p1, hd, (CT)p1.w, dim), nr);
     }
     lpos += cnt_s;
     if (__any(scan)) {
@@ -123,7 +125,8 @@ __global__ __launch_bounds__(kBlock) void density_list(Grid g, PassArgs<float> a
           if (scan) row_range_cull(g, S.cstart, cx, cy + dy, cz + dz, ring, cu, j0, j1);
           for (int j = j0; j < j1; ++j) {
             const float4 ps = S.pos4[j];
-            if (accept_exact(ps, pd, r2f, r2d)) nr += w_term<CT>(pd, ps, hd, (CT)S.vel4[j].w, dim);
+            if (accept_exact(ps, pd, r2f, r2d))
+              nr = fma_((CT)S.vel4[j].w, w_value<CT>(pd, ps, hd, (CT)ps.w, dim), nr);
           }
         }
       }
@@ -222,7 +225,57 @@ __global__ __launch_bounds__(kBlock) void momentum_list(Grid g, PassArgs<float> 
     }
   }
   if (!valid) return;
-  mom_epilogue<CT, MODE>(a, i, local, acc, dv, D.vd);
+  const float disp = mom_epilogue<CT, MODE>(a, i, local, acc, dv, D.vd);
+  if (MODE != 0 && a.disp_out != nullptr) wave_raise_max(a.disp_out, disp);
+}
+
+// ---------------------------------------------------------------------------
+// small sets: groups of 2^log2 lanes per destination (the bodies' comment)
+// ---------------------------------------------------------------------------
+// Blocks [0, nb0) serve a0's destinations, the others a1's (a single
+// destination set passes nb0 = its blocks).
+template <bool TAIT, int DIM>
+__global__ __launch_bounds__(kBlock) void density_small(Grid g, PassArgs<float> a0,
+                                                        PassArgs<float> a1, int nb0, int log2) {
+  __shared__ SmallLds lds[kBlock / 64];
+  const Group gr(log2);
+  const int wid = threadIdx.x >> 6;
+  const int bid = xcd_block(blockIdx.x, gridDim.x);
+  const int per = kBlock >> log2;
+  const int in_block = wid * (64 >> log2) + gr.index;
+  if (bid < nb0)
+    density_small_body<TAIT, DIM>(g, a0, gr, bid * per + in_block, lds[wid]);
+  else
+    density_small_body<TAIT, DIM>(g, a1, gr, (bid - nb0) * per + in_block, lds[wid]);
+}
+
+template <int MODE, int DIM>
+__global__ __launch_bounds__(kBlock) void momentum_small(Grid g, PassArgs<float> a, int log2) {
+  __shared__ SmallLds lds[kBlock / 64];
+  const Group gr(log2);
+  const int wid = threadIdx.x >> 6;
+  const int bid = xcd_block(blockIdx.x, gridDim.x);
+  momentum_small_body<MODE, DIM>(g, a, gr, bid * (kBlock >> log2) + wid * (64 >> log2) + gr.index,
+                                 lds[wid]);
+}
+
+// Lanes per destination (log2) of the packed FP32 passes over n destinations,
+// 0: the scans of one lane per destination.  Groups win while those scans
+// leave SIMDs idle and lose once the waves suffice, sooner for the cheap
+// density and in 2D (fewer rows and pairs to share out).  Microseconds per
+// launch, scan / 8 lanes / 16 lanes:
+//   stage, 2D   1.5k: 31 / 14 / 12   8k: 29 / 13 / 12   30k: 31 / 24 / 31
+//               (drops, one source) 20k: 22 / 13 / 19   50k: 23 / 27 / 37
+//   stage, 3D   8k: 95 / 33 / 25     40k: 104 / 68 / 81  80k: 111 / 119 / 141
+//   density, 2D 2.3k: 18 / 13 / 12   9k: 18 / 15 / 14   20k: 14.0 / 14.3 / 19
+//   density, 3D 24k: 56 / 35 / 48    80k: 62 / 115 / 138
+static int small_log2(int64_t n, int dim, bool density) {
+  if (density) {
+    if (dim != 3) return n < 12000 ? 4 : 0;
+    return n < 8000 ? 4 : (n < 32000 ? 3 : 0);
+  }
+  if (dim != 3) return n < 12000 ? 4 : (n < 36000 ? 3 : 0);
+  return n < 16000 ? 4 : (n < 64000 ? 3 : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -299,10 +352,30 @@ static void density_scan_launch(hipStream_t st, int nb, const Grid& G, const Pas
 #undef SPH_DENS
 }
 
+template <bool TAIT>
+static void density_small_launch(hipStream_t st, const Grid& G, const PassArgs<float>& a0,
+                                 const PassArgs<float>& a1, int64_t n1, int log2) {
+  const int nb0 = group_blocks(a0.dst.n, log2), nb1 = group_blocks(n1, log2);
+  if (nb0 + nb1 == 0) return;
+  const dim3 nb(nb0 + nb1), th(kBlock);
+  switch (scan_dim<float>(a0.dim)) {
+    case 2: hipLaunchKernelGGL((density_small<TAIT, 2>), nb, th, 0, st, G, a0, a1, nb0, log2); break;
+    case 3: hipLaunchKernelGGL((density_small<TAIT, 3>), nb, th, 0, st, G, a0, a1, nb0, log2); break;
+    default: hipLaunchKernelGGL((density_small<TAIT, 0>), nb, th, 0, st, G, a0, a1, nb0, log2);
+  }
+}
+
 template <typename CT>
 static void density_launch(hipStream_t st, const Grid& G, const PassArgs<float>& a, bool tait) {
   const int nb = nblocks_for(a.dst.n);
   const bool list = a.nl_idx != nullptr;
+  const int small = sizeof(CT) == 4 && !list && !a.lds_rows && a.cache_src < 0
+                        ? small_log2(a.dst.n, a.dim, true) : 0;
+  if (small) {
+    if (tait) density_small_launch<true>(st, G, a, a, 0, small);
+    else density_small_launch<false>(st, G, a, a, 0, small);
+    return;
+  }
   const bool build = list && a.nl_mode == 0;
   if (list && !build) {
     if (tait)
@@ -359,6 +432,12 @@ static void density_pair_launch(hipStream_t st, const Grid& G, const PassArgs<fl
 int32_t fast_density_pair(hipStream_t st, const sph_grid& g, double rmax, PassArgs<float> a0,
                           PassArgs<float> a1, bool tait) {
   const Grid G = make_grid(g, rmax);
+  const int small = a0.lds_rows ? 0 : small_log2((int64_t)a0.dst.n + a1.dst.n, a0.dim, true);
+  if (small) {
+    if (tait) density_small_launch<true>(st, G, a0, a1, a1.dst.n, small);
+    else density_small_launch<false>(st, G, a0, a1, a1.dst.n, small);
+    return launch_status("sph_density_multi");
+  }
   switch (scan_dim<float>(a0.dim)) {
     case 2: density_pair_launch<2>(st, G, a0, a1, tait); break;
     case 3: density_pair_launch<3>(st, G, a0, a1, tait); break;
@@ -372,6 +451,16 @@ static void momentum_launch_mode(hipStream_t st, int nb, const Grid& G,
                                  const PassArgs<float>& a) {
   if (a.nl_idx != nullptr) {
     hipLaunchKernelGGL((momentum_list<CT, MODE>), dim3(nb), dim3(kBlock), 0, st, G, a);
+    return;
+  }
+  const int small = sizeof(CT) == 4 ? small_log2(a.dst.n, a.dim, false) : 0;
+  if (small) {
+    const dim3 nbs(group_blocks(a.dst.n, small)), th(kBlock);
+    switch (scan_dim<CT>(a.dim)) {
+      case 2: hipLaunchKernelGGL((momentum_small<MODE, 2>), nbs, th, 0, st, G, a, small); break;
+      case 3: hipLaunchKernelGGL((momentum_small<MODE, 3>), nbs, th, 0, st, G, a, small); break;
+      default: hipLaunchKernelGGL((momentum_small<MODE, 0>), nbs, th, 0, st, G, a, small);
+    }
     return;
   }
   switch (scan_dim<CT>(a.dim)) {
