@@ -8,6 +8,7 @@
 // (nnps.pyx:271-356, :525-620).
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "sph_group.h"
@@ -144,44 +145,81 @@ int32_t fill_i32(hipStream_t st, int32_t* p, int64_t n, int32_t v) {
 // ---------------------------------------------------------------------------
 // bounds
 // ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(kBlock) void bounds_partial(View<T> a, double* __restrict__ part) {
-  double mn[3] = {INFINITY, INFINITY, INFINITY}, mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < a.n;
-       i += (int64_t)gridDim.x * kBlock) {
-    double c[3] = {(double)a.x[i], (double)a.y[i], (double)a.z[i]};
+constexpr int kBoundsBlock = 1024;
+constexpr int kBoundsBlocks = 64;  // SPH_BOUNDS_WORDS = 8 + 7 * 64
+
+__device__ __forceinline__ void wave_bounds(double (&v)[7]) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      mn[d] = fmin(mn[d], c[d]);
-      mx[d] = fmax(mx[d], c[d]);
+  for (int d = 0; d < 7; ++d)
+    for (int o = 32; o > 0; o >>= 1) {
+      const double w = __shfl_xor(v[d], o, 64);
+      v[d] = d < 3 ? fmin(v[d], w) : fmax(v[d], w);
     }
-    mx[3] = fmax(mx[3], (double)a.h[i]);
-  }
-  __shared__ double red[7][kBlock];
-  for (int d = 0; d < 3; ++d) {
-    red[d][threadIdx.x] = mn[d];
-    red[3 + d][threadIdx.x] = mx[d];
-  }
-  red[6][threadIdx.x] = mx[3];
-  __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      for (int d = 0; d < 3; ++d)
-        red[d][threadIdx.x] = fmin(red[d][threadIdx.x], red[d][threadIdx.x + s]);
-      for (int d = 3; d < 7; ++d)
-        red[d][threadIdx.x] = fmax(red[d][threadIdx.x], red[d][threadIdx.x + s]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x < 7) part[blockIdx.x * 7 + threadIdx.x] = red[threadIdx.x][0];
 }
 
+// xmin, ymin, zmin, xmax, ymax, zmax, hmax of the block's particles.  Four
+// particles per thread and turn keep 16 loads in flight (4.2M particles in
+// FP32: 123 -> 28 us for the pass over x, y, z, h).
+template <typename T>
+__global__ __launch_bounds__(kBoundsBlock) void bounds_partial(View<T> a,
+                                                               double* __restrict__ part) {
+  T mn[3], mx[4];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) mn[d] = (T)INFINITY;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) mx[d] = (T)-INFINITY;
+  auto take = [&](T x, T y, T z, T h) {
+    const T c[4] = {x, y, z, h};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      mn[d] = c[d] < mn[d] ? c[d] : mn[d];  // NaN is skipped, as by fmin
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) mx[d] = c[d] > mx[d] ? c[d] : mx[d];
+  };
+  const int64_t step = (int64_t)gridDim.x * kBoundsBlock;
+  int64_t i = (int64_t)blockIdx.x * kBoundsBlock + threadIdx.x;
+  for (; i + 3 * step < a.n; i += 4 * step) {
+    T x[4], y[4], z[4], h[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      x[k] = a.x[i + k * step];
+      y[k] = a.y[i + k * step];
+      z[k] = a.z[i + k * step];
+      h[k] = a.h[i + k * step];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) take(x[k], y[k], z[k], h[k]);
+  }
+  for (; i < a.n; i += step) take(a.x[i], a.y[i], a.z[i], a.h[i]);
+  double v[7] = {(double)mn[0], (double)mn[1], (double)mn[2], (double)mx[0],
+                 (double)mx[1], (double)mx[2], (double)mx[3]};
+  wave_bounds(v);
+  __shared__ double red[kBoundsBlock / 64][7];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane == 0)
+    for (int d = 0; d < 7; ++d) red[wid][d] = v[d];
+  __syncthreads();
+  if (threadIdx.x < 7) {
+    const int d = threadIdx.x;
+    double r = red[0][d];
+    for (int w = 1; w < kBoundsBlock / 64; ++w)
+      r = d < 3 ? fmin(r, red[w][d]) : fmax(r, red[w][d]);
+    part[blockIdx.x * 7 + d] = r;
+  }
+}
+
+// One wave, a lane per block's partial (seven lanes walking the partials one
+// after another took 11 us).
 __global__ void bounds_final(const double* __restrict__ part, int nb, double* __restrict__ out) {
-  const int d = threadIdx.x;
-  if (d >= 7) return;
-  double v = d < 3 ? INFINITY : -INFINITY;
-  for (int b = 0; b < nb; ++b) v = d < 3 ? fmin(v, part[b * 7 + d]) : fmax(v, part[b * 7 + d]);
-  out[d] = v;
+  const int lane = threadIdx.x;
+  double v[7];
+#pragma unroll
+  for (int d = 0; d < 7; ++d)
+    v[d] = lane < nb ? part[lane * 7 + d] : (d < 3 ? INFINITY : -INFINITY);
+  wave_bounds(v);
+  if (lane == 0)
+    for (int d = 0; d < 7; ++d) out[d] = v[d];
 }
 
 // ---------------------------------------------------------------------------
@@ -197,6 +235,24 @@ struct BinGrid {
 // floor(a / k) for k >= 1 and any sign of a.
 __device__ __forceinline__ int floor_div(int a, int k) {
   return a >= 0 ? a / k : -((-a + k - 1) / k);
+}
+
+// Whether the reference cell (floor(bin / k)) moved by more than one from
+// previous bin pc to (cx, cy, cz).
+__device__ __forceinline__ bool bin_jumped(const BinGrid& g, int pc, int cx, int cy, int cz) {
+  int px = pc % g.dims[0], t = pc / g.dims[0];
+  int py = t % g.dims[1], pz = t / g.dims[1];
+  int qx = cx, qy = cy, qz = cz;
+  if (g.k > 1) {
+    // compare reference cells, floor(x / cell_size) = floor(bin / k)
+    px = floor_div(px + g.lo[0], g.k);
+    py = floor_div(py + g.lo[1], g.k);
+    pz = floor_div(pz + g.lo[2], g.k);
+    qx = floor_div(qx + g.lo[0], g.k);
+    qy = floor_div(qy + g.lo[1], g.k);
+    qz = floor_div(qz + g.lo[2], g.k);
+  }
+  return abs(px - qx) > 1 || abs(py - qy) > 1 || abs(pz - qz) > 1;
 }
 
 // floor(x/cs) as the reference computes it (cell.pyx:57), shifted into the
@@ -253,22 +309,8 @@ __global__ __launch_bounds__(kBlock) void bin_count(View<T> a, BinGrid g,
   }
   const WaveRun r = wave_run(c, valid);
   if (r.is_head) atomicAdd(&counts[c], r.len);
-  if (valid && prev_cell != nullptr) {
-    const int pc = prev_cell[i];
-    int px = pc % g.dims[0], t = pc / g.dims[0];
-    int py = t % g.dims[1], pz = t / g.dims[1];
-    int qx = cx, qy = cy, qz = cz;
-    if (g.k > 1) {
-      // compare reference cells, floor(x / cell_size) = floor(bin / k)
-      px = floor_div(px + g.lo[0], g.k);
-      py = floor_div(py + g.lo[1], g.k);
-      pz = floor_div(pz + g.lo[2], g.k);
-      qx = floor_div(qx + g.lo[0], g.k);
-      qy = floor_div(qy + g.lo[1], g.k);
-      qz = floor_div(qz + g.lo[2], g.k);
-    }
-    if (abs(px - qx) > 1 || abs(py - qy) > 1 || abs(pz - qz) > 1) atomicAdd(jumps, 1);
-  }
+  if (valid && prev_cell != nullptr && bin_jumped(g, prev_cell[i], cx, cy, cz))
+    atomicAdd(jumps, 1);
 }
 
 // The jump check of CellManager.update (cell.pyx:1422-1437) on the
@@ -377,6 +419,85 @@ __global__ __launch_bounds__(kBlock) void bin_rank(int n, const int* __restrict_
   cell_out[s + rank] = c;
 }
 
+// The whole binning of a small set in one block: counts and cell starts in
+// LDS, the members of a cell ranked by their slots.  The general path's eight
+// launches (two fills, count, three scans, scatter, rank) take 26 us and as
+// many gaps on 2k to 5k particles, this one 6 to 11.  Each thread keeps its (at
+// most kTinyPer) particles' cells in registers; cell c's count is at
+// c + c / 32, so that threads scanning 32 consecutive cells each use
+// different banks.
+constexpr int kTinyBlock = 1024;
+constexpr int kTinyPer = 8;
+constexpr int kTinyN = kTinyBlock * kTinyPer;   // 8192 particles
+constexpr int kTinyCells = 32768 - 1;           // 32 per thread, one for the total
+constexpr int kTinyChunk = 32;
+
+__device__ __forceinline__ int tiny_at(int c) { return c + (c >> 5); }
+
+template <typename T>
+__global__ __launch_bounds__(kTinyBlock) void bin_tiny(View<T> a, BinGrid g, int ncells,
+                                                       int* __restrict__ perm,
+                                                       int* __restrict__ cell_out,
+                                                       int* __restrict__ cstart,
+                                                       const int* __restrict__ prev_cell,
+                                                       int* __restrict__ jumps) {
+  __shared__ int count[32768 + 32768 / 32];
+  __shared__ uint16_t bucket[kTinyN];
+  __shared__ int wsum[kTinyBlock / 64];
+  const int t = threadIdx.x;
+  const int chunks = (ncells + kTinyChunk) / kTinyChunk;  // covers ncells + 1 entries
+  for (int c = t; c < chunks * kTinyChunk; c += kTinyBlock) count[tiny_at(c)] = 0;
+  __syncthreads();
+  int cell[kTinyPer], pos[kTinyPer];
+#pragma unroll
+  for (int k = 0; k < kTinyPer; ++k) {
+    const int i = t + k * kTinyBlock;
+    cell[k] = -1;
+    if (i < a.n) {
+      const int cx = grid_coord((double)a.x[i], g.cs, g.lo[0], g.dims[0]);
+      const int cy = grid_coord((double)a.y[i], g.cs, g.lo[1], g.dims[1]);
+      const int cz = grid_coord((double)a.z[i], g.cs, g.lo[2], g.dims[2]);
+      cell[k] = (cz * g.dims[1] + cy) * g.dims[0] + cx;
+      pos[k] = atomicAdd(&count[tiny_at(cell[k])], 1);
+      if (prev_cell != nullptr && bin_jumped(g, prev_cell[i], cx, cy, cz)) atomicAdd(jumps, 1);
+    }
+  }
+  __syncthreads();
+  // exclusive scan: 32 consecutive cells per thread
+  int sum = 0;
+  if (t < chunks)
+    for (int k = 0; k < kTinyChunk; ++k) sum += count[tiny_at(t * kTinyChunk + k)];
+  const int inc = wave_inclusive_scan(sum);
+  if ((t & 63) == 63) wsum[t >> 6] = inc;
+  __syncthreads();
+  int run = inc - sum;
+  for (int w = 0; w < (t >> 6); ++w) run += wsum[w];
+  if (t < chunks)
+    for (int k = 0; k < kTinyChunk; ++k) {
+      int* p = &count[tiny_at(t * kTinyChunk + k)];
+      const int v = *p;
+      *p = run;
+      run += v;
+    }
+  __syncthreads();
+  for (int c = t; c <= ncells; c += kTinyBlock) cstart[c] = count[tiny_at(c)];
+#pragma unroll
+  for (int k = 0; k < kTinyPer; ++k)
+    if (cell[k] >= 0)
+      bucket[count[tiny_at(cell[k])] + pos[k]] = (uint16_t)(t + k * kTinyBlock);
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kTinyPer; ++k) {
+    if (cell[k] < 0) continue;
+    const int me = t + k * kTinyBlock;
+    const int s = count[tiny_at(cell[k])], e = count[tiny_at(cell[k] + 1)];
+    int rank = 0;
+    for (int q = s; q < e; ++q) rank += bucket[q] < me ? 1 : 0;
+    perm[s + rank] = me;
+    cell_out[s + rank] = cell[k];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // permutation gather
 // ---------------------------------------------------------------------------
@@ -416,8 +537,9 @@ __global__ __launch_bounds__(kBlock) void permute_kernel(int n, const int* __res
     for (int k = 0; k < kPermPer; ++k) j[k] = p + k < n ? perm[p + k] : 0;
   }
   const bool run = full && j[1] == j[0] + 1 && j[2] == j[0] + 2 && j[3] == j[0] + 3;
+  // blockIdx.y: every gridDim.y-th field
 #pragma unroll 4
-  for (int f = 0; f < a.nf; ++f) {
+  for (int f = blockIdx.y; f < a.nf; f += gridDim.y) {
     const int esz = a.esz[f];
     const __amdgpu_buffer_rsrc_t rs = perm_rsrc(a.src[f], (int64_t)n * esz);
     if (esz == 4) {
@@ -758,18 +880,17 @@ int32_t sph_bounds(void* stream, const sph_view* a, double* out_dev) {
     return SPH_EINVAL;
   }
   hipStream_t st = as_stream(stream);
-  // partials live at the tail of the output buffer's companion: use a small
-  // fixed number of blocks and reduce them in a second single-block pass.
-  const int nb = 64;
-  static_assert(nb * 7 <= 4096, "partials");
-  double* part = nullptr;
-  // The 7-double output is followed by caller-provided room for partials.
-  part = out_dev + 8;
+  static_assert(8 + kBoundsBlocks * 7 <= SPH_BOUNDS_WORDS, "partials");
+  // the partials follow the seven results in the caller's buffer; small sets
+  // take fewer blocks
+  double* part = out_dev + 8;
+  const int64_t want = (a->n + kBoundsBlock - 1) / kBoundsBlock;
+  const int nb = (int)(want < 1 ? 1 : (want < kBoundsBlocks ? want : kBoundsBlocks));
   if (a->dtype == SPH_F32)
-    hipLaunchKernelGGL(bounds_partial<float>, dim3(nb), dim3(kBlock), 0, st, to_view<float>(*a),
-                       part);
+    hipLaunchKernelGGL(bounds_partial<float>, dim3(nb), dim3(kBoundsBlock), 0, st,
+                       to_view<float>(*a), part);
   else
-    hipLaunchKernelGGL(bounds_partial<double>, dim3(nb), dim3(kBlock), 0, st,
+    hipLaunchKernelGGL(bounds_partial<double>, dim3(nb), dim3(kBoundsBlock), 0, st,
                        to_view<double>(*a), part);
   hipLaunchKernelGGL(bounds_final, dim3(1), dim3(64), 0, st, part, nb, out_dev);
   return launch_status("sph_bounds");
@@ -823,6 +944,17 @@ int32_t sph_bin(void* stream, const sph_view* a, const sph_grid* g, int32_t* per
     bg.dims[d] = g->dims[d];
   }
   bg.k = g->bins_per_cell > 1 ? g->bins_per_cell : 1;
+  if (n > 0 && n <= kTinyN && ncells <= kTinyCells) {
+    if (a->dtype == SPH_F32)
+      hipLaunchKernelGGL(bin_tiny<float>, dim3(1), dim3(kTinyBlock), 0, st, to_view<float>(*a), bg,
+                         (int)ncells, perm_dev, cell_dev, cell_start_dev, prev_cell_dev,
+                         jump_count_dev);
+    else
+      hipLaunchKernelGGL(bin_tiny<double>, dim3(1), dim3(kTinyBlock), 0, st, to_view<double>(*a),
+                         bg, (int)ncells, perm_dev, cell_dev, cell_start_dev, prev_cell_dev,
+                         jump_count_dev);
+    return launch_status("sph_bin");
+  }
   SPH_TRY(fill_i32(st, counts, ncells, 0));
   const int nb = nblocks_for(n);
   if (n > 0) {
@@ -903,8 +1035,13 @@ int32_t sph_permute(void* stream, int64_t n, const int32_t* perm_dev, int32_t nf
       hipLaunchKernelGGL(permute_kernel_wide, dim3(nblocks_for(n)), dim3(kBlock), 0, st, (int)n,
                          perm_dev, pa);
     else
-      hipLaunchKernelGGL(permute_kernel, dim3(nblocks_for(n, kBlock * kPermPer)), dim3(kBlock), 0,
-                         st, (int)n, perm_dev, pa);
+      // a thread moves its slots of every field in turn; small sets, whose
+      // blocks do not fill the GPU, share the fields out over several blocks
+      // (22 fields of 5k particles: 12 -> 4 us)
+      hipLaunchKernelGGL(permute_kernel,
+                         dim3(nblocks_for(n, kBlock * kPermPer),
+                              n >= (1 << 18) ? 1 : std::min(pa.nf, 24)),
+                         dim3(kBlock), 0, st, (int)n, perm_dev, pa);
   }
   return launch_status("sph_permute");
 }
