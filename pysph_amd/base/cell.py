@@ -17,7 +17,7 @@ import numpy as np
 import torch
 
 from .. import _abi
-from .._device import dtype_code, require_gpu
+from .._device import dtype_code, require_gpu, stream_handle
 from .point import IntPoint
 
 
@@ -141,6 +141,9 @@ class CellManager:
         self._jump_read = None
         self._jump_seen = 0
         self._bounds_read = None
+        # buffers of those read-backs, used again once a read was taken
+        self._bounds_slot = None
+        self._jump_slot = None
         self._h_versions = None
         # set while a step is captured into a HIP graph: binning keeps the
         # current grid and starts no host read-back (the graph's owner reads
@@ -278,20 +281,32 @@ class CellManager:
             return None
         dev = arrs[0].device
         stream = require_gpu(arrs[0].get_carray("x"))
-        buf = torch.empty((len(arrs), _abi.SPH_BOUNDS_WORDS), dtype=torch.float64, device=dev)
-        for k, pa in enumerate(arrs):
-            _abi.call("sph_bounds", stream, pa.view(("x", "y", "z", "h")), buf[k].data_ptr())
-        return _AsyncRead(buf)
+        slot = self._bounds_slot
+        if slot is None or not slot.reusable(stream) or slot.dev.shape[0] != len(arrs) or \
+                slot.dev.device != dev:
+            slot = self._bounds_slot = _AsyncRead(torch.empty(
+                (len(arrs), _abi.SPH_BOUNDS_WORDS), dtype=torch.float64, device=dev), stream)
+        out = slot.dev.data_ptr()
+        for pa in arrs:
+            _abi.call("sph_bounds", stream, pa.view(("x", "y", "z", "h")), out)
+            out += 8 * _abi.SPH_BOUNDS_WORDS
+        return slot.start()
 
     @staticmethod
     def _reduce_bounds(b):
         """lo[3], hi[3] and max h over rows of sph_bounds output."""
-        lo = np.min(b[:, :3], axis=0)
-        hi = np.max(b[:, 3:6], axis=0)
-        bad = ~(np.isfinite(lo) & np.isfinite(hi))
-        lo[bad] = 0.0
-        hi[bad] = 0.0
-        return lo, hi, float(np.max(b[:, 6]))
+        rows = b[:, :7].tolist()
+        if not math.isfinite(sum(map(sum, rows))):
+            lo = np.min(b[:, :3], axis=0)
+            hi = np.max(b[:, 3:6], axis=0)
+            bad = ~(np.isfinite(lo) & np.isfinite(hi))
+            lo[bad] = 0.0
+            hi[bad] = 0.0
+            return lo, hi, float(np.max(b[:, 6]))
+        # the usual two or three rows: plain numbers are quicker than arrays
+        lo = [min(r[d] for r in rows) for d in range(3)]
+        hi = [max(r[3 + d] for r in rows) for d in range(3)]
+        return lo, hi, max(r[6] for r in rows)
 
     def make_grid(self, lo, hi):
         k = self.auto_bins(lo, hi)
@@ -452,7 +467,13 @@ class CellManager:
         """Start the asynchronous read-back of the device jump count (steps
         replayed from a graph, whose binnings start none)."""
         if self.check_jumps is True and self._jump_acc is not None and self._jump_read is None:
-            self._jump_read = _AsyncRead(self._jump_acc)
+            self._jump_read = self._read_jumps()
+
+    def _read_jumps(self):
+        slot, stream = self._jump_slot, stream_handle()
+        if slot is None or not slot.reusable(stream) or slot.dev is not self._jump_acc:
+            slot = self._jump_slot = _AsyncRead(self._jump_acc, stream)
+        return slot.start()
 
     def bin_array(self, pa, g, pos=None, extra=(), extra_out=None):
         """Counting-sort pa by cell on grid g and permute its properties.
@@ -517,7 +538,7 @@ class CellManager:
             _abi.call("sph_jump_check", stream, v, float(self.cell_size or 1.0), ref.data_ptr(),
                       self._jump_acc.data_ptr())
             if self.check_jumps is True and self._jump_read is None and not self.capturing:
-                self._jump_read = _AsyncRead(self._jump_acc)
+                self._jump_read = self._read_jumps()
         else:
             bb["ref_valid"] = False
         _abi.call("sph_bin", stream, v, g, perm.data_ptr(), cell.data_ptr(),
@@ -660,18 +681,32 @@ class CellManager:
 
 class _AsyncRead:
     """A small device tensor copied to pinned host memory on the current
-    stream behind an event; value() is the host copy once the copy has
-    completed (None before, unless wait)."""
+    stream behind an event: start() queues the copy, value() is the host copy
+    once it has completed (None before, unless wait).  After that the buffers
+    serve another read on the same stream (reusable()); a read that was
+    dropped while under way does not come back."""
 
-    def __init__(self, t):
+    def __init__(self, t, stream):
+        self.dev = t
+        self.stream = stream
         self.host = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)
-        self.host.copy_(t, non_blocking=True)
+        self.np = self.host.numpy()
         self.event = torch.cuda.Event()
+        self.free = True
+
+    def reusable(self, stream):
+        return self.free and self.stream == stream
+
+    def start(self):
+        self.free = False
+        self.host.copy_(self.dev, non_blocking=True)
         self.event.record()
+        return self
 
     def value(self, wait=False):
         if wait:
             self.event.synchronize()
         elif not self.event.query():
             return None
-        return self.host.numpy()
+        self.free = True
+        return self.np

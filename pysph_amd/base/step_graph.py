@@ -37,6 +37,17 @@ from .. import _abi
 from .._device import stream_handle
 
 
+def _grid_key(g):
+    return None if g is None else (g.cell_size, *g.lo, *g.dims)
+
+
+def _array_key(pa, props, spare, order, cell, cstart, gkey, dirty, ref):
+    return (id(pa), pa.get_number_of_particles(),
+            frozenset(zip(props, map(id, props.values()))),
+            frozenset(zip(spare, map(id, spare.values()))),
+            id(order), id(cell), id(cstart), gkey, bool(dirty), id(ref))
+
+
 class StepGraphs:
     def __init__(self, arrays, cell_manager, get_extra=None, set_extra=None, key_extra=None,
                  warmup=2, max_period=6, max_lead=8):
@@ -52,6 +63,7 @@ class StepGraphs:
         self.max_period = int(max_period)
         self.max_lead = int(max_lead)
         self._events = collections.deque()
+        self._spare_events = []
         self.enabled = True
         self.replays = 0
         self.captures = 0
@@ -91,15 +103,20 @@ class StepGraphs:
     def key(st):
         """Identity of a state: the buffers, grid and dirty flags a captured
         step reads (versions and counters excluded)."""
-        g = st["grid"]
-        key = [None if g is None else (g.cell_size, tuple(g.lo), tuple(g.dims))]
-        for pa, props, spare, order, cell, cstart, gkey, _, dirty, ref in st["arrays"]:
-            key.append((id(pa), pa.get_number_of_particles(),
-                        tuple(sorted((k, id(t)) for k, t in props.items())),
-                        tuple(sorted((k, id(t)) for k, t in spare.items())),
-                        id(order), id(cell), id(cstart), gkey, bool(dirty), id(ref)))
-        key.append(st["xkey"])
-        return tuple(key)
+        return (_grid_key(st["grid"]), st["xkey"]) + tuple(
+            _array_key(pa, props, spare, order, cell, cstart, gkey, dirty, ref)
+            for pa, props, spare, order, cell, cstart, gkey, _, dirty, ref in st["arrays"])
+
+    def live_key(self):
+        """key(state()) of the arrays as they stand, which a replayed step
+        looks up each time: no copy of the state is made for it."""
+        out = [_grid_key(self.cm.grid), self.key_extra() if self.key_extra else None]
+        for pa in self.arrays:
+            d = pa.__dict__
+            out.append(_array_key(pa, pa._props, d.get("_spare", {}), d.get("_order"),
+                                  d.get("_cell"), d.get("_cell_start"), d.get("_grid_key"),
+                                  d.get("is_dirty"), d.get("_refcell")))
+        return tuple(out)
 
     # ---------------------------------------------------------------- graphs
     def drop(self):
@@ -163,7 +180,7 @@ class StepGraphs:
             self.enabled = False
             return False
         self._g = {"tag": tag, "exec": graphs, "states": states,
-                   "keys": [self.key(s) for s in states[:-1]]}
+                   "keys": {self.key(s): i for i, s in reversed(list(enumerate(states[:-1])))}}
         self.captures += 1
         return True
 
@@ -186,19 +203,23 @@ class StepGraphs:
             if not self._capture(fn, tag):
                 fn()
                 return False
-        k = self.key(self.state())
-        keys = self._g["keys"]
-        if k not in keys:
+        i = self._g["keys"].get(self.live_key())
+        if i is None:
             self.drop()
             fn()
             return False
-        i = keys.index(k)
-        _abi.call("sph_graph_launch", self._g["exec"][i], stream_handle())
-        self.set_state(self._g["states"][i + 1])
+        self._replay(i)
+        return True
+
+    def _replay(self, i):
+        g = self._g
+        _abi.call("sph_graph_launch", g["exec"][i], stream_handle())
+        self.set_state(g["states"][i + 1])
         self.replays += 1
-        ev = torch.cuda.Event()
+        ev = self._spare_events.pop() if self._spare_events else torch.cuda.Event()
         ev.record()
         self._events.append(ev)
         while len(self._events) > self.max_lead:
-            self._events.popleft().synchronize()
-        return True
+            ev = self._events.popleft()
+            ev.synchronize()
+            self._spare_events.append(ev)
