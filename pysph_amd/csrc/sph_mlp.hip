@@ -614,17 +614,120 @@ __device__ __forceinline__ void split_bf16(float x, __bf16& hi, __bf16& lo) {
 // tiles of 32 hidden units, each as three products of the features' and
 // W_c's BF16 high and low parts (the FP32 products to ~2^-16).  In the
 // product's layout, lane l holds hidden unit 32t + (l & 31) of the 16 edge
-// rows 8(r / 4) + 4(l / 32) + (r % 4); it adds P_i + b and Q_j of each row,
-// applies the ReLU and sums its rows, and the two half-waves' row sums are
-// added at the end.  Rows past the node's last edge read that edge and are
-// masked out of the sums.  The block splits W_c into its BF16 fragments in
-// LDS once (8 KB, in the lanes' fragment order, so each read is one
-// conflict-free ds_read_b128); then each wave takes nodes w, w + nwaves, ...
+// rows 8(r / 4) + 4(l / 32) + (r % 4); it adds P_i + b, applies the ReLU and
+// sums its rows, and the two half-waves' row sums are added at the end.  The
+// block splits W_c into its BF16 fragments in LDS once (8 KB, in the lanes'
+// fragment order, so each read is one conflict-free ds_read_b128); then each
+// wave takes nodes w, w + nwaves, ...
+//
+// Bound by the return of neighbour rows from L1 (21 edges of 512 B a node in
+// 2D: TD 73 % busy) beside its vector instructions (52 %), so the matrix
+// cores take what they can: Q_j is the
+// products' initial accumulator, and rows past the node's last edge (which
+// re-read that edge) get kPastEnd through feature slot 13, one of the three
+// that edge_feat_kernel leaves zero, and so leave the ReLU as 0: no adds or
+// masks per element.  Neighbour rows are addressed by 32-bit byte offsets
+// from the uniform base.  The rows of the next tile are in flight while a
+// tile is summed, the next block's features and indices while the last two
+// tiles are.  43k nodes, 0.9M edges: 59 us with adds and masks per element
+// and nothing loaded ahead, 45 us so (three and four waves per SIMD alike,
+// five spill).
 #ifndef SPH_EDGE_WAVES
-#define SPH_EDGE_WAVES 3  // 154 VGPRs: three waves per SIMD without spills
+#define SPH_EDGE_WAVES 4
 #endif
+constexpr float kPastEnd = -8.507059173e37f;  // -2^126, a BF16 value
+constexpr int kPastSlot = 13;
+
+// The nodes of one block of a persistent edge kernel: a run of consecutive
+// (cell-ordered) nodes, whose neighbourhoods overlap, taken in turn by the
+// block's four waves; an XCD's blocks get neighbouring runs.
+struct NodeRun {
+  int lo, hi;
+};
+__device__ __forceinline__ NodeRun node_run(int n) {
+  const int nb = gridDim.x, lb = xcd_block(blockIdx.x, nb);
+  const int per = n / nb, rem = n % nb;  // block lb has per + (lb < rem) nodes
+  const int lo = lb * per + (lb < rem ? lb : rem);
+  return {lo, lo + per + (lb < rem ? 1 : 0)};
+}
+
+// v is complete here and no later load starts before: without it the sums
+// of all tiles move behind all of their loads.
+__device__ __forceinline__ void hold_order(float& v) {
+  asm volatile("" : "+v"(v)::"memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The next 32 edges of a wave: the lane's half of edge row m's features and
+// the row's neighbour.  A node without edges reads some edge of the graph,
+// which has at least one, and sums none.
+struct EdgeRows {
+  float4 x0, x1;
+  int j;
+};
+__device__ __forceinline__ EdgeRows edge_rows(const EdgeArgs& a, int64_t e0, int64_t e1, int m,
+                                              int kh) {
+  EdgeRows x;
+  const int64_t e = e0 + m < e1 ? e0 + m : (e1 > 0 ? e1 - 1 : 0);
+  x.x0 = *(const float4*)(a.E + e * kE + kh);
+  x.x1 = *(const float4*)(a.E + e * kE + kh + 4);
+  x.j = (int)a.nbr[e];
+  return x;
+}
+
+// One block of up to 32 edges: the four tiles' products and sums, with the
+// next block's features, neighbours and P row loaded on the way.  (Leaving
+// out the eights of rows past the last edge, in copies of this for 16 and 24
+// edges, gained nothing.)
+__device__ __forceinline__ EdgeRows edge_block(const EdgeArgs& a, int64_t ne0, int64_t ne1, int pi,
+                                               int m, int kh, const unsigned (&qoff)[16],
+                                               bf16x8 ah, bf16x8 al, const bf16x8* wfrag,
+                                               const float (&pb)[4], float (&sum)[4],
+                                               float (&pn)[4]) {
+  const char* const Qb = (const char*)(a.PQ + kH);
+  const int lane = threadIdx.x & 63;
+  EdgeRows x;
+  f32x16 acc[2];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[0][r] = *(const float*)(Qb + qoff[r]);
+  hold_order(sum[0]);  // not mixed with the next tile's
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    if (t < 3) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        acc[(t + 1) & 1][r] = *(const float*)(Qb + 128 * (t + 1) + qoff[r]);
+    }
+    if (t == 2) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) pn[c] = a.PQ[(int64_t)pi * 2 * kH + 32 * c + m];
+      x = edge_rows(a, ne0, ne1, m, kh);
+    }
+    // one tile's rows in flight ahead, not all of them
+    __builtin_amdgcn_sched_barrier(0);
+    const bf16x8 bh = wfrag[t * 64 + lane], bl = wfrag[256 + t * 64 + lane];
+    f32x16& z = acc[t & 1];
+    z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, z, 0, 0, 0);
+    z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, z, 0, 0, 0);
+    z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, z, 0, 0, 0);
+    float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) {
+      s0 += fmaxf(z[r] + pb[t], 0.f);
+      s1 += fmaxf(z[r + 1] + pb[t], 0.f);
+    }
+    sum[t] += s0 + s1;
+    hold_order(sum[t]);
+  }
+  return x;
+}
+
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPH_EDGE_WAVES)))
-void edge_fwd_mfma_kernel(EdgeArgs a) {
+void edge_fwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
+  const int n = a.n;
+  const float* const PQ = a.PQ;
+  __bf16* const A = a.A;
+  const int64_t lda = a.lda;
   __shared__ bf16x8 wfrag[2 * 4 * 64];  // [hi, lo][tile][lane]
   for (int f = threadIdx.x; f < 2 * 4 * 64; f += 256) {
     const int l = f & 63, t = (f >> 6) & 3, lo = f >> 8;
@@ -635,76 +738,84 @@ void edge_fwd_mfma_kernel(EdgeArgs a) {
       __bf16 h, l2;
       split_bf16(a.Wc[(k0 + s) * kH + c], h, l2);
       v[s] = lo ? l2 : h;
+      if (k0 + s >= kPastSlot)
+        v[s] = (__bf16)(k0 + s == kPastSlot && !lo ? kPastEnd : 0.f);
     }
     wfrag[f] = v;
   }
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  const int nwaves = gridDim.x * 4;
+  const NodeRun run = node_run(n);
+  int i = __builtin_amdgcn_readfirstlane(run.lo + (int)(threadIdx.x >> 6));
+  if (i >= run.hi) return;
+  if (off[n] <= 0) {  // a graph without edges
+    for (; i < run.hi; i += 4) {
+      A[(int64_t)i * lda + lane] = (__bf16)0.f;
+      A[(int64_t)i * lda + 64 + lane] = (__bf16)0.f;
+    }
+    return;
+  }
   const int m = lane & 31, kh = 8 * (lane >> 5);
   const int mr0 = 4 * (lane >> 5);  // edge row of r is mr0 + 8(r / 4) + r % 4
-  float be[4];
+  float be[4], pn[4], pb[4], sum[4] = {};
 #pragma unroll
-  for (int t = 0; t < 4; ++t) be[t] = a.be[32 * t + m];
-  for (int i = wave; i < a.n; i += nwaves) {
-    const int64_t e0 = a.off[i], e1 = a.off[i + 1];
-    float pb[4], sum[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      pb[t] = a.PQ[(int64_t)i * 2 * kH + 32 * t + m] + be[t];
-      sum[t] = 0.f;
-    }
-    for (int64_t eb = e0; eb < e1; eb += 32) {
-      const int64_t em = eb + m < e1 ? eb + m : e1 - 1;  // feature row of this lane
-      const float4 x0 = *(const float4*)(a.E + em * kE + kh);
-      const float4 x1 = *(const float4*)(a.E + em * kE + kh + 4);
-      const int jm = (int)a.nbr[em];
-      const int lim = (int)(e1 - eb);  // rows below lim are edges of node i
-      const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-      bf16x8 ah, al;
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        __bf16 h, l;
-        split_bf16(xs[s], h, l);
-        ah[s] = h;
-        al[s] = l;
-      }
-      int qoff[16];  // Q_j row of edge row r, in floats
-      float okf[16];  // 1 for the edges of node i, 0 for the rows past them
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int mr = mr0 + 8 * (r >> 2) + (r & 3);
-        const int j = __shfl(jm, mr);
-        qoff[r] = j * 2 * kH + kH + m;
-        okf[r] = mr < lim ? 1.f : 0.f;
-      }
+  for (int t = 0; t < 4; ++t) {
+    be[t] = a.be[32 * t + m];
+    pn[t] = PQ[(int64_t)i * 2 * kH + 32 * t + m];
+  }
+  int64_t e0 = off[i], e1 = off[i + 1];
+  EdgeRows x = edge_rows(a, e0, e1, m, kh);
+  bool first = true;  // first block of node i
+  // as many stores behind the loads as at the loop's end, so that its top
+  // waits for the loads alone (overwritten)
+  A[(int64_t)i * lda + lane] = (__bf16)0.f;
+  A[(int64_t)i * lda + 64 + lane] = (__bf16)0.f;
+  for (;;) {
+    // the block after this one (past the last node: this one again, unused)
+    const bool last = e0 + 32 >= e1;
+    const int ni = last ? i + 4 : i;
+    const bool more = ni < run.hi;
+    const int64_t ne0 = last ? off[more ? ni : i] : e0 + 32;
+    const int64_t ne1 = last ? off[(more ? ni : i) + 1] : e1;
+    const int lim = (int)(e1 - e0);  // rows below lim are edges of node i
+    if (first) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        float q[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) q[r] = a.PQ[(int64_t)qoff[r] + 32 * t];
-        const bf16x8 bh = wfrag[t * 64 + lane], bl = wfrag[256 + t * 64 + lane];
-        f32x16 acc = {};
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, acc, 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          // a masked row's z is finite (it re-reads a valid edge): x 0 adds 0
-          const float z = acc[r] + pb[t] + q[r];
-          sum[t] = fmaf(fmaxf(z, 0.f), okf[r], sum[t]);
-        }
-        // one tile's 16 neighbour-row loads in flight at a time: hoisting all
-        // 64 spills at the occupancy set above
-        __builtin_amdgcn_sched_barrier(0);
+        pb[t] = pn[t] + be[t];
+        sum[t] = 0.f;
       }
     }
+    unsigned qoff[16];  // byte offset of Q_j's element m, edge row r
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      qoff[r] = ((unsigned)__shfl(x.j, mr0 + 8 * (r >> 2) + (r & 3)) * 2 * kH + m) * 4;
+    const float xs[8] = {x.x0.x, x.x0.y, x.x0.z, x.x0.w, x.x1.x, x.x1.y, x.x1.z, x.x1.w};
+    bf16x8 ah, al;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      __bf16 h, l;
+      split_bf16(xs[s], h, l);
+      if (s == kPastSlot - 8 && kh) h = (__bf16)(m < lim ? 0.f : 1.f);
+      ah[s] = h;
+      al[s] = l;
+    }
+    x = edge_block(a, ne0, ne1, more ? ni : i, m, kh, qoff, ah, al, wfrag, pb, sum, pn);
+    first = last;
+    // stored after every block, whole after the node's last one: without a
+    // branch around the stores, the loads above need not wait for them
+    float tot[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const float tot = sum[t] + __shfl_xor(sum[t], 32);
-      if (lane < 32) a.A[(int64_t)i * a.lda + 32 * t + m] = (__bf16)tot;
+      tot[t] = sum[t] + __shfl_xor(sum[t], 32);
+      if (lim <= 0) tot[t] = 0.f;  // no edges
     }
+    __bf16* const Ai = A + (int64_t)i * lda + lane + (kh ? 32 : 0);
+    Ai[0] = (__bf16)(kh ? tot[2] : tot[0]);
+    Ai[32] = (__bf16)(kh ? tot[3] : tot[1]);
+    if (!more) return;
+    i = ni;
+    e0 = ne0;
+    e1 = ne1;
   }
 }
 
@@ -1388,7 +1499,7 @@ int32_t sph_mlp_forward(void* model, void* stream, const sph_mlp_graph* gr, floa
     T.begin(2);
     // the MFMA kernel indexes Q rows with 32-bit offsets (n * 2 * kH < 2^31)
     if (SPH_EDGE_MFMA && !(gr->flags & SPH_MLP_EDGE_FP32) && n < (int64_t(1) << 22))
-      hipLaunchKernelGGL(edge_fwd_mfma_kernel, dim3(edge_fwd_blocks(n)), dim3(256), 0, st, e);
+      hipLaunchKernelGGL(edge_fwd_mfma_kernel, dim3(edge_fwd_blocks(n)), dim3(256), 0, st, e, e.off);
     else
       hipLaunchKernelGGL(edge_fwd_kernel, dim3((int)((n + 3) / 4)), dim3(256), 0, st, e);
     T.end();

@@ -228,3 +228,41 @@ def test_gradients_at_chunk_remainders(width, height):
     got = M.unflatten(model.grads().astype(np.float64))
     for k in ref:
         assert _rel(got[k], ref[k]) < 3e-3, (k, g.n)
+
+
+@pytest.mark.parametrize("degrees", [
+    [0], [1], [0, 0, 0, 0, 0], [32], [0, 33, 0], [1, 0, 31, 32, 33, 0, 64, 65, 2, 96, 0],
+    [21] * 9, [65, 1] * 20, [40] * 3 + [0] + [7] * 4099])
+def test_edge_blocks_and_node_runs(degrees):
+    """The matrix-core edge aggregation on given edge counts (none, whole and
+    partial blocks of 32, several blocks; fewer nodes than waves up to several nodes
+    per wave) against the FP32 vector-unit one on the same graph.  What
+    differs is the split-BF16 products (2^-16) and BF16 copies of the
+    aggregate that round the other way (2^-8 of a value, on a share of about
+    2^-7 of them): below 1e-3, as in the test above."""
+    g, _ = _graph()
+    n = len(degrees)
+    base = g.n
+    if n > base:
+        degrees = degrees[:base]
+        n = base
+    rng = np.random.Generator(np.random.PCG64(n))
+    off = torch.tensor(np.concatenate([[0], np.cumsum(degrees)]), dtype=torch.int64,
+                       device=g.device)
+    # nearby nodes as neighbours (repeated ones are edges of their own)
+    dst = np.repeat(np.arange(n), degrees)
+    nbr = torch.tensor(np.clip(dst + rng.integers(-9, 10, len(dst)), 0, n - 1),
+                       dtype=torch.int64, device=g.device)
+    if len(dst) == 0:
+        nbr = torch.zeros(1, dtype=torch.int64, device=g.device)
+    s, keep = g.struct, (g.n, g.struct.n, g.struct.off, g.struct.nbr, g.struct.nedges)
+    model = EdgeMLP(params=_params(5))
+    try:
+        g.n = s.n = n
+        s.off, s.nbr, s.nedges = off.data_ptr(), nbr.data_ptr(), len(dst)
+        y = model.forward(g)[:n].double().cpu().numpy()
+        ref = model.forward(g, edge_fp32=True)[:n].double().cpu().numpy()
+    finally:
+        g.n, s.n, s.off, s.nbr, s.nedges = keep
+    assert np.isfinite(y).all()
+    assert _rel(y, ref) < 1e-3
