@@ -548,9 +548,8 @@ struct EdgeArgs {
   // backward
   const float* dA;      // [n x ldda] gradient of the aggregate
   int64_t ldda;
-  float* dPQ;           // [n x 2H]
-  __bf16* dPQb;         // BF16 copy
-  float* part;          // [nwaves x (kE + 1) x H] partial dWc, dbe
+  __bf16* dPQb;         // [n x 2H]: dP | dQ, rounded to BF16
+  float* part;          // [slabs x (kE + 1) x H] partial dWc, dbe
 };
 
 __global__ __launch_bounds__(256) void edge_fwd_kernel(EdgeArgs a) {
@@ -767,9 +766,10 @@ void edge_fwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
   EdgeRows x = edge_rows(a, e0, e1, m, kh);
   bool first = true;  // first block of node i
   // as many stores behind the loads as at the loop's end, so that its top
-  // waits for the loads alone (overwritten)
-  A[(int64_t)i * lda + lane] = (__bf16)0.f;
-  A[(int64_t)i * lda + 64 + lane] = (__bf16)0.f;
+  // waits for the loads alone (the same lanes overwrite them)
+  const int cl = lane + (kh ? 32 : 0);
+  A[(int64_t)i * lda + cl] = (__bf16)0.f;
+  A[(int64_t)i * lda + cl + 32] = (__bf16)0.f;
   for (;;) {
     // the block after this one (past the last node: this one again, unused)
     const bool last = e0 + 32 >= e1;
@@ -809,7 +809,7 @@ void edge_fwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
       tot[t] = sum[t] + __shfl_xor(sum[t], 32);
       if (lim <= 0) tot[t] = 0.f;  // no edges
     }
-    __bf16* const Ai = A + (int64_t)i * lda + lane + (kh ? 32 : 0);
+    __bf16* const Ai = A + (int64_t)i * lda + cl;
     Ai[0] = (__bf16)(kh ? tot[2] : tot[0]);
     Ai[32] = (__bf16)(kh ? tot[3] : tot[1]);
     if (!more) return;
@@ -877,11 +877,6 @@ __global__ __launch_bounds__(256) void edge_bwd_kernel(EdgeArgs a) {
       dq0 += t0 > 0.f ? daj0 : 0.f;
       dq1 += t1 > 0.f ? daj1 : 0.f;
     }
-    float* d = a.dPQ + (int64_t)i * 2 * kH;
-    d[lane] = dp0;
-    d[lane + 64] = dp1;
-    d[kH + lane] = dq0;
-    d[kH + lane + 64] = dq1;
     __bf16* db = a.dPQb + (int64_t)i * 2 * kH;
     db[lane] = (__bf16)dp0;
     db[lane + 64] = (__bf16)dp1;
@@ -896,6 +891,188 @@ __global__ __launch_bounds__(256) void edge_bwd_kernel(EdgeArgs a) {
   }
   p[kE * kH + lane] = gb0;
   p[kE * kH + lane + 64] = gb1;
+}
+
+// The same on the matrix cores.  A wave takes node i's edges 32 at a time, in
+// the layout of the forward aggregation (lane l: hidden unit 32t + (l & 31) of
+// 16 edge rows).  Per tile of 32 hidden units:
+//   s = Q_j + e_ij Wc and t = P_j + e_ji Wc: products whose initial
+//     accumulators are the gathered rows.  e_ji Wc is e_ij times Wc with its
+//     rows' signs and places changed as reverse_feat changes the features'.
+//     The signs of s + P_i + b and t + Q_i + b are compared without the sum.
+//   dQ_i: the lane's dA_j of the rows whose t is positive, summed.
+//   dWc: dA_i is one value for all of the node's edges, so the sum over them
+//     is dA_i * (x^T mask): a product with the 0 / 1 mask of s, which BF16
+//     holds exactly, and x as three BF16 parts (the FP32 features, exactly):
+//     rows 0-15 of the first product are the high parts, 16-31 the middle
+//     ones, rows 0-15 of the second the low ones.  The mask needs no move
+//     between lanes: the 8 rows a lane holds are a product's 8 depth slots when
+//     x^T is read in the same row order.  Feature slot 13, always zero, is
+//     one here: its row counts the masked edges (dP_i = count * dA_i, dbe).
+// Rows past the last edge are pushed below zero as in the forward pass.
+// dWc is kept in registers and summed over the block's waves at the end.
+// Bound by the return of gathered rows from L1 (1.5 KB an edge: TD 83 % busy);
+// vector arithmetic alone (110 FP32 instructions per edge and wave) took
+// 156 us for 33k nodes, this 110.  Loading a tile's rows ahead gained
+// nothing, leaving out rows past the last edge spilled.
+__device__ __forceinline__ void split3_bf16(float x, __bf16& h, __bf16& m, __bf16& l) {
+  h = (__bf16)x;
+  const float d = x - (float)h;
+  m = (__bf16)d;
+  l = (__bf16)(d - (float)m);
+}
+
+// Row of Wc that feature k multiplies in the reverse edge, and its sign.
+__device__ __forceinline__ int reverse_row(int k) { return k == 5 ? 6 : (k == 6 ? 5 : k); }
+__device__ __forceinline__ float reverse_sign(int k) {
+  return k == 0 || k == 1 || k == 3 || k == 4 || (k >= 8 && k <= 11) ? -1.f : 1.f;
+}
+
+constexpr int kBwdWaves = 2;  // per SIMD
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBwdWaves)))
+void edge_bwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
+  __shared__ bf16x8 wfrag[4 * 4 * 64];  // [s hi, s lo, t hi, t lo][tile][lane]
+  __shared__ float slab[(kE + 1) * kH];
+  for (int f = threadIdx.x; f < 4 * 4 * 64; f += 256) {
+    const int l = f & 63, t = (f >> 6) & 3, lo = (f >> 8) & 1, rev = f >> 9;
+    const int c = 32 * t + (l & 31), k0 = 8 * (l >> 5);
+    bf16x8 v;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int k = k0 + s;
+      const float w = rev ? reverse_sign(k) * a.Wc[reverse_row(k) * kH + c] : a.Wc[k * kH + c];
+      __bf16 h, l2;
+      split_bf16(w, h, l2);
+      v[s] = lo ? l2 : h;
+      if (k >= kPastSlot) v[s] = (__bf16)(k == kPastSlot && !lo ? kPastEnd : 0.f);
+    }
+    wfrag[f] = v;
+  }
+  for (int f = threadIdx.x; f < (kE + 1) * kH; f += 256) slab[f] = 0.f;
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int m = lane & 31, hf = lane >> 5, kh = 8 * hf;
+  const int mr0 = 4 * hf;  // edge row of r is mr0 + 8(r / 4) + r % 4
+  const int fk = m & 15;   // feature of this lane's row of x^T
+  const char* const Pb = (const char*)a.PQ;
+  const char* const Db = (const char*)a.dA;
+  const unsigned dpitch = (unsigned)a.ldda * 4;
+  float be[4], gt[4][8];  // gt[t][r]: feature 8(r / 4) + mr0 + r % 4, hidden unit 32t + m
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    be[t] = a.be[32 * t + m];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) gt[t][r] = 0.f;
+  }
+  const NodeRun run = node_run(a.n);
+  for (int i = __builtin_amdgcn_readfirstlane(run.lo + wv); i < run.hi; i += 4) {
+    const int64_t e0 = off[i], e1 = off[i + 1];
+    float npb[4], nqb[4], dai[4], dq[4], cnt[4];  // npb = -(P_i + b), nqb = -(Q_i + b)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float* p = a.PQ + (int64_t)i * 2 * kH + 32 * t + m;
+      npb[t] = -(p[0] + be[t]);
+      nqb[t] = -(p[kH] + be[t]);
+      dai[t] = a.dA[(int64_t)i * a.ldda + 32 * t + m];
+      dq[t] = 0.f;
+      cnt[t] = 0.f;
+    }
+    for (int64_t eb = e0; eb < e1; eb += 32) {
+      const EdgeRows x = edge_rows(a, eb, e1, m, kh);
+      const int lim = (int)(e1 - eb);  // rows below lim are edges of node i
+      float xt[16];
+      unsigned poff[16], doff[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = mr0 + 8 * (r >> 2) + (r & 3);
+        const unsigned j = (unsigned)__shfl(x.j, row);
+        poff[r] = j * (2 * kH * 4) + 4 * m;
+        doff[r] = j * dpitch + 4 * m;
+        xt[r] = a.E[(eb + (row < lim ? row : lim - 1)) * kE + fk];
+      }
+      const float xs[8] = {x.x0.x, x.x0.y, x.x0.z, x.x0.w, x.x1.x, x.x1.y, x.x1.z, x.x1.w};
+      bf16x8 ah, al, f1[2], f2[2];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        __bf16 h, l;
+        split_bf16(xs[s], h, l);
+        if (s == kPastSlot - 8 && kh) h = (__bf16)(m < lim ? 0.f : 1.f);
+        ah[s] = h;
+        al[s] = l;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        __bf16 h, md, l;
+        split3_bf16(m == kPastSlot ? 1.f : xt[r], h, md, l);
+        f1[r >> 3][r & 7] = m < 16 ? h : md;
+        f2[r >> 3][r & 7] = m < 16 ? l : (__bf16)0.f;
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        f32x16 zs, zt;
+        float d[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zt[r] = *(const float*)(Pb + 128 * t + poff[r]);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zs[r] = *(const float*)(Pb + kH * 4 + 128 * t + poff[r]);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) d[r] = *(const float*)(Db + 128 * t + doff[r]);
+        __builtin_amdgcn_sched_barrier(0);
+        const bf16x8* w = wfrag + t * 64 + lane;
+        zt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, w[512], zt, 0, 0, 0);
+        zt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, w[768], zt, 0, 0, 0);
+        zt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, w[512], zt, 0, 0, 0);
+        zs = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, w[0], zs, 0, 0, 0);
+        zs = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, w[256], zs, 0, 0, 0);
+        zs = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, w[0], zs, 0, 0, 0);
+        float q0 = 0.f, q1 = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          q0 += zt[r] > nqb[t] ? d[r] : 0.f;
+          q1 += zt[r + 1] > nqb[t] ? d[r + 1] : 0.f;
+        }
+        dq[t] += q0 + q1;
+        bf16x8 mk[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          mk[r >> 3][r & 7] = (__bf16)(zs[r] > npb[t] ? 1.f : 0.f);
+        f32x16 g = {};
+        g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f2[0], mk[0], g, 0, 0, 0);
+        g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f2[1], mk[1], g, 0, 0, 0);
+        g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f1[0], mk[0], g, 0, 0, 0);
+        g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f1[1], mk[1], g, 0, 0, 0);
+        cnt[t] += g[5];  // row 13 in the upper half-wave
+#pragma unroll
+        for (int r = 0; r < 8; ++r) gt[t][r] = fmaf(dai[t], g[r] + g[8 + r], gt[t][r]);
+        hold_order(dq[t]);
+      }
+    }
+    // the lower half-wave stores dQ, the upper one dP
+    __bf16* const o = a.dPQb + (int64_t)i * 2 * kH + (hf ? 0 : kH) + m;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float q = dq[t] + __shfl_xor(dq[t], 32);
+      o[32 * t] = (__bf16)(hf ? cnt[t] * dai[t] : q);
+    }
+  }
+  // the block's sum in wave order
+  for (int w = 0; w < 4; ++w) {
+    if (w == wv) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const int k = 8 * (r >> 2) + mr0 + (r & 3), c = 32 * t + m;
+          if (k == kPastSlot)
+            slab[kE * kH + c] += gt[t][r];
+          else
+            slab[k * kH + c] += gt[t][r];
+        }
+    }
+    __syncthreads();
+  }
+  float* p = a.part + (int64_t)blockIdx.x * (kE + 1) * kH;
+  for (int f = threadIdx.x; f < (kE + 1) * kH; f += 256) p[f] = slab[f];
 }
 
 // ---------------------------------------------------------------------------
@@ -1107,7 +1284,7 @@ struct Model {
   double t_ms[4] = {0, 0, 0, 0};
   int64_t t_calls = 0;
   std::vector<hipEvent_t> ev;
-  Buf X, E, N4, H[kR + 1], HA[kR], PQ[kR], U[kR], dH, dZb, dA, dPQ, dPQb, part, lossp;
+  Buf X, E, N4, H[kR + 1], HA[kR], PQ[kR], U[kR], dH, dZb, dA, dPQb, part, lossp;
   int64_t n_act = -1, e_act = -1;
   bool acts = false;  // the last forward pass stored what the backward pass reads
 };
@@ -1346,7 +1523,7 @@ int32_t sph_mlp_destroy(void* model) {
                   (void*)M->v})
     (void)hipFree(p);
   for (hipEvent_t e : M->ev) (void)hipEventDestroy(e);
-  for (Buf* b : {&M->X, &M->E, &M->N4, &M->dH, &M->dZb, &M->dA, &M->dPQ, &M->dPQb, &M->part,
+  for (Buf* b : {&M->X, &M->E, &M->N4, &M->dH, &M->dZb, &M->dA, &M->dPQb, &M->part,
                  &M->lossp})
     (void)hipFree(b->p);
   for (int r = 0; r <= kR; ++r) (void)hipFree(M->H[r].p);
@@ -1573,7 +1750,6 @@ int32_t sph_mlp_backward(void* model, void* stream, const sph_mlp_graph* gr,
   SPH_TRY(ensure(M->dH, (size_t)n * kH * 4));
   SPH_TRY(ensure(M->dZb, (size_t)n * kH * 2));
   SPH_TRY(ensure(M->dA, (size_t)n * kH * 4));
-  SPH_TRY(ensure(M->dPQ, (size_t)n * 2 * kH * 4));
   SPH_TRY(ensure(M->dPQb, (size_t)n * 2 * kH * 2));
   {
     // one scratch buffer serves every partial reduction of this pass: size
@@ -1625,15 +1801,21 @@ int32_t sph_mlp_backward(void* model, void* stream, const sph_mlp_graph* gr,
     e.be = M->w + L.b_e[r];
     e.dA = (const float*)M->dA.p;
     e.ldda = kH;
-    e.dPQ = (float*)M->dPQ.p;
     e.dPQb = (__bf16*)M->dPQb.p;
-    const int nbk = (int)std::min<int64_t>(1024, (n + 3) / 4);
+    // the matrix-core kernel addresses rows by 32-bit byte offsets, as in the
+    // forward pass; one slab per block, else per wave
+    const bool mfma = SPH_EDGE_MFMA && !(gr->flags & SPH_MLP_EDGE_FP32) && n < (int64_t(1) << 22);
+    const int nbk = (int)std::min<int64_t>(mfma ? 256 * kBwdWaves : 1024, (n + 3) / 4);
+    const int nslab = mfma ? nbk : nbk * 4;
     const int64_t per = (int64_t)(kE + 1) * kH;
-    SPH_TRY(ensure(M->part, (size_t)nbk * 4 * per * 4 + 1024));
+    SPH_TRY(ensure(M->part, (size_t)nslab * per * 4 + 1024));
     e.part = (float*)M->part.p;
-    hipLaunchKernelGGL(edge_bwd_kernel, dim3(nbk), dim3(256), 0, st, e);
+    if (mfma)
+      hipLaunchKernelGGL(edge_bwd_mfma_kernel, dim3(nbk), dim3(256), 0, st, e, e.off);
+    else
+      hipLaunchKernelGGL(edge_bwd_kernel, dim3(nbk), dim3(256), 0, st, e);
     // W_c and b_e are contiguous
-    slab_sum(st, (const float*)M->part.p, nbk * 4, per, (int)per, M->g + L.w_c[r], 1);
+    slab_sum(st, (const float*)M->part.p, nslab, per, (int)per, M->g + L.w_c[r], 1);
     SPH_TRY(launch_status("sph_mlp_backward/edges"));
     // dW_ab += H^T dPQ
     SPH_TRY(weight_grad(M, st, (int)n, kH, 2 * kH, (const __bf16*)M->HA[r].p, 2 * kH,

@@ -230,39 +230,70 @@ def test_gradients_at_chunk_remainders(width, height):
         assert _rel(got[k], ref[k]) < 3e-3, (k, g.n)
 
 
-@pytest.mark.parametrize("degrees", [
-    [0], [1], [0, 0, 0, 0, 0], [32], [0, 33, 0], [1, 0, 31, 32, 33, 0, 64, 65, 2, 96, 0],
-    [21] * 9, [65, 1] * 20, [40] * 3 + [0] + [7] * 4099])
+DEGREES = [[0], [1], [0, 0, 0, 0, 0], [32], [0, 33, 0], [1, 0, 31, 32, 33, 0, 64, 65, 2, 96, 0],
+           [21] * 9, [65, 1] * 20, [40] * 3 + [0] + [7] * 4099]
+
+
+def _set_edges(g, degrees):
+    """Give the graph's first nodes these edge counts, with nearby nodes as
+    neighbours (repeated ones are edges of their own)."""
+    degrees = degrees[:g.n]
+    n = len(degrees)
+    rng = np.random.Generator(np.random.PCG64(n))
+    dst = np.repeat(np.arange(n), degrees)
+    nbr = np.clip(dst + rng.integers(-9, 10, len(dst)), 0, n - 1)
+    off = torch.tensor(np.concatenate([[0], np.cumsum(degrees)]), dtype=torch.int64,
+                       device=g.device)
+    nbr = torch.tensor(nbr if len(nbr) else [0], dtype=torch.int64, device=g.device)
+    g.n = g.struct.n = n
+    g.struct.off, g.struct.nbr, g.struct.nedges = off.data_ptr(), nbr.data_ptr(), len(dst)
+    return off, nbr
+
+
+@pytest.mark.parametrize("degrees", DEGREES)
 def test_edge_blocks_and_node_runs(degrees):
     """The matrix-core edge aggregation on given edge counts (none, whole and
-    partial blocks of 32, several blocks; fewer nodes than waves up to several nodes
-    per wave) against the FP32 vector-unit one on the same graph.  What
+    partial blocks of 32, several blocks; fewer nodes than waves up to several
+    nodes per wave) against the FP32 vector-unit one on the same graph.  What
     differs is the split-BF16 products (2^-16) and BF16 copies of the
     aggregate that round the other way (2^-8 of a value, on a share of about
     2^-7 of them): below 1e-3, as in the test above."""
     g, _ = _graph()
-    n = len(degrees)
-    base = g.n
-    if n > base:
-        degrees = degrees[:base]
-        n = base
-    rng = np.random.Generator(np.random.PCG64(n))
-    off = torch.tensor(np.concatenate([[0], np.cumsum(degrees)]), dtype=torch.int64,
-                       device=g.device)
-    # nearby nodes as neighbours (repeated ones are edges of their own)
-    dst = np.repeat(np.arange(n), degrees)
-    nbr = torch.tensor(np.clip(dst + rng.integers(-9, 10, len(dst)), 0, n - 1),
-                       dtype=torch.int64, device=g.device)
-    if len(dst) == 0:
-        nbr = torch.zeros(1, dtype=torch.int64, device=g.device)
-    s, keep = g.struct, (g.n, g.struct.n, g.struct.off, g.struct.nbr, g.struct.nedges)
+    keep = _set_edges(g, degrees)
     model = EdgeMLP(params=_params(5))
-    try:
-        g.n = s.n = n
-        s.off, s.nbr, s.nedges = off.data_ptr(), nbr.data_ptr(), len(dst)
-        y = model.forward(g)[:n].double().cpu().numpy()
-        ref = model.forward(g, edge_fp32=True)[:n].double().cpu().numpy()
-    finally:
-        g.n, s.n, s.off, s.nbr, s.nedges = keep
+    y = model.forward(g)[:g.n].double().cpu().numpy()
+    ref = model.forward(g, edge_fp32=True)[:g.n].double().cpu().numpy()
     assert np.isfinite(y).all()
     assert _rel(y, ref) < 1e-3
+    del keep
+
+
+@pytest.mark.parametrize("degrees", DEGREES)
+def test_edge_backward_blocks_and_node_runs(degrees):
+    """The matrix-core edge backward pass against the FP32 vector-unit one
+    after the same forward pass.  The masks of edges whose pre-activation is
+    within 2^-16 of its terms of zero can differ (a share of about 1e-5 of
+    them, each a term of the sums of the size of the others), then the BF16
+    copies of dP and dQ round the other way; feature and mask products are
+    exact: below 1e-3."""
+    from pysph_amd import _abi
+    g, _ = _graph()
+    keep = _set_edges(g, degrees)
+    model = EdgeMLP(params=_params(6))
+    rng = np.random.Generator(np.random.PCG64(len(degrees)))
+    dout = torch.tensor(rng.normal(0, 1, (g.n, 2)), dtype=torch.float32, device=g.device)
+    stream = torch.cuda.current_stream().cuda_stream
+    model.forward(g)
+    grads = []
+    for flags in (0, _abi.SPH_MLP_EDGE_FP32):
+        model.zero_grad(stream)
+        g.struct.flags = flags
+        _abi.call("sph_mlp_backward", model.handle, stream, ctypes.byref(g.struct),
+                  dout.data_ptr())
+        grads.append(M.unflatten(model.grads().astype(np.float64)))
+    for k in grads[0]:
+        assert np.isfinite(grads[0][k]).all()
+        assert _rel(grads[0][k], grads[1][k]) < 1e-3 or np.abs(grads[1][k]).max() == 0, k
+        if np.abs(grads[1][k]).max() == 0:
+            assert np.abs(grads[0][k]).max() == 0, k
+    del keep
