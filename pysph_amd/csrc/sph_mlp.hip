@@ -19,6 +19,7 @@
 // gradient into a gather.  Weight gradients are reduced through per-block
 // partials, so every result is deterministic.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "sph_internal.h"
@@ -119,26 +120,56 @@ __device__ __forceinline__ void epi_load(const GemmArgs& g, int orow0, int col, 
   }
 }
 
+// Each output's flags are tested once, and a tile inside the matrix stores
+// without a branch per element (43k rows: K = 128, N = 256 18.2 -> 15.9 us,
+// K = 256, N = 128 20.5 -> 18.3; what is left is the rate of the stores,
+// 44 MB and 33 MB).
 template <bool SPLIT = false>
 __device__ __forceinline__ void epi_store(const GemmArgs& g, const f32x16& acc, int col,
                                           const EpiIn& in) {
   const bool second = SPLIT && col >= g.n2;  // uniform over the block
   float* C = second ? g.C2 - g.n2 : g.C;
   const int64_t ldc = second ? g.ldc2 : g.ldc;
+  float v[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
-    float v = acc[r];
-    if (g.bias) v += in.bv;
-    if (g.relu) v = fmaxf(v, 0.f);
-    const bool ok = in.rows[r] >= 0;
-    if (g.U && ok) g.U[(int64_t)in.rows[r] * g.ldu + col] = v;
-    if (g.res) v += in.rv[r];
-    if (C) {
-      if (g.accumulate && !second) v += in.cv[r];
-      if (ok) C[(int64_t)in.rows[r] * ldc + col] = v;
-    }
-    if (g.Cb && ok) g.Cb[(int64_t)in.rows[r] * g.ldcb + col] = (__bf16)v;
+    v[r] = acc[r];
+    if (g.bias) v[r] += in.bv;
   }
+  if (g.relu) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = fmaxf(v[r], 0.f);
+  }
+  bool whole = true;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) whole = whole && in.rows[r] >= 0;
+  whole = __all(whole);
+  auto put = [&](auto* out, int64_t ld) {
+    out += col;
+    if (whole) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        out[(int64_t)in.rows[r] * ld] = (std::remove_pointer_t<decltype(out)>)v[r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (in.rows[r] >= 0)
+          out[(int64_t)in.rows[r] * ld] = (std::remove_pointer_t<decltype(out)>)v[r];
+    }
+  };
+  if (g.U) put(g.U, g.ldu);
+  if (g.res) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] += in.rv[r];
+  }
+  if (C) {
+    if (g.accumulate && !second) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v[r] += in.cv[r];
+    }
+    put(C, ldc);
+  }
+  if (g.Cb) put(g.Cb, g.ldcb);
 }
 
 // C = A B^T-stored for K = 16 (the encoder): A [M x 16] row-major, B given as
