@@ -141,7 +141,8 @@ class CellManager:
         self._jump_read = None
         self._jump_seen = 0
         self._bounds_read = None
-        # buffers of those read-backs, used again once a read was taken
+        # buffers of the read-backs of replayed steps, used again once a read
+        # was taken (others return theirs: most managers bin a few times)
         self._bounds_slot = None
         self._jump_slot = None
         self._h_versions = None
@@ -273,19 +274,22 @@ class CellManager:
     def _h_state(self):
         return tuple(pa.__dict__.get("_h_version", 0) for pa in self.arrays_to_bin)
 
-    def _launch_bounds(self):
+    def _launch_bounds(self, keep=False):
         """Bounds of every array into one device buffer, copied to pinned
-        host memory on the stream behind an event (no wait)."""
+        host memory on the stream behind an event (no wait).
+        `keep`: with buffers kept for the next such call."""
         arrs = [pa for pa in self.arrays_to_bin if pa.get_number_of_particles() > 0]
         if not arrs:
             return None
         dev = arrs[0].device
         stream = require_gpu(arrs[0].get_carray("x"))
-        slot = self._bounds_slot
+        slot = self._bounds_slot if keep else None
         if slot is None or not slot.reusable(stream) or slot.dev.shape[0] != len(arrs) or \
                 slot.dev.device != dev:
-            slot = self._bounds_slot = _AsyncRead(torch.empty(
-                (len(arrs), _abi.SPH_BOUNDS_WORDS), dtype=torch.float64, device=dev), stream)
+            slot = _AsyncRead(torch.empty((len(arrs), _abi.SPH_BOUNDS_WORDS),
+                                          dtype=torch.float64, device=dev), stream)
+            if keep:
+                self._bounds_slot = slot
         out = slot.dev.data_ptr()
         for pa in arrs:
             _abi.call("sph_bounds", stream, pa.view(("x", "y", "z", "h")), out)
@@ -460,20 +464,17 @@ class CellManager:
                     self.grid, self.make_grid(lo, hi)):
                 return False
             self._bounds_read = None
-        self._bounds_read = self._launch_bounds()
+        self._bounds_read = self._launch_bounds(keep=True)
         return True
 
     def start_jump_read(self):
         """Start the asynchronous read-back of the device jump count (steps
         replayed from a graph, whose binnings start none)."""
         if self.check_jumps is True and self._jump_acc is not None and self._jump_read is None:
-            self._jump_read = self._read_jumps()
-
-    def _read_jumps(self):
-        slot, stream = self._jump_slot, stream_handle()
-        if slot is None or not slot.reusable(stream) or slot.dev is not self._jump_acc:
-            slot = self._jump_slot = _AsyncRead(self._jump_acc, stream)
-        return slot.start()
+            slot, stream = self._jump_slot, stream_handle()
+            if slot is None or not slot.reusable(stream) or slot.dev is not self._jump_acc:
+                slot = self._jump_slot = _AsyncRead(self._jump_acc, stream)
+            self._jump_read = slot.start()
 
     def bin_array(self, pa, g, pos=None, extra=(), extra_out=None):
         """Counting-sort pa by cell on grid g and permute its properties.
@@ -538,7 +539,7 @@ class CellManager:
             _abi.call("sph_jump_check", stream, v, float(self.cell_size or 1.0), ref.data_ptr(),
                       self._jump_acc.data_ptr())
             if self.check_jumps is True and self._jump_read is None and not self.capturing:
-                self._jump_read = self._read_jumps()
+                self._jump_read = _AsyncRead(self._jump_acc, stream).start()
         else:
             bb["ref_valid"] = False
         _abi.call("sph_bin", stream, v, g, perm.data_ptr(), cell.data_ptr(),

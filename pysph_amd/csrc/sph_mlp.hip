@@ -13,8 +13,8 @@
 // correction that turns it into the acceleration over a 4x time step.
 // Weights are kept in FP32 (Adam) with BF16 copies that feed the MFMA GEMMs
 // (v_mfma_f32_32x32x16_bf16, FP32 accumulation).  Edge work is a fused
-// gather / ReLU / sum per destination (one wave per node, two channels per
-// lane); the backward pass recomputes the edge pre-activations and uses the
+// gather / ReLU / sum per destination (one wave per node, its edges 32 at a
+// time on the matrix cores); the backward pass recomputes the edge pre-activations and uses the
 // graph's symmetry (j in N(i) <=> i in N(j)) to turn the scatter into Q's
 // gradient into a gather.  Weight gradients are reduced through per-block
 // partials, so every result is deterministic.
