@@ -116,7 +116,9 @@ __device__ __forceinline__ bool accept_exact(const float4& s, const float4& d, f
 // The pair arithmetic below spells out its fused multiply-adds and forbids
 // the compiler others, so that a pair gives the same bits in every kernel it
 // is inlined into (the scan of one lane per destination, the groups of lanes
-// that share one, the batched scenes).
+// that share one, the batched scenes).  Sums of products round as
+// fma(z, z, fma(x, x, y * y)): the y product alone is rounded, which is how
+// the compiler contracts x * x + y * y + z * z by itself.
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_(double a, double b, double c) {
   return __builtin_fma(a, b, c);
@@ -128,7 +130,7 @@ __device__ __forceinline__ CT pair_d2(const float4& d, const float4& s, CT& rx, 
   rx = (CT)d.x - (CT)s.x;
   ry = (CT)d.y - (CT)s.y;
   rz = (CT)d.z - (CT)s.z;
-  return fma_(rz, rz, fma_(ry, ry, rx * rx));
+  return fma_(rz, rz, fma_(rx, rx, ry * ry));
 }
 
 // Reciprocal and square root: hardware 1-ulp instructions for FP32 pair
@@ -350,7 +352,7 @@ __device__ __forceinline__ void density_direct_block(__amdgpu_buffer_rsrc_t rs, 
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const float dx = c[u].x - pd.x, dy = c[u].y - pd.y, dz = c[u].z - pd.z;
-    d2[u] = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+    d2[u] = fmaf(dz, dz, fmaf(dx, dx, dy * dy));
     const bool in = kStride * u < rem;
     const bool lo = d2[u] < r2lo;
     const bool hi = d2[u] <= r2hi;
@@ -792,7 +794,7 @@ __device__ __forceinline__ PairTerms<CT> mom_terms_r(const MomDst<CT>& D, const 
   const CT Ab = sizeof(CT) == 8 ? (CT)as.w / (rhob * rhob) : (CT)as.z;
   const CT cab = CT(0.5) * (D.ca + (CT)as.y);
   if (DM) {
-    const CT dot = fma_(T.vz, T.rz, fma_(T.vy, T.ry, T.vx * T.rx));
+    const CT dot = fma_(T.vz, T.rz, fma_(T.vx, T.rx, T.vy * T.ry));
     const CT mu = hab * dot * frcp<CT>(fma_(D.eta2 * hab, hab, d2));
     const CT piab = fma_(D.beta * mu, mu, -D.alpha * cab * mu) * irhoab;
     const CT tmp = D.Aa + Ab + (dot < CT(0) ? piab : CT(0));
@@ -844,7 +846,7 @@ __device__ __forceinline__ PairTerms<float> mom_terms_u(const MomDst<float>& D, 
   const float Ab = as.z;
   const float cab = 0.5f * (D.ca + as.y);
   if (DM) {
-    const float dot = fma_(T.vz, T.rz, fma_(T.vy, T.ry, T.vx * T.rx));
+    const float dot = fma_(T.vz, T.rz, fma_(T.vx, T.rx, T.vy * T.ry));
     const float mu = U.hab * dot * frcp<float>(d2 + U.eta2hh);
     const float piab = fma_(D.beta * mu, mu, -D.alpha * cab * mu) * irhoab;
     const float tmp = D.Aa + Ab + (dot < 0.f ? piab : 0.f);
@@ -1155,7 +1157,7 @@ __device__ __forceinline__ void density_small_body(const Grid& g, const PassArgs
           if (uni) {
             const float4 c = ld4(S.pm4, j);
             const float dx = c.x - pd.x, dy = c.y - pd.y, dz = c.z - pd.z;
-            const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+            const float d2 = fmaf(dz, dz, fmaf(dx, dx, dy * dy));
             m = c.w;
             w = direct_w4(d2, -inv, -kCbrt4 * inv);
           } else {
