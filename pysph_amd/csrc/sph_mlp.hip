@@ -644,24 +644,26 @@ __device__ __forceinline__ void split_bf16(float x, __bf16& hi, __bf16& lo) {
 // tiles of 32 hidden units, each as three products of the features' and
 // W_c's BF16 high and low parts (the FP32 products to ~2^-16).  In the
 // product's layout, lane l holds hidden unit 32t + (l & 31) of the 16 edge
-// rows 8(r / 4) + 4(l / 32) + (r % 4); it adds P_i + b, applies the ReLU and
-// sums its rows, and the two half-waves' row sums are added at the end.  The
-// block splits W_c into its BF16 fragments in LDS once (8 KB, in the lanes'
-// fragment order, so each read is one conflict-free ds_read_b128); then each
-// wave takes nodes w, w + nwaves, ...
+// rows 8(r / 4) + 4(l / 32) + (r % 4); it adds P_i + b, then Q_j, applies the
+// ReLU and sums its rows one after another, and the two half-waves' row sums
+// are added at the end.  That order is part of the result: A is stored in
+// BF16, where a last bit of a sum can become 2^-8 of a value, and a
+// surrogate run carries it through all of its steps.  The block splits W_c
+// into its BF16 fragments in LDS once (8 KB, in the lanes' fragment order, so
+// each read is one conflict-free ds_read_b128); then its waves take the nodes
+// of the block's run (node_run) in turn.
 //
 // Bound by the return of neighbour rows from L1 (21 edges of 512 B a node in
-// 2D: TD 73 % busy) beside its vector instructions (52 %), so the matrix
-// cores take what they can: Q_j is the
-// products' initial accumulator, and rows past the node's last edge (which
-// re-read that edge) get kPastEnd through feature slot 13, one of the three
-// that edge_feat_kernel leaves zero, and so leave the ReLU as 0: no adds or
-// masks per element.  Neighbour rows are addressed by 32-bit byte offsets
-// from the uniform base.  The rows of the next tile are in flight while a
-// tile is summed, the next block's features and indices while the last two
-// tiles are.  43k nodes, 0.9M edges: 59 us with adds and masks per element
-// and nothing loaded ahead, 45 us so (three and four waves per SIMD alike,
-// five spill).
+// 2D: TD 73 % busy) beside its vector instructions, so the matrix cores take
+// the masks: rows past the node's last edge (which re-read that edge) get
+// kPastEnd through feature slot 13, one of the three that edge_feat_kernel
+// leaves zero, and so leave the ReLU as 0.  Neighbour rows are addressed by
+// 32-bit byte offsets from the uniform base.  The rows of the next tile are in
+// flight while a tile is summed, the next block's features and indices while
+// the last two tiles are.  43k nodes, 0.9M edges: 59 us with a mask per
+// element and nothing loaded ahead, 45.4 so (46.7 with three waves per SIMD,
+// five spill; with Q_j as the products' initial accumulator and two
+// interleaved sums, which round differently, 44.5).
 #ifndef SPH_EDGE_WAVES
 #define SPH_EDGE_WAVES 4
 #endif
@@ -717,16 +719,16 @@ __device__ __forceinline__ EdgeRows edge_block(const EdgeArgs& a, int64_t ne0, i
   const char* const Qb = (const char*)(a.PQ + kH);
   const int lane = threadIdx.x & 63;
   EdgeRows x;
-  f32x16 acc[2];
+  float q[2][16];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[0][r] = *(const float*)(Qb + qoff[r]);
+  for (int r = 0; r < 16; ++r) q[0][r] = *(const float*)(Qb + qoff[r]);
   hold_order(sum[0]);  // not mixed with the next tile's
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     if (t < 3) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        acc[(t + 1) & 1][r] = *(const float*)(Qb + 128 * (t + 1) + qoff[r]);
+        q[(t + 1) & 1][r] = *(const float*)(Qb + 128 * (t + 1) + qoff[r]);
     }
     if (t == 2) {
 #pragma unroll
@@ -736,17 +738,12 @@ __device__ __forceinline__ EdgeRows edge_block(const EdgeArgs& a, int64_t ne0, i
     // one tile's rows in flight ahead, not all of them
     __builtin_amdgcn_sched_barrier(0);
     const bf16x8 bh = wfrag[t * 64 + lane], bl = wfrag[256 + t * 64 + lane];
-    f32x16& z = acc[t & 1];
+    f32x16 z = {};
     z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, z, 0, 0, 0);
     z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, z, 0, 0, 0);
     z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, z, 0, 0, 0);
-    float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; r += 2) {
-      s0 += fmaxf(z[r] + pb[t], 0.f);
-      s1 += fmaxf(z[r + 1] + pb[t], 0.f);
-    }
-    sum[t] += s0 + s1;
+    for (int r = 0; r < 16; ++r) sum[t] += fmaxf((z[r] + pb[t]) + q[t & 1][r], 0.f);
     hold_order(sum[t]);
   }
   return x;

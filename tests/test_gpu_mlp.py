@@ -297,3 +297,66 @@ def test_edge_backward_blocks_and_node_runs(degrees):
         if np.abs(grads[1][k]).max() == 0:
             assert np.abs(grads[0][k]).max() == 0, k
     del keep
+
+
+def _aggregate_order(x, b, q):
+    """The edge aggregation's roundings, z = (x + b) + q per edge and FP32
+    sums in the order of the matrix cores' rows: edges are taken 32 at a time,
+    half-wave h sums rows 4h + 8k .. 4h + 8k + 3 for k = 0 .. 3 one after
+    another, and the halves are added at the end."""
+    half = [np.float32(0), np.float32(0)]
+    z = np.maximum((x + np.float32(b)) + np.float32(q), np.float32(0))
+    for e, v in enumerate(z):
+        h = (e >> 2) & 1
+        half[h] = np.float32(half[h] + v)
+    return half[0] + half[1]
+
+
+def test_edge_aggregation_rounds_in_a_fixed_order():
+    """Outputs of the matrix-core aggregation bit for bit against its
+    roundings on the host: P + b is added to the edge product first, Q_j
+    second, and the rows one after another.  Every product is exact here: the
+    network passes one edge feature, a velocity difference of at most 16
+    bits, through two units of one round to the output.  Unit 0 sums 1 + 2^-8
+    (halfway between two bfloat16 values) and terms below half its last bit,
+    so that the order of the sum decides how it rounds; unit 1 has b = 2^14
+    and Q = -2^14, so that the order of the additions decides which bits of
+    the feature are kept."""
+    g, _ = _graph()
+    rng = np.random.Generator(np.random.PCG64(21))
+    n = 600
+    vals = np.zeros(n, dtype=np.float32)
+    vals[0] = 1 + 2.0 ** -8
+    vals[1:10] = 3 * 2.0 ** -26
+    vals[10:40] = rng.integers(1, 2 ** 12, 30) * 2.0 ** -12
+    lists = [rng.permutation([0] + [1 + k % 9 for k in range(d)]) for d in range(1, 70)]
+    lists += [rng.integers(10, 40, d) for d in rng.integers(0, 70, 200)]
+    lists = [np.zeros(0, np.int64)] * 40 + lists
+    lists += [rng.integers(1, 40, 3)] * (n - len(lists))
+    off = np.concatenate([[0], np.cumsum([len(v) for v in lists])])
+    nbr = np.concatenate(lists)
+    dev = [torch.from_numpy(a).to(g.device) for a in
+           (off.astype(np.int64), nbr.astype(np.int64),
+            np.stack([-vals, 0 * vals, 0 * vals, 0 * vals + 1], 1), 0 * vals + 1)]
+    s = g.struct
+    s.off, s.nbr, s.vel4, s.rho = (t.data_ptr() for t in dev)
+    g.n = s.n = n
+    s.nedges = len(nbr)
+    s.rho0 = s.u_scale = 1.0
+    s.alpha = 0.0  # with rho = rho0: no pressure or viscous terms in the output
+    B, c = 2.0 ** 14, (3, 77)
+    p = {k: 0 * v for k, v in M.unflatten(_params(0).astype(np.float64)).items()}
+    p["b_in"][5] = 1.0
+    p["w_ab0"][5, M.H + c[1]] = -B
+    p["b_e0"][c[1]] = B
+    for k in range(2):
+        p["w_c0"][3, c[k]] = 1.0
+        p["w_u0"][M.H + c[k], c[k]] = 1.0
+        p["w_out"][c[k], k] = 1.0
+    y = EdgeMLP(params=M.flatten(p).astype(np.float32)).forward(g)[:n].cpu().numpy()
+    own = vals.copy()
+    for i in range(n):
+        x = vals[lists[i]] - own[i]
+        for k, (b, q) in enumerate(((0.0, 0.0), (B, -B))):
+            want = M.bf16(_aggregate_order(x, b, q))
+            assert y[i, k] == want, (i, k, len(x), y[i, k], want)
