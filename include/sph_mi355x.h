@@ -585,11 +585,13 @@ typedef struct sph_mlp_graph {
     int32_t dim;          /* 2 or 3 */
     /* SPH_MLP_INFER: sph_mlp_forward for inference only; it does not store
      * the activations sph_mlp_backward reads, which then returns SPH_EINVAL
-     * until a forward pass without the flag.  SPH_MLP_EDGE_FP32: aggregate
-     * the edges with FP32 FMAs on the vector units instead of split-BF16
-     * products on the matrix cores (the path graphs of 2^22 nodes or more
-     * always take; the products agree to ~2^-16, the outputs to ~1e-3, as
-     * the aggregate's BF16 copy can round either way) */
+     * until a forward pass without the flag.  SPH_MLP_EDGE_FP32: the edge
+     * work of sph_mlp_forward and of sph_mlp_backward runs as FP32 FMAs on
+     * the vector units instead of split-BF16 products on the matrix cores
+     * (the path graphs of 2^22 nodes or more always take).  The forward
+     * pass's products agree to ~2^-16, the outputs to ~1e-3, as the
+     * aggregate's BF16 copy can round either way; the backward pass's are
+     * FP32 ones on both paths, its sums in another order */
     int32_t flags;
     const float *pos4;    /* (x, y, z, h) per node */
     const float *vel4;    /* (u, v, w, m) per node */

@@ -928,6 +928,9 @@ __global__ __launch_bounds__(256) void edge_bwd_kernel(EdgeArgs a) {
 //     accumulators are the gathered rows.  e_ji Wc is e_ij times Wc with its
 //     rows' signs and places changed as reverse_feat changes the features'.
 //     The signs of s + P_i + b and t + Q_i + b are compared without the sum.
+//     They decide the masks, so the products are FP32 ones: three BF16 parts
+//     hold a feature or a weight exactly, and six of their nine products
+//     leave 2^-27 of one (the forward pass's two parts: 2^-16).
 //   dQ_i: the lane's dA_j of the rows whose t is positive, summed.
 //   dWc: dA_i is one value for all of the node's edges, so the sum over them
 //     is dA_i * (x^T mask): a product with the 0 / 1 mask of s, which BF16
@@ -941,7 +944,7 @@ __global__ __launch_bounds__(256) void edge_bwd_kernel(EdgeArgs a) {
 // dWc is kept in registers and summed over the block's waves at the end.
 // Bound by the return of gathered rows from L1 (1.5 KB an edge: TD 83 % busy);
 // vector arithmetic alone (110 FP32 instructions per edge and wave) took
-// 156 us for 33k nodes, this 110.  Loading a tile's rows ahead gained
+// 156 us for 33k nodes, this 124 (112 with two parts in s and t).  Loading a tile's rows ahead gained
 // nothing, leaving out rows past the last edge spilled.
 __device__ __forceinline__ void split3_bf16(float x, __bf16& h, __bf16& m, __bf16& l) {
   h = (__bf16)x;
@@ -956,23 +959,36 @@ __device__ __forceinline__ float reverse_sign(int k) {
   return k == 0 || k == 1 || k == 3 || k == 4 || (k >= 8 && k <= 11) ? -1.f : 1.f;
 }
 
+// c + x w of the parts of x (ah, am, al) and w (wf: high, middle and low
+// fragments 256 apart), smallest products first.
+__device__ __forceinline__ f32x16 edge_product(bf16x8 ah, bf16x8 am, bf16x8 al, const bf16x8* wf,
+                                               f32x16 c) {
+  const bf16x8 wh = wf[0], wm = wf[256], wl = wf[512];
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, wh, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, wl, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, wm, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, wh, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, wm, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, wh, c, 0, 0, 0);
+}
+
 constexpr int kBwdWaves = 2;  // per SIMD
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBwdWaves)))
 void edge_bwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
-  __shared__ bf16x8 wfrag[4 * 4 * 64];  // [s hi, s lo, t hi, t lo][tile][lane]
+  __shared__ bf16x8 wfrag[6 * 4 * 64];  // [s, t][high, middle, low part][tile][lane]
   __shared__ float slab[(kE + 1) * kH];
-  for (int f = threadIdx.x; f < 4 * 4 * 64; f += 256) {
-    const int l = f & 63, t = (f >> 6) & 3, lo = (f >> 8) & 1, rev = f >> 9;
+  for (int f = threadIdx.x; f < 6 * 4 * 64; f += 256) {
+    const int l = f & 63, t = (f >> 6) & 3, part = (f >> 8) % 3, rev = (f >> 8) / 3;
     const int c = 32 * t + (l & 31), k0 = 8 * (l >> 5);
     bf16x8 v;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const int k = k0 + s;
       const float w = rev ? reverse_sign(k) * a.Wc[reverse_row(k) * kH + c] : a.Wc[k * kH + c];
-      __bf16 h, l2;
-      split_bf16(w, h, l2);
-      v[s] = lo ? l2 : h;
-      if (k >= kPastSlot) v[s] = (__bf16)(k == kPastSlot && !lo ? kPastEnd : 0.f);
+      __bf16 h, md, lo;
+      split3_bf16(w, h, md, lo);
+      v[s] = part == 0 ? h : (part == 1 ? md : lo);
+      if (k >= kPastSlot) v[s] = (__bf16)(k == kPastSlot && part == 0 ? kPastEnd : 0.f);
     }
     wfrag[f] = v;
   }
@@ -1019,13 +1035,14 @@ void edge_bwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
         xt[r] = a.E[(eb + (row < lim ? row : lim - 1)) * kE + fk];
       }
       const float xs[8] = {x.x0.x, x.x0.y, x.x0.z, x.x0.w, x.x1.x, x.x1.y, x.x1.z, x.x1.w};
-      bf16x8 ah, al, f1[2], f2[2];
+      bf16x8 ah, am, al, f1[2], f2[2];
 #pragma unroll
       for (int s = 0; s < 8; ++s) {
-        __bf16 h, l;
-        split_bf16(xs[s], h, l);
+        __bf16 h, md, l;
+        split3_bf16(xs[s], h, md, l);
         if (s == kPastSlot - 8 && kh) h = (__bf16)(m < lim ? 0.f : 1.f);
         ah[s] = h;
+        am[s] = md;
         al[s] = l;
       }
 #pragma unroll
@@ -1047,12 +1064,8 @@ void edge_bwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
         for (int r = 0; r < 16; ++r) d[r] = *(const float*)(Db + 128 * t + doff[r]);
         __builtin_amdgcn_sched_barrier(0);
         const bf16x8* w = wfrag + t * 64 + lane;
-        zt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, w[512], zt, 0, 0, 0);
-        zt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, w[768], zt, 0, 0, 0);
-        zt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, w[512], zt, 0, 0, 0);
-        zs = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, w[0], zs, 0, 0, 0);
-        zs = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, w[256], zs, 0, 0, 0);
-        zs = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, w[0], zs, 0, 0, 0);
+        zt = edge_product(ah, am, al, w + 3 * 256, zt);
+        zs = edge_product(ah, am, al, w, zs);
         float q0 = 0.f, q1 = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {

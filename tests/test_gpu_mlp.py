@@ -360,3 +360,64 @@ def test_edge_aggregation_rounds_in_a_fixed_order():
         for k, (b, q) in enumerate(((0.0, 0.0), (B, -B))):
             want = M.bf16(_aggregate_order(x, b, q))
             assert y[i, k] == want, (i, k, len(x), y[i, k], want)
+
+
+@pytest.mark.parametrize("edge_fp32", [False, True])
+def test_edge_backward_masks_in_fp32(edge_fp32):
+    """The ReLU masks of the edge backward pass where the pre-activations of
+    both directions differ from zero by a few last bits of an FP32 product:
+    features of 24 bits times 1, and weights of 24 bits times a feature of 1,
+    against biases next to them.  With a gradient of 1 at every aggregate,
+    the bias's gradient and the two halves of dW_ab count the masks, whole
+    numbers that FP32 (and BF16, up to 256 a node) holds exactly."""
+    from pysph_amd import _abi
+    g, _ = _graph()
+    rng = np.random.Generator(np.random.PCG64(31))
+    n, nd = 600, 400  # nodes; the first nd have edges, the others are their sources
+    thr = np.float32(1.2345678)
+    units = list(range(4, 4 + 48, 3))
+    w = np.ones(len(units), dtype=np.float32)
+    w[1:] = rng.uniform(1.0, 2.0, len(units) - 1)
+    b = -w * np.float32(1)
+    b[0] = -thr
+    for k in range(1, len(units)):  # a few last bits to either side of w
+        for _ in range(1 + k % 3):
+            b[k] = np.nextafter(b[k], np.float32(-9 if k & 1 else 0))
+    vals = np.zeros(n, dtype=np.float32)
+    k = rng.integers(1, 9, n - nd) * rng.choice([-1, 1], n - nd)
+    vals[nd:] = rng.choice([-1, 1], n - nd) * np.where(
+        rng.random(n - nd) < 0.3, np.float32(1), thr + (k * 2.0 ** -23).astype(np.float32))
+    deg = rng.integers(0, 80, n)
+    deg[nd:] = 0
+    off = np.concatenate([[0], np.cumsum(deg)])
+    nbr = rng.integers(nd, n, off[-1])
+    dev = [torch.from_numpy(a).to(g.device) for a in
+           (off.astype(np.int64), nbr.astype(np.int64),
+            np.stack([-vals, 0 * vals, 0 * vals, 0 * vals + 1], 1), 0 * vals + 1)]
+    s = g.struct
+    s.off, s.nbr, s.vel4, s.rho = (t.data_ptr() for t in dev)
+    g.n = s.n = n
+    s.nedges = len(nbr)
+    s.rho0 = s.u_scale = 1.0
+    s.alpha = 0.0
+    p = {key: 0 * v for key, v in M.unflatten(_params(0).astype(np.float64)).items()}
+    p["b_in"][5] = 1.0
+    for q, c in enumerate(units):
+        p["w_c1"][3, c], p["b_e1"][c] = w[q], b[q]
+        p["w_u1"][M.H + c, c] = p["c_u1"][c] = p["w_out"][c, 0] = 1.0
+    model = EdgeMLP(params=M.flatten(p).astype(np.float32))
+    model.forward(g)
+    stream = torch.cuda.current_stream().cuda_stream
+    dout = torch.zeros((n, 2), dtype=torch.float32, device=g.device)
+    dout[:, 0] = 1.0
+    s.flags = _abi.SPH_MLP_EDGE_FP32 if edge_fp32 else 0
+    model.zero_grad(stream)
+    _abi.call("sph_mlp_backward", model.handle, stream, ctypes.byref(s), dout.data_ptr())
+    got = M.unflatten(model.grads().astype(np.float64))
+    x = vals[nbr].astype(np.float64)
+    for q, c in enumerate(units):
+        fwd = x * w[q] + b[q].astype(np.float64)
+        rev = -x * w[q] + b[q].astype(np.float64)
+        assert (fwd != 0).all() and (rev != 0).all()
+        want = int((fwd > 0).sum()), int((fwd > 0).sum()), int((rev > 0).sum())
+        assert (got["b_e1"][c], got["w_ab1"][5, c], got["w_ab1"][5, M.H + c]) == want, q
