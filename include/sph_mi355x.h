@@ -580,7 +580,8 @@ int32_t sph_batch_stage(void *handle, void *stream, int32_t stage,
 #define SPH_MLP_ROUNDS 2
 typedef struct sph_mlp_graph {
     int64_t n;            /* nodes */
-    int64_t nedges;
+    int64_t nedges;       /* entries of nbr: the edges, or the room for them;
+                           * rows that offsets past it name end there */
     int64_t n_fluid;      /* nodes with btype 0 (loss normalisation) */
     int32_t dim;          /* 2 or 3 */
     /* SPH_MLP_INFER: sph_mlp_forward for inference only; it does not store

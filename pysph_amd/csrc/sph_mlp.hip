@@ -429,9 +429,16 @@ struct FeatArgs {
   const int* btype;
   const int64_t* off;
   const int64_t* nbr;
+  int64_t ne;  // entries of nbr, see edge_end
   float rho0, co, gamma, B, u_scale, g, rho_scale, alpha, eta;
   int dim;
 };
+
+// CSR offset `o` of a graph with room for `ne` edges.  A build that found
+// more (sph_neighbor_fill_capped flags it, the caller reads the flag later)
+// leaves offsets past the room: rows end there, so that no kernel reads
+// neighbours or features that were never written.
+__device__ __forceinline__ int64_t edge_end(int64_t o, int64_t ne) { return o < ne ? o : ne; }
 
 __device__ __forceinline__ float tait_p(const FeatArgs& f, float rho) {
   return f.B * (powf(rho / f.rho0, f.gamma) - 1.f);
@@ -496,7 +503,8 @@ __global__ __launch_bounds__(256) void edge_feat_kernel(FeatArgs f, float* __res
   const int lane = threadIdx.x % kFeatLanes;
   // every lane stays for the group reductions below (no early return)
   const bool node = i < f.n;
-  const int64_t e0 = node ? f.off[i] : 0, e1 = node ? f.off[i + 1] : 0;
+  const int64_t e0 = node ? edge_end(f.off[i], f.ne) : 0;
+  const int64_t e1 = node ? edge_end(f.off[i + 1], f.ne) : 0;
   const float4 pi = f.pos4[node ? i : 0], vi = f.vel4[node ? i : 0];
   const float ri = f.rho[node ? i : 0];
   const float pri = tait_p(f, ri);
@@ -570,6 +578,7 @@ struct EdgeArgs {
   int n;
   const int64_t* off;
   const int64_t* nbr;
+  int64_t ne;           // entries of nbr and rows of E, see edge_end
   const float* E;       // [edges x kE]
   const float* PQ;      // [n x 2H]: P | Q
   const float* Wc;      // [kE x H]
@@ -596,7 +605,7 @@ __global__ __launch_bounds__(256) void edge_fwd_kernel(EdgeArgs a) {
   const float p0 = a.PQ[(int64_t)i * 2 * kH + lane] + a.be[lane];
   const float p1 = a.PQ[(int64_t)i * 2 * kH + lane + 64] + a.be[lane + 64];
   float s0 = 0.f, s1 = 0.f;
-  const int64_t e0 = a.off[i], e1 = a.off[i + 1];
+  const int64_t e0 = edge_end(a.off[i], a.ne), e1 = edge_end(a.off[i + 1], a.ne);
   // four edges per iteration: their neighbour rows are in flight together
   constexpr int U = 4;
   for (int64_t e = e0; e < e1; e += U) {
@@ -775,7 +784,7 @@ void edge_fwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
   const NodeRun run = node_run(n);
   int i = __builtin_amdgcn_readfirstlane(run.lo + (int)(threadIdx.x >> 6));
   if (i >= run.hi) return;
-  if (off[n] <= 0) {  // a graph without edges
+  if (edge_end(off[n], a.ne) <= 0) {  // a graph without edges
     for (; i < run.hi; i += 4) {
       A[(int64_t)i * lda + lane] = (__bf16)0.f;
       A[(int64_t)i * lda + 64 + lane] = (__bf16)0.f;
@@ -790,7 +799,7 @@ void edge_fwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
     be[t] = a.be[32 * t + m];
     pn[t] = PQ[(int64_t)i * 2 * kH + 32 * t + m];
   }
-  int64_t e0 = off[i], e1 = off[i + 1];
+  int64_t e0 = edge_end(off[i], a.ne), e1 = edge_end(off[i + 1], a.ne);
   EdgeRows x = edge_rows(a, e0, e1, m, kh);
   bool first = true;  // first block of node i
   // as many stores behind the loads as at the loop's end, so that its top
@@ -803,8 +812,8 @@ void edge_fwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
     const bool last = e0 + 32 >= e1;
     const int ni = last ? i + 4 : i;
     const bool more = ni < run.hi;
-    const int64_t ne0 = last ? off[more ? ni : i] : e0 + 32;
-    const int64_t ne1 = last ? off[(more ? ni : i) + 1] : e1;
+    const int64_t ne0 = last ? edge_end(off[more ? ni : i], a.ne) : e0 + 32;
+    const int64_t ne1 = last ? edge_end(off[(more ? ni : i) + 1], a.ne) : e1;
     const int lim = (int)(e1 - e0);  // rows below lim are edges of node i
     if (first) {
 #pragma unroll
@@ -870,7 +879,7 @@ __global__ __launch_bounds__(256) void edge_bwd_kernel(EdgeArgs a) {
     const float dai0 = a.dA[(int64_t)i * a.ldda + lane];
     const float dai1 = a.dA[(int64_t)i * a.ldda + lane + 64];
     float dp0 = 0.f, dp1 = 0.f, dq0 = 0.f, dq1 = 0.f;
-    const int64_t e0 = a.off[i], e1 = a.off[i + 1];
+    const int64_t e0 = edge_end(a.off[i], a.ne), e1 = edge_end(a.off[i + 1], a.ne);
     for (int64_t e = e0; e < e1; ++e) {
       const int j = (int)a.nbr[e];
       const float* x = a.E + e * kE;
@@ -1012,7 +1021,7 @@ void edge_bwd_mfma_kernel(EdgeArgs a, const int64_t* __restrict__ off) {
   }
   const NodeRun run = node_run(a.n);
   for (int i = __builtin_amdgcn_readfirstlane(run.lo + wv); i < run.hi; i += 4) {
-    const int64_t e0 = off[i], e1 = off[i + 1];
+    const int64_t e0 = edge_end(off[i], a.ne), e1 = edge_end(off[i + 1], a.ne);
     float npb[4], nqb[4], dai[4], dq[4], cnt[4];  // npb = -(P_i + b), nqb = -(Q_i + b)
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -1481,6 +1490,7 @@ static FeatArgs feat_args(const sph_mlp_graph* g) {
   f.btype = g->btype;
   f.off = g->off;
   f.nbr = g->nbr;
+  f.ne = g->nedges;
   f.rho0 = (float)g->rho0;
   f.co = (float)g->co;
   f.gamma = (float)g->gamma;
@@ -1710,6 +1720,7 @@ int32_t sph_mlp_forward(void* model, void* stream, const sph_mlp_graph* gr, floa
     e.n = (int)n;
     e.off = gr->off;
     e.nbr = gr->nbr;
+    e.ne = gr->nedges;
     e.E = (const float*)M->E.p;
     e.PQ = PQ;
     e.Wc = M->w + L.w_c[r];
@@ -1838,6 +1849,7 @@ int32_t sph_mlp_backward(void* model, void* stream, const sph_mlp_graph* gr,
     e.n = (int)n;
     e.off = gr->off;
     e.nbr = gr->nbr;
+    e.ne = gr->nedges;
     e.E = (const float*)M->E.p;
     e.PQ = (const float*)M->PQ[r].p;
     e.Wc = M->w + L.w_c[r];

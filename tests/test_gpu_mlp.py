@@ -421,3 +421,36 @@ def test_edge_backward_masks_in_fp32(edge_fp32):
         assert (fwd != 0).all() and (rev != 0).all()
         want = int((fwd > 0).sum()), int((fwd > 0).sum()), int((rev > 0).sum())
         assert (got["b_e1"][c], got["w_ab1"][5, c], got["w_ab1"][5, M.H + c]) == want, q
+
+
+@pytest.mark.parametrize("edge_fp32", [False, True])
+def test_edges_past_the_capacity_are_left_out(edge_fp32):
+    """A graph with more edges than its room: the offsets of the rows that did
+    not fit point past the neighbour array, and the network's passes end
+    every row at the room's end (the same bits as with clamped offsets).  The
+    array read here has spare entries behind the room, so that a pass that
+    read on would differ, not fault."""
+    from pysph_amd import _abi
+    g, _ = _graph(max_per=8)
+    total, cap = g.nedges_exact(), g.cap
+    assert total > cap and int(g.overflow.item()) == 1
+    with pytest.raises(RuntimeError, match="more than 8 neighbours"):
+        g.check_overflow()
+    s = g.struct
+    nbr = torch.cat([g.nbr, torch.zeros(total - cap, dtype=torch.int64, device=g.device)])
+    clamped = g.off.clamp(max=cap)
+    s.nbr = nbr.data_ptr()
+    model = EdgeMLP(params=_params(5))
+    rng = np.random.Generator(np.random.PCG64(4))
+    dout = torch.tensor(rng.normal(0, 1, (g.n, 2)), dtype=torch.float32, device=g.device)
+    stream = torch.cuda.current_stream().cuda_stream
+    res = []
+    for off in (clamped, g.off):
+        s.off = off.data_ptr()
+        y = model.forward(g, edge_fp32=edge_fp32)
+        model.zero_grad(stream)
+        _abi.call("sph_mlp_backward", model.handle, stream, ctypes.byref(s), dout.data_ptr())
+        res.append((y.cpu().numpy(), model.grads()))
+    assert np.isfinite(res[0][0]).all()
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
