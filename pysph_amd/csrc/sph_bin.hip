@@ -812,7 +812,7 @@ static NbrArgs<T> nbr_args(const sph_view* dst, const sph_view* src, double radi
 
 template <bool FILL, typename T>
 static void launch_nbr(hipStream_t st, const Grid& G, const NbrArgs<T>& a) {
-  const int k = group_log2(a.dst.n, 1);
+  const int k = a.dst.n < (1 << 14) ? 4 : 3;
   const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
   if (G.periodic)
     hipLaunchKernelGGL((nbr_kernel<T, FILL, true>), nb, th, 0, st, G, a, k);

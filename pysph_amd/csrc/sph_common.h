@@ -145,6 +145,68 @@ __device__ __forceinline__ void cell_xyz(int c, const Grid& g, int& cx, int& cy,
   cz = t / g.dims[1];
 }
 
+// Walk the stencil of cell (cx,cy,cz) with the given ring: cells of one
+// (dy,dz) row are contiguous in the cell-sorted layout, so each row is one
+// particle range [cell_start[first], cell_start[last+1]).
+template <class F>
+__device__ __forceinline__ void for_each_row(const Grid& g, const int* __restrict__ cstart,
+                                             int cx, int cy, int cz, int ring, F&& f) {
+  const int x0 = max(cx - ring, 0), x1 = min(cx + ring, g.dims[0] - 1);
+  const int y0 = max(cy - ring, 0), y1 = min(cy + ring, g.dims[1] - 1);
+  const int z0 = max(cz - ring, 0), z1 = min(cz + ring, g.dims[2] - 1);
+  for (int z = z0; z <= z1; ++z) {
+    for (int y = y0; y <= y1; ++y) {
+      const int base = (z * g.dims[1] + y) * g.dims[0];
+      const int j0 = cstart[base + x0];
+      const int j1 = cstart[base + x1 + 1];
+      f(j0, j1);
+    }
+  }
+}
+
+// Periodic images of a destination at p in cell (cx,cy,cz): f(ox,oy,oz,
+// icx,icy,icz,image) runs for the destination itself (offset 0) and, along
+// periodic axes, for every shift s in {-1,0,1}^3 whose image point p - s*L
+// comes within `reach` of the domain: sources are then seen at x_j + s*L,
+// the ghost copy's coordinate (cell.pyx:1277-1376).  With period > 2*reach
+// a source matches at most one image.  Image cells come from the image
+// point in FP64; unshifted axes keep the destination's own cell.
+template <class F>
+__device__ __forceinline__ void for_each_image(const Grid& g, double px, double py, double pz,
+                                               int cx, int cy, int cz, double reach, F&& f) {
+  f(0.0, 0.0, 0.0, cx, cy, cz, false);
+  if (!g.periodic) return;
+  const double p[3] = {px, py, pz};
+  const int c0[3] = {cx, cy, cz};
+  int lo[3], hi[3];
+  for (int a = 0; a < 3; ++a) {
+    lo[a] = 0;
+    hi[a] = 0;
+    if (g.per[a] > 0.0) {
+      if (p[a] + reach >= g.pmin[a] + g.per[a]) hi[a] = 1;
+      if (p[a] - reach < g.pmin[a]) lo[a] = -1;
+    }
+  }
+  for (int sx = lo[0]; sx <= hi[0]; ++sx)
+    for (int sy = lo[1]; sy <= hi[1]; ++sy)
+      for (int sz = lo[2]; sz <= hi[2]; ++sz) {
+        if (sx == 0 && sy == 0 && sz == 0) continue;
+        const int sh[3] = {sx, sy, sz};
+        double o[3];
+        int c[3];
+        for (int a = 0; a < 3; ++a) {
+          o[a] = sh[a] * g.per[a];
+          if (sh[a] == 0) {
+            c[a] = c0[a];
+          } else {
+            const double k = floor((p[a] - o[a]) / g.cs) - (double)g.lo[a];
+            c[a] = !(k >= 0.0) ? 0 : (k > (double)(g.dims[a] - 1) ? g.dims[a] - 1 : (int)k);
+          }
+        }
+        f(o[0], o[1], o[2], c[0], c[1], c[2], true);
+      }
+}
+
 template <typename T>
 struct View {
   int n;

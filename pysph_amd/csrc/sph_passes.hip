@@ -8,8 +8,8 @@
 //
 // These are the passes over the SoA fields: FP64 storage, variable-h
 // symmetric pairs, periodic axes, density rates and FP32 arrays without
-// packed copies.  A group of 4 to 32 lanes serves one destination
-// (sph_group.h).  Destinations are visited in the cell-sorted layout, so the
+// packed copies.  A group of 4 to 16 lanes serves one destination, in large
+// sets one lane (sph_group.h).  Destinations are visited in the cell-sorted layout, so the
 // groups of a wave share stencil rows and their source reads hit in L1/L2.
 // Candidates are screened in the storage precision and accepted by the
 // reference's exact FP64 test.
@@ -64,75 +64,107 @@ struct GroupDst {
   }
 };
 
+// How the accepted sources of a destination reach its sums.  kQueued: a group
+// of lanes collects them in LDS and runs the pair arithmetic on G of them at a
+// time, so that it keeps the lanes busy (about 60 % of the candidates are
+// accepted with bins of half the search radius, 20 % with bins of the radius).
+// The k-th accepted source goes to lane k mod G, whenever the queue is emptied
+// in between: the sums depend on the neighbours and their order only, not on
+// how far the stencil was widened.  kEach: a group whose lanes sum each pair
+// as they find it, for bodies that cost about as much as queueing.  kAlone:
+// one lane walks the destination's rows itself (group_log2 is 0).
+enum Scan { kEach, kQueued, kAlone };
+
+// LDS of a block for a scan.
+template <Scan SCAN>
+struct ScanLds {
+  GroupRows rows[SCAN == kAlone ? 1 : kBlock / 64];
+  GroupQueue queue[SCAN == kQueued ? kBlock / 64 : 1];
+};
+
 // Every accepted source of source array S: body(j, d2, rx, ry, rz), each lane
-// of the group its share of them.  Accepted candidates are collected in LDS
-// per group and body runs on G of them at a time, so that the pair arithmetic
-// keeps the lanes busy (about 60 % of the candidates are accepted with bins
-// of half the search radius, 20 % with bins of the radius).  The k-th
-// accepted source goes to lane k mod G, whenever the queue is emptied in
-// between: the sums depend on the neighbours and their order only, not on
-// how far the stencil was widened.  Not QUEUED: body runs on each candidate as
-// it is found, for bodies that cost about as much as queueing.
-template <typename T, typename CT, bool PERIODIC, bool QUEUED, class F>
+// of the group its share of them.
+template <typename T, typename CT, bool PERIODIC, Scan SCAN, class F>
 __device__ __forceinline__ void scan_pairs(const Grid& g, const PassArgs<T>& a, const View<T>& S,
-                                           const Group& gr, const GroupDst<T>& D, GroupRows& rows,
-                                           GroupQueue& queue, F&& body) {
-  const int cap = kGroupQueue / (64 / gr.size);
-  int* qj = queue.j + gr.index * cap;
-  uint8_t* qi = queue.image + gr.index * cap;
-  // entries [start, count); start = sources summed so far, mod G
-  int start = 0, count = 0;
-  auto geom = [&](int j, int code, CT& d2, CT& rx, CT& ry, CT& rz) {
-    if (PERIODIC && code != 0)
-      return pair_geom<T, CT>(a, S, j, D.x, D.y, D.z, D.r2f, D.r2d, true,
-                              image_offset(code, 0, g.per[0]), image_offset(code, 1, g.per[1]),
-                              image_offset(code, 2, g.per[2]), d2, rx, ry, rz);
-    return pair_geom<T, CT>(a, S, j, D.x, D.y, D.z, D.r2f, D.r2d, false, 0.0, 0.0, 0.0, d2, rx,
-                            ry, rz);
-  };
-  auto drain = [&]() {
-    wave_lds_fence();
-    for (int k = gr.rank; __any(k - gr.rank < count); k += gr.size) {
-      if (k >= start && k < count) {
-        CT d2, rx, ry, rz;
-        const int j = qj[k];
-        if (geom(j, PERIODIC ? qi[k] : 0, d2, rx, ry, rz)) body(j, d2, rx, ry, rz);
+                                           const Group& gr, const GroupDst<T>& D,
+                                           ScanLds<SCAN>& lds, F&& body) {
+  if constexpr (SCAN == kAlone) {
+    if (!D.local) return;
+    auto rows = [&](double ox, double oy, double oz, int cx, int cy, int cz, bool image) {
+      for_each_row(g, S.cstart, cx, cy, cz, image ? D.ring + 1 : D.ring, [&](int j0, int j1) {
+        for (int j = j0; j < j1; ++j) {
+          CT d2, rx, ry, rz;
+          if (pair_geom<T, CT>(a, S, j, D.x, D.y, D.z, D.r2f, D.r2d, PERIODIC && image, ox, oy, oz,
+                               d2, rx, ry, rz))
+            body(j, d2, rx, ry, rz);
+        }
+      });
+    };
+    if (PERIODIC)
+      for_each_image(g, (double)D.x, (double)D.y, (double)D.z, D.cx, D.cy, D.cz, D.ring * g.cs,
+                     rows);
+    else
+      rows(0.0, 0.0, 0.0, D.cx, D.cy, D.cz, false);
+  } else {
+    const int wid = threadIdx.x >> 6;
+    GroupQueue& queue = lds.queue[SCAN == kQueued ? wid : 0];
+    const int cap = kGroupQueue / (64 / gr.size);
+    int* qj = queue.j + gr.index * cap;
+    uint8_t* qi = queue.image + gr.index * cap;
+    // entries [start, count); start = sources summed so far, mod G
+    int start = 0, count = 0;
+    auto geom = [&](int j, int code, CT& d2, CT& rx, CT& ry, CT& rz) {
+      if (PERIODIC && code != 0)
+        return pair_geom<T, CT>(a, S, j, D.x, D.y, D.z, D.r2f, D.r2d, true,
+                                image_offset(code, 0, g.per[0]), image_offset(code, 1, g.per[1]),
+                                image_offset(code, 2, g.per[2]), d2, rx, ry, rz);
+      return pair_geom<T, CT>(a, S, j, D.x, D.y, D.z, D.r2f, D.r2d, false, 0.0, 0.0, 0.0, d2, rx,
+                              ry, rz);
+    };
+    auto drain = [&]() {
+      wave_lds_fence();
+      for (int k = gr.rank; __any(k - gr.rank < count); k += gr.size) {
+        if (k >= start && k < count) {
+          CT d2, rx, ry, rz;
+          const int j = qj[k];
+          if (geom(j, PERIODIC ? qi[k] : 0, d2, rx, ry, rz)) body(j, d2, rx, ry, rz);
+        }
       }
-    }
-    start = count = count & (gr.size - 1);
-    wave_lds_fence();
-  };
-  group_scan<PERIODIC>(g, S.cstart, gr, rows, D.local, (double)D.x, (double)D.y, (double)D.z, D.cx,
-                       D.cy, D.cz, D.ring, D.rc, [&](bool valid, int j, int code) {
-    CT d2, rx, ry, rz;
-    const bool ok = valid && geom(j, code, d2, rx, ry, rz);
-    if constexpr (QUEUED) {
-      const unsigned m = gr.mine(__ballot(ok));
-      if (ok) {
-        const int at = count + gr.before(m);
-        qj[at] = j;
-        if (PERIODIC) qi[at] = (uint8_t)code;
+      start = count = count & (gr.size - 1);
+      wave_lds_fence();
+    };
+    group_scan<PERIODIC>(g, S.cstart, gr, lds.rows[wid], D.local, (double)D.x, (double)D.y,
+                         (double)D.z, D.cx, D.cy, D.cz, D.ring, D.rc,
+                         [&](bool valid, int j, int code) {
+      CT d2, rx, ry, rz;
+      const bool ok = valid && geom(j, code, d2, rx, ry, rz);
+      if constexpr (SCAN == kQueued) {
+        const unsigned m = gr.mine(__ballot(ok));
+        if (ok) {
+          const int at = count + gr.before(m);
+          qj[at] = j;
+          if (PERIODIC) qi[at] = (uint8_t)code;
+        }
+        count += __popc(m);
+        if (__any(count > cap - gr.size)) drain();
+      } else {
+        if (ok) body(j, d2, rx, ry, rz);
       }
-      count += __popc(m);
-      if (__any(count > cap - gr.size)) drain();
-    } else {
-      if (ok) body(j, d2, rx, ry, rz);
-    }
-  });
-  if constexpr (QUEUED) drain();
+    });
+    if constexpr (SCAN == kQueued) drain();
+  }
 }
 
-// QUEUED when the stencil may be widened (disp) or sums are cached: sums over
+// kQueued when the stencil may be widened (disp) or sums are cached: sums over
 // a widened stencil then have the bits of the plain ones.  Otherwise each
 // pair is summed as it is found (FP64, 300k clustered points: 349 against
 // 406 us a pass).
-template <typename T, typename CT, bool TAIT, bool PERIODIC, bool QUEUED>
+template <typename T, typename CT, bool TAIT, bool PERIODIC, Scan SCAN>
 __global__ __launch_bounds__(kBlock) void density_kernel(Grid g, PassArgs<T> a, int log2) {
-  __shared__ GroupRows rows[kBlock / 64];
-  __shared__ GroupQueue queue[QUEUED ? kBlock / 64 : 1];
-  const Group gr(log2);
-  const GroupDst<T> D(g, a, gr, log2);
-  const int i = D.i, wid = threadIdx.x >> 6;
+  __shared__ ScanLds<SCAN> lds;
+  const Group gr(SCAN == kAlone ? 0 : log2);
+  const GroupDst<T> D(g, a, gr, SCAN == kAlone ? 0 : log2);
+  const int i = D.i;
   const int dim = a.dim;
   CT rho = CT(0);
   for (int s = 0; s < a.nsrc; ++s) {
@@ -142,8 +174,7 @@ __global__ __launch_bounds__(kBlock) void density_kernel(Grid g, PassArgs<T> a, 
       // stored partial sum of a static source
       if (D.local) nr = (CT)a.cache_sums[i];
     } else {
-      scan_pairs<T, CT, PERIODIC, QUEUED>(g, a, S, gr, D, rows[wid],
-                                          queue[QUEUED ? wid : 0], [&](int j, CT d2, CT, CT, CT) {
+      scan_pairs<T, CT, PERIODIC, SCAN>(g, a, S, gr, D, lds, [&](int j, CT d2, CT, CT, CT) {
         const CT hab = CT(0.5) * ((CT)D.h + (CT)S.h[j]);
         const CT inv = CT(1) / hab;
         const CT q = sqrt(d2) * inv;
@@ -182,13 +213,12 @@ __global__ __launch_bounds__(kBlock) void density_kernel(Grid g, PassArgs<T> a, 
 
 // SPHDensityRate (density_funcs.pyx:89-158): sum_b m_b (v_a - v_b) .
 // grad_a W_ab with h_ab = (h_a + h_b)/2; non-LocalReal destinations get 0.
-template <typename T, typename CT, bool PERIODIC>
+template <typename T, typename CT, bool PERIODIC, Scan SCAN>
 __global__ __launch_bounds__(kBlock) void density_rate_kernel(Grid g, PassArgs<T> a, int log2) {
-  __shared__ GroupRows rows[kBlock / 64];
-  __shared__ GroupQueue queue[kBlock / 64];
-  const Group gr(log2);
-  const GroupDst<T> D(g, a, gr, log2);
-  const int i = D.i, wid = threadIdx.x >> 6;
+  __shared__ ScanLds<SCAN> lds;
+  const Group gr(SCAN == kAlone ? 0 : log2);
+  const GroupDst<T> D(g, a, gr, SCAN == kAlone ? 0 : log2);
+  const int i = D.i;
   T ud = T(0), vd = T(0), wd = T(0);
   if (D.local) {
     ud = a.dst.u[i];
@@ -201,8 +231,7 @@ __global__ __launch_bounds__(kBlock) void density_rate_kernel(Grid g, PassArgs<T
   for (int s = 0; s < a.nsrc; ++s) {
     const View<T> S = a.src[s];
     CT nr = CT(0);
-    scan_pairs<T, CT, PERIODIC, true>(g, a, S, gr, D, rows[wid], queue[wid],
-                                      [&](int j, CT d2, CT rx, CT ry, CT rz) {
+    scan_pairs<T, CT, PERIODIC, SCAN>(g, a, S, gr, D, lds, [&](int j, CT d2, CT rx, CT ry, CT rz) {
       const CT hab = CT(0.5) * (ha + (CT)S.h[j]);
       const CT inv = CT(1) / hab;
       const CT rr = sqrt(d2);
@@ -237,13 +266,12 @@ __global__ __launch_bounds__(kBlock) void tait_kernel(int n, const T* __restrict
 
 // MODE 0: write acc / dv.  MODE 1: RK2 predictor.  MODE 2: RK2 final.
 // MODE 3: Euler.
-template <typename T, typename CT, int MODE, bool PERIODIC>
+template <typename T, typename CT, int MODE, bool PERIODIC, Scan SCAN>
 __global__ __launch_bounds__(kBlock) void momentum_kernel(Grid g, PassArgs<T> a, int log2) {
-  __shared__ GroupRows rows[kBlock / 64];
-  __shared__ GroupQueue queue[kBlock / 64];
-  const Group gr(log2);
-  const GroupDst<T> D(g, a, gr, log2);
-  const int i = D.i, wid = threadIdx.x >> 6;
+  __shared__ ScanLds<SCAN> lds;
+  const Group gr(SCAN == kAlone ? 0 : log2);
+  const GroupDst<T> D(g, a, gr, SCAN == kAlone ? 0 : log2);
+  const int i = D.i;
   const int dim = a.dim;
   const bool local = D.local;
   CT acc[3] = {CT(0), CT(0), CT(0)};
@@ -269,8 +297,7 @@ __global__ __launch_bounds__(kBlock) void momentum_kernel(Grid g, PassArgs<T> a,
     if (!do_m && !do_x) continue;
     CT am[3] = {CT(0), CT(0), CT(0)};
     CT ax[3] = {CT(0), CT(0), CT(0)};
-    scan_pairs<T, CT, PERIODIC, true>(g, a, S, gr, D, rows[wid], queue[wid],
-                                      [&](int j, CT d2, CT rx, CT ry, CT rz) {
+    scan_pairs<T, CT, PERIODIC, SCAN>(g, a, S, gr, D, lds, [&](int j, CT d2, CT rx, CT ry, CT rz) {
       const CT hab = CT(0.5) * (ha + (CT)S.h[j]);
       const CT inv = CT(1) / hab;
       const CT rr = sqrt(d2);
@@ -369,7 +396,7 @@ __global__ __launch_bounds__(kBlock) void momentum_kernel(Grid g, PassArgs<T> a,
     float disp = move_bound(mv2);
     for (int off = 32; off > 0; off >>= 1) disp = fmaxf(disp, __shfl_xor(disp, off, 64));
     __shared__ float bmax[kBlock / 64];
-    if ((threadIdx.x & 63) == 0) bmax[wid] = disp;
+    if ((threadIdx.x & 63) == 0) bmax[threadIdx.x >> 6] = disp;
     __syncthreads();
     if (threadIdx.x == 0) {
       for (int k = 1; k < kBlock / 64; ++k) disp = fmaxf(disp, bmax[k]);
@@ -421,64 +448,82 @@ static int32_t check_common(const sph_grid* g, const sph_params* prm, const sph_
 }
 
 
-template <typename T, typename CT, bool TAIT, bool QUEUED>
-static void launch_density_q(hipStream_t st, const Grid& G, const PassArgs<T>& a) {
-  const int k = group_log2(a.dst.n, a.nsrc);
+template <typename T, typename CT, bool TAIT, Scan SCAN>
+static void launch_density_s(hipStream_t st, const Grid& G, const PassArgs<T>& a, int k) {
   const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
   if (G.periodic)
-    hipLaunchKernelGGL((density_kernel<T, CT, TAIT, true, QUEUED>), nb, th, 0, st, G, a, k);
+    hipLaunchKernelGGL((density_kernel<T, CT, TAIT, true, SCAN>), nb, th, 0, st, G, a, k);
   else
-    hipLaunchKernelGGL((density_kernel<T, CT, TAIT, false, QUEUED>), nb, th, 0, st, G, a, k);
+    hipLaunchKernelGGL((density_kernel<T, CT, TAIT, false, SCAN>), nb, th, 0, st, G, a, k);
+}
+
+template <typename T, typename CT, bool TAIT>
+static void launch_density_t(hipStream_t st, const Grid& G, const PassArgs<T>& a) {
+  const int k = group_log2(a.dst.n, a.nsrc, a.dim < 3, G.periodic);
+  if (k == 0)
+    launch_density_s<T, CT, TAIT, kAlone>(st, G, a, k);
+  else if (a.disp != nullptr || a.cache_src >= 0)
+    launch_density_s<T, CT, TAIT, kQueued>(st, G, a, k);
+  else
+    launch_density_s<T, CT, TAIT, kEach>(st, G, a, k);
 }
 
 template <typename T, typename CT>
 static void launch_density(hipStream_t st, const Grid& G, const PassArgs<T>& a, bool tait) {
-  const bool queued = a.disp != nullptr || a.cache_src >= 0;
-  if (tait) {
-    if (queued) launch_density_q<T, CT, true, true>(st, G, a);
-    else launch_density_q<T, CT, true, false>(st, G, a);
-  } else {
-    if (queued) launch_density_q<T, CT, false, true>(st, G, a);
-    else launch_density_q<T, CT, false, false>(st, G, a);
-  }
+  if (tait)
+    launch_density_t<T, CT, true>(st, G, a);
+  else
+    launch_density_t<T, CT, false>(st, G, a);
+}
+
+template <typename T, typename CT, Scan SCAN>
+static void launch_rate_s(hipStream_t st, const Grid& G, const PassArgs<T>& a, int k) {
+  const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
+  if (G.periodic)
+    hipLaunchKernelGGL((density_rate_kernel<T, CT, true, SCAN>), nb, th, 0, st, G, a, k);
+  else
+    hipLaunchKernelGGL((density_rate_kernel<T, CT, false, SCAN>), nb, th, 0, st, G, a, k);
 }
 
 template <typename T, typename CT>
 static void launch_rate(hipStream_t st, const Grid& G, const PassArgs<T>& a) {
-  const int k = group_log2(a.dst.n, a.nsrc);
-  const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
-  if (G.periodic)
-    hipLaunchKernelGGL((density_rate_kernel<T, CT, true>), nb, th, 0, st, G, a, k);
+  const int k = group_log2(a.dst.n, a.nsrc, a.dim < 3, G.periodic);
+  if (k == 0)
+    launch_rate_s<T, CT, kAlone>(st, G, a, k);
   else
-    hipLaunchKernelGGL((density_rate_kernel<T, CT, false>), nb, th, 0, st, G, a, k);
+    launch_rate_s<T, CT, kQueued>(st, G, a, k);
 }
 
-template <typename T, typename CT, bool PERIODIC>
-static void launch_momentum_p(hipStream_t st, const Grid& G, const PassArgs<T>& a, int mode) {
-  const int k = group_log2(a.dst.n, a.nsrc);
+template <typename T, typename CT, bool PERIODIC, Scan SCAN>
+static void launch_momentum_s(hipStream_t st, const Grid& G, const PassArgs<T>& a, int mode,
+                              int k) {
   const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
   switch (mode) {
     case 0:
-      hipLaunchKernelGGL((momentum_kernel<T, CT, 0, PERIODIC>), nb, th, 0, st, G, a, k);
+      hipLaunchKernelGGL((momentum_kernel<T, CT, 0, PERIODIC, SCAN>), nb, th, 0, st, G, a, k);
       break;
     case 1:
-      hipLaunchKernelGGL((momentum_kernel<T, CT, 1, PERIODIC>), nb, th, 0, st, G, a, k);
+      hipLaunchKernelGGL((momentum_kernel<T, CT, 1, PERIODIC, SCAN>), nb, th, 0, st, G, a, k);
       break;
     case 2:
-      hipLaunchKernelGGL((momentum_kernel<T, CT, 2, PERIODIC>), nb, th, 0, st, G, a, k);
+      hipLaunchKernelGGL((momentum_kernel<T, CT, 2, PERIODIC, SCAN>), nb, th, 0, st, G, a, k);
       break;
     default:
-      hipLaunchKernelGGL((momentum_kernel<T, CT, 3, PERIODIC>), nb, th, 0, st, G, a, k);
+      hipLaunchKernelGGL((momentum_kernel<T, CT, 3, PERIODIC, SCAN>), nb, th, 0, st, G, a, k);
       break;
   }
 }
 
 template <typename T, typename CT>
 static void launch_momentum(hipStream_t st, const Grid& G, const PassArgs<T>& a, int mode) {
-  if (G.periodic)
-    launch_momentum_p<T, CT, true>(st, G, a, mode);
-  else
-    launch_momentum_p<T, CT, false>(st, G, a, mode);
+  const int k = group_log2(a.dst.n, a.nsrc, a.dim < 3, G.periodic);
+  if (G.periodic) {
+    if (k == 0) launch_momentum_s<T, CT, true, kAlone>(st, G, a, mode, k);
+    else launch_momentum_s<T, CT, true, kQueued>(st, G, a, mode, k);
+  } else {
+    if (k == 0) launch_momentum_s<T, CT, false, kAlone>(st, G, a, mode, k);
+    else launch_momentum_s<T, CT, false, kQueued>(st, G, a, mode, k);
+  }
 }
 
 template <typename T>
