@@ -665,15 +665,18 @@ __device__ __forceinline__ void group_sort(const Group& gr, int64_t* v, int n) {
 // Neighbour counts, or the CSR rows, each sorted ascending by id.  A group of
 // lanes collects a row's ids in LDS, ranks every entry against the others
 // there and writes it to its place; rows longer than the group's share of LDS
-// go to the output as they are found and are sorted in place.  (One lane per
-// destination, insertion-sorting its row in global memory: 626 us for 50k
-// particles with 58 neighbours each in FP64; now 127 us.)
+// go to the output as they are found and are sorted in place.  Rows whose ids
+// are found in ascending order (slots of cell-ordered sources) are neither
+// ranked nor sorted.  (One lane per destination, insertion-sorting its row in
+// global memory: 626 us for 50k particles with 58 neighbours each in FP64; now
+// 127 us.  Ascending ids, FP32, 100k particles in 3D: 201 and 115 us, 4M in 2D:
+// 1.09 and 1.10 ms; ranked and sorted all the same: 287 us and 2.16 ms.)
 template <typename T, bool FILL, bool PERIODIC>
 __global__ __launch_bounds__(kBlock) void nbr_kernel(Grid g, NbrArgs<T> a, int log2) {
   __shared__ GroupRows rows[kBlock / 64];
   // odd pitch: the groups of a wave read one entry each at a time, in
   // different banks
-  __shared__ int64_t qbuf[FILL ? kBlock / 64 : 1][FILL ? kNbrQueue + 16 : 1];
+  __shared__ int64_t qbuf[FILL ? kBlock / 64 : 1][FILL ? kNbrQueue + 64 : 1];
   const Group gr(log2);
   const int wid = threadIdx.x >> 6;
   const int bid = xcd_block(blockIdx.x, gridDim.x);
@@ -712,7 +715,9 @@ __global__ __launch_bounds__(kBlock) void nbr_kernel(Grid g, NbrArgs<T> a, int l
   group_scan<PERIODIC>(g, S.cstart, gr, rows[wid], valid, (double)xd, (double)yd, (double)zd, cx,
                        cy, cz, ring, reach, [&](bool has, int j, int code) {
     bool hit = false;
+    int64_t id = 0;
     if (has) {
+      if (FILL) id = a.ids != nullptr ? a.ids[j] : j;  // beside the position, not after the test
       double r2 = r2d;
       if (a.rmax_sym > 0) {
         // the reverse locator's test: d2 < (h_s * rs)^2 (nnps.pyx:735-747)
@@ -729,7 +734,6 @@ __global__ __launch_bounds__(kBlock) void nbr_kernel(Grid g, NbrArgs<T> a, int l
     }
     const unsigned m = gr.mine(__ballot(hit));
     if constexpr (FILL) {
-      const int64_t id = hit ? (a.ids != nullptr ? a.ids[j] : j) : 0;
       const bool spill = !spilled && count + __popc(m) > cap;
       if (__any(spill)) {
         // the row outgrows its place in LDS: move it to the output
@@ -757,20 +761,28 @@ __global__ __launch_bounds__(kBlock) void nbr_kernel(Grid g, NbrArgs<T> a, int l
   const int64_t self = a.self_last ? row : -1;
   wave_lds_fence();
   if (!spilled) {
-    // rank of each entry among the row's (ties: by place)
-    bool own = false;
-    int below = 0;  // rank of the own id
-    if (a.self_last)
-      for (int k = 0; k < count; ++k) {
-        own = own || q[k] == self;
-        below += q[k] < self ? 1 : 0;
+    bool mixed = false, found = false;
+    int less = 0;
+    for (int k = gr.rank; k < count; k += gr.size) {
+      mixed = mixed || (k > 0 && !(q[k - 1] < q[k]));
+      if (a.self_last) {
+        found = found || q[k] == self;
+        less += q[k] < self ? 1 : 0;
       }
+    }
+    const bool sorted = gr.mine(__ballot(mixed)) == 0;
+    const bool own = a.self_last && gr.mine(__ballot(found)) != 0;
+    const int below = gr.sum(less);  // rank of the own id
     for (int e = gr.rank; e < count; e += gr.size) {
       const int64_t id = q[e];
-      int rank = 0;
-      for (int k = 0; k < count; ++k) {
-        const int64_t o = q[k];
-        rank += o < id || (o == id && k < e) ? 1 : 0;
+      int rank = e;
+      if (!sorted) {
+        // rank among the row's entries (ties: by place)
+        rank = 0;
+        for (int k = 0; k < count; ++k) {
+          const int64_t o = q[k];
+          rank += o < id || (o == id && k < e) ? 1 : 0;
+        }
       }
       if (own) {  // the own id and the last entry change places
         if (id == self) rank = count - 1;
@@ -786,11 +798,15 @@ __global__ __launch_bounds__(kBlock) void nbr_kernel(Grid g, NbrArgs<T> a, int l
     const int64_t room = limit - first;
     const int len = !spilled || room <= 0 ? 0 : (int)(room < count ? room : count);
     int64_t* v = a.out + (len > 0 ? first : 0);
-    group_sort(gr, v, len);
+    bool mixed = false;
+    for (int k = gr.rank + 1; k < len; k += gr.size) mixed = mixed || !(v[k - 1] < v[k]);
+    const bool sorted = gr.mine(__ballot(mixed)) == 0;
+    if (__any(!sorted)) group_sort(gr, v, sorted ? 0 : len);
     if (a.self_last) {
-      int at = -1;
-      for (int k = 0; k < len; ++k)
-        if (v[k] == self) at = k;
+      int at = 0;  // place of the own id, which a row holds at most once
+      for (int k = gr.rank; k < len; k += gr.size)
+        if (v[k] == self) at = k + 1;
+      at = gr.sum(at) - 1;
       if (at >= 0 && gr.rank == 0) {
         v[at] = v[len - 1];
         v[len - 1] = self;
@@ -812,7 +828,7 @@ static NbrArgs<T> nbr_args(const sph_view* dst, const sph_view* src, double radi
 
 template <bool FILL, typename T>
 static void launch_nbr(hipStream_t st, const Grid& G, const NbrArgs<T>& a) {
-  const int k = a.dst.n < (1 << 14) ? 4 : 3;
+  const int k = a.dst.n < (1 << 14) ? 4 : (G.dims[2] == 1 && a.dst.n >= (1 << 17) ? 2 : 3);
   const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
   if (G.periodic)
     hipLaunchKernelGGL((nbr_kernel<T, FILL, true>), nb, th, 0, st, G, a, k);

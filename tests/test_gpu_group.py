@@ -11,6 +11,7 @@ terms of one sign per particle: 1e3 * 2^-53 = 1.1e-13 relative; accelerations
 normwise)."""
 import numpy as np
 import pytest
+import torch
 
 import pysph_amd.base.api as base
 import pysph_amd.solver.api as solver
@@ -180,3 +181,61 @@ def test_row_fill_sorts_short_and_long_rows(n, dim, h, shuffled):
     off2, nb2 = neighbor_csr(particles.cell_manager, a, a, 2.0)
     assert np.array_equal(off2, off)
     assert all(np.all(np.diff(nb2[off2[i]:off2[i + 1]]) > 0) for i in range(n))
+
+
+@pytest.mark.parametrize("n,dim,h", [(65, 3, 0.2), (3000, 2, 0.15), (3000, 3, 0.25),
+                                     (17000, 3, 0.06), ((1 << 17) + 5, 2, 0.0045)])
+@pytest.mark.parametrize("kind", ["varh", "periodic"])
+@pytest.mark.parametrize("ascending", [False, True])
+def test_row_fill_of_symmetric_and_periodic_rows(n, dim, h, kind, ascending):
+    """Short rows and rows of several hundred entries of the symmetric
+    variable-h sets and of periodic ones (whose walk order is not ascending),
+    with user ids and with slot ids, which are found in order: the oracle's
+    sets, sorted."""
+    from pysph_amd import _abi
+    from pysph_amd._device import require_gpu
+    a = _points(n, dim, h, 12, Fluid)
+    rng = np.random.Generator(np.random.PCG64(3))
+    if kind == "varh":
+        a.set(h=h * (0.6 + 0.8 * rng.random(n)))
+    dom = None
+    if kind == "periodic":
+        if 4 * h >= 1:
+            pytest.skip("the box holds less than two search radii")
+        dom = base.PeriodicDomain(xmin=0.0, xmax=1.0, ymin=0.0, ymax=1.0)
+    particles = base.Particles([a], variable_h=kind == "varh", periodic_domain=dom)
+    cm = particles.cell_manager
+    cm.update()
+    ao = to_oracle(a)
+    if kind == "periodic":
+        ext, origin = O.with_ghosts(ao, (1.0, 1.0, 0.0), (0.0, 0.0, 0.0), cm.cell_size,
+                                    cm.cell_size)
+        off_o, nb_o = O.nnps_csr(ao, ext, radius_scale=2.0, cell_size=cm.cell_size)
+        nb_o = origin[nb_o]
+    else:
+        off_o, nb_o = O.nnps_csr(ao, radius_scale=2.0, varh=True)
+    stream = require_gpu(a.get_carray("x"))
+    v = a.view()
+    slots = torch.arange(n, dtype=torch.int64, device=a.device)
+    order = slots if a._order is None else a._order
+    ids = slots if ascending else order
+    counts = torch.empty(n, dtype=torch.int64, device=a.device)
+    off = torch.empty(n + 1, dtype=torch.int64, device=a.device)
+    total = _abi.ctypes.c_int64(0)
+    rmax = 2.0 * cm.max_h if kind == "varh" else 0.0
+    _abi.call("sph_neighbor_row_counts", stream, cm.grid, v, v, 2.0, rmax, order.data_ptr(),
+              counts.data_ptr())
+    _abi.call("sph_scan_counts", stream, n, counts.data_ptr(), off.data_ptr(),
+              _abi.ctypes.byref(total))
+    nbr = torch.empty(total.value, dtype=torch.int64, device=a.device)
+    _abi.call("sph_neighbor_row_fill", stream, cm.grid, v, v, 2.0, rmax, order.data_ptr(),
+              ids.data_ptr(), off.data_ptr(), nbr.data_ptr(), total.value, total.value, 0)
+    assert np.array_equal(off.cpu().numpy(), off_o)
+    nb = nbr.cpu().numpy()
+    rows = np.repeat(np.arange(n), np.diff(off_o))
+    inside = rows[1:] == rows[:-1]
+    assert (nb[1:] > nb[:-1])[inside].all()
+    users = order.cpu().numpy()[nb] if ascending else nb
+    key = np.lexsort((users, rows))
+    ref = np.lexsort((nb_o, rows))
+    assert np.array_equal(users[key], nb_o[ref])
