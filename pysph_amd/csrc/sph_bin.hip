@@ -635,6 +635,24 @@ __device__ __forceinline__ bool pair_within<double>(double xs, double ys, double
   return exact_within(xs, ys, zs, xd, yd, zd, r2d);
 }
 
+// Radius and stencil of destination i (none: -1): r = h * scale, the
+// eff_radius of nnps.pyx:552; ring = ceil(r/cs) cells (cell.pyx:1127-1129).
+// The symmetric sets also reach sources whose own radius covers the pair.
+struct NbrReach {
+  double r2d, reach;
+  int ring;
+  template <typename T>
+  __device__ __forceinline__ NbrReach(const Grid& g, const NbrArgs<T>& a, int i) {
+    const double r = i >= 0 ? (double)a.dst.h[i] * a.rs : 0.0;
+    r2d = r * r;
+    reach = a.rmax_sym > fabs(r) ? a.rmax_sym : fabs(r);
+    const double rd = ceil(reach / g.cs);
+    const int full = max(g.dims[0], max(g.dims[1], g.dims[2]));
+    ring = !(rd < (double)full) ? full : (int)rd;
+    if (ring < 1) ring = 1;
+  }
+};
+
 constexpr int kNbrQueue = 1024;  // row entries in LDS per wave, shared by its groups
 
 // Ascending in-place sort of v[0..n) in global memory by the lanes of a group
@@ -683,25 +701,17 @@ __global__ __launch_bounds__(kBlock) void nbr_kernel(Grid g, NbrArgs<T> a, int l
   const int i = (bid * (kBlock / 64) + wid) * (64 >> log2) + gr.index;
   const bool valid = i < a.dst.n;
   T xd = T(0), yd = T(0), zd = T(0);
-  double r = 0.0;
   int cx = 0, cy = 0, cz = 0;
   int64_t row = 0;
   if (valid) {
     xd = a.dst.x[i];
     yd = a.dst.y[i];
     zd = a.dst.z[i];
-    r = (double)a.dst.h[i] * a.rs;  // eff_radius (nnps.pyx:552)
     cell_xyz(a.dst.cell[i], g, cx, cy, cz);
     row = a.rows != nullptr ? a.rows[i] : i;
   }
-  const double r2d = r * r;
-  // ring = ceil(r/cs) for this destination (cell.pyx:1127-1129); the
-  // symmetric sets also reach sources whose own radius covers the pair
-  const double reach = a.rmax_sym > fabs(r) ? a.rmax_sym : fabs(r);
-  const double rd = ceil(reach / g.cs);
-  const int full = max(g.dims[0], max(g.dims[1], g.dims[2]));
-  int ring = !(rd < (double)full) ? full : (int)rd;
-  if (ring < 1) ring = 1;
+  const NbrReach R(g, a, valid ? i : -1);
+  const double r2d = R.r2d;
   const View<T>& S = a.src;
   const int cap = kNbrQueue / (64 / gr.size);
   int64_t* q = FILL ? &qbuf[wid][gr.index * (cap + 1)] : nullptr;
@@ -713,7 +723,7 @@ __global__ __launch_bounds__(kBlock) void nbr_kernel(Grid g, NbrArgs<T> a, int l
     if (first + k < limit) a.out[first + k] = id;
   };
   group_scan<PERIODIC>(g, S.cstart, gr, rows[wid], valid, (double)xd, (double)yd, (double)zd, cx,
-                       cy, cz, ring, reach, [&](bool has, int j, int code) {
+                       cy, cz, R.ring, R.reach, [&](bool has, int j, int code) {
     bool hit = false;
     int64_t id = 0;
     if (has) {
@@ -826,14 +836,87 @@ static NbrArgs<T> nbr_args(const sph_view* dst, const sph_view* src, double radi
   return a;
 }
 
+// Counts of a large set, one lane per destination: rows narrowed to the search
+// sphere (as in group_scan) where the ring holds more than the adjacent bins.
+template <typename T, bool PERIODIC>
+__global__ __launch_bounds__(kBlock) void nbr_count_kernel(Grid g, NbrArgs<T> a) {
+  const int i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  if (i >= a.dst.n) return;
+  const T xd = a.dst.x[i], yd = a.dst.y[i], zd = a.dst.z[i];
+  int cx, cy, cz;
+  cell_xyz(a.dst.cell[i], g, cx, cy, cz);
+  const NbrReach R(g, a, i);
+  const View<T>& S = a.src;
+  int count = 0;
+  auto pairs = [&](int j0, int j1, double ox, double oy, double oz, bool image) {
+    for (int j = j0; j < j1; ++j) {
+      bool hit;
+      if (!PERIODIC || !image)
+        hit = pair_within<T>(S.x[j], S.y[j], S.z[j], xd, yd, zd, (float)R.r2d, R.r2d);
+      else  // a ghost copy's coordinate, x_j + s*L, in FP64 (cell.pyx:1277-1376)
+        hit = exact_within((double)S.x[j] + ox, (double)S.y[j] + oy, (double)S.z[j] + oz,
+                           (double)xd, (double)yd, (double)zd, R.r2d);
+      count += hit ? 1 : 0;
+    }
+  };
+  if (PERIODIC) {
+    for_each_image(g, (double)xd, (double)yd, (double)zd, cx, cy, cz, R.ring * g.cs,
+                   [&](double ox, double oy, double oz, int ix, int iy, int iz, bool image) {
+      for_each_row(g, S.cstart, ix, iy, iz, image ? R.ring + 1 : R.ring,
+                   [&](int j0, int j1) { pairs(j0, j1, ox, oy, oz, image); });
+    });
+  } else if (R.ring > 1 && can_cull(g, (double)xd, (double)yd, (double)zd, R.reach)) {
+    const Cull cu = make_cull(make_float4((float)xd, (float)yd, (float)zd, 0.f), R.reach, g);
+    for (int z = max(cz - R.ring, 0); z <= min(cz + R.ring, g.dims[2] - 1); ++z)
+      for (int y = max(cy - R.ring, 0); y <= min(cy + R.ring, g.dims[1] - 1); ++y) {
+        int j0, j1;
+        row_range_cull(g, S.cstart, cx, y, z, R.ring, cu, j0, j1);
+        pairs(j0, j1, 0.0, 0.0, 0.0, false);
+      }
+  } else {
+    for_each_row(g, S.cstart, cx, cy, cz, R.ring,
+                 [&](int j0, int j1) { pairs(j0, j1, 0.0, 0.0, 0.0, false); });
+  }
+  a.counts[a.rows != nullptr ? a.rows[i] : i] = count;
+}
+
+// Lanes per destination (log2) of the groups, 0: nbr_count_kernel.  Counting
+// costs little beside a group's rows and ballots, so one lane pays from 2^17
+// particles on in flat sets (one layer of bins) and, in FP32, whose pairs are
+// half the bytes, from 2^19 in 3D.  In us, 1 / 4 / 8 lanes:
+//   2D FP32  100k: 18 / 16 / 16   200k: 23 / 24 / 27   1M: 73 / 90 / 112
+//            4M: 257 / 342 / 431   (FP64: 381 / 395 / 504)
+//   3D FP32  200k: 99 / 102 / 91   400k: 164 / 175 / 168   1M: 351 / 406 / 400
+//            16M, bins of 1 and of 1/2 the radius: 7157, 5034 / 7115, 6339 / 7418, 6324
+//   3D FP64  1M: 523 / 416 / 437   4M: 1904 / 1541 / 1677
+// Symmetric rows are dearer: 2D FP32 4M: 518 / 512 / 614, 3D 3413 / 3207 / 2853.
+// Filled rows need the group's share of LDS: 128 entries with eight lanes, 64
+// with four, enough in 2D (4M: 1.96 / 2.16 ms; 3D 1M: 4.88 / 2.53 ms).
+template <typename T>
+static int nbr_log2(const Grid& G, const NbrArgs<T>& a, bool fill) {
+  const int64_t n = a.dst.n;
+  const bool flat = G.dims[2] == 1;
+  if (n < (1 << 14)) return 4;
+  if (!fill && a.rmax_sym <= 0 && (flat ? n >= (1 << 17) : sizeof(T) == 4 && n >= (1 << 19)))
+    return 0;
+  if (flat) return n >= (1 << 17) ? 2 : 3;
+  return !fill && a.rmax_sym <= 0 && n >= (1 << 19) ? 2 : 3;
+}
+
 template <bool FILL, typename T>
 static void launch_nbr(hipStream_t st, const Grid& G, const NbrArgs<T>& a) {
-  const int k = a.dst.n < (1 << 14) ? 4 : (G.dims[2] == 1 && a.dst.n >= (1 << 17) ? 2 : 3);
+  const int k = nbr_log2(G, a, FILL);
   const dim3 nb(group_blocks(a.dst.n, k)), th(kBlock);
-  if (G.periodic)
+  if (!FILL && k == 0) {
+    if (G.periodic)
+      hipLaunchKernelGGL((nbr_count_kernel<T, true>), nb, th, 0, st, G, a);
+    else
+      hipLaunchKernelGGL((nbr_count_kernel<T, false>), nb, th, 0, st, G, a);
+  } else if (G.periodic) {
     hipLaunchKernelGGL((nbr_kernel<T, FILL, true>), nb, th, 0, st, G, a, k);
-  else
+  } else {
     hipLaunchKernelGGL((nbr_kernel<T, FILL, false>), nb, th, 0, st, G, a, k);
+  }
 }
 
 }  // namespace sph

@@ -34,6 +34,12 @@ __device__ __forceinline__ Cull make_cull(const float4& pd, double rc, const Gri
   return c;
 }
 
+// The cull runs in FP32 (its radius carries the margin for that); points,
+// radii or cells outside its range take the whole ring.
+__device__ __forceinline__ bool can_cull(const Grid& g, double x, double y, double z, double rc) {
+  return fabs(x) + fabs(y) + fabs(z) < 1e30 && fabs(rc) < 1e15 && g.cs > 1e-15 && g.cs < 1e15;
+}
+
 // Stencil offsets [a, b] (within +-ring) along one axis whose cells can
 // hold a point within the cull radius of v; border cells reach to infinity.
 // The margin of the cull radius covers the FP32 rounding of the bounds, as

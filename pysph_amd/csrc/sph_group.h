@@ -195,10 +195,7 @@ __device__ __forceinline__ void group_scan(const Grid& g, const int* __restrict_
       code = d[0] + 3 * d[1] + 9 * d[2];
       iring = ring + 1;
     }
-    // the cull runs in FP32 (its radius carries the margin for that); points,
-    // radii or cells outside its range take the whole ring
-    const bool cull = fabs(qx) + fabs(qy) + fabs(qz) < 1e30 && fabs(rc) < 1e15 &&
-                      g.cs > 1e-15 && g.cs < 1e15;
+    const bool cull = can_cull(g, qx, qy, qz, rc);
     Cull cu{};
     int ylo = max(-iring, -icy), yhi = min(iring, g.dims[1] - 1 - icy);
     int zlo = max(-iring, -icz), zhi = min(iring, g.dims[2] - 1 - icz);
