@@ -359,6 +359,11 @@ int32_t sph_density_multi(void *stream, const sph_grid *g, const sph_params *prm
                           const sph_view *srcs, double rmax, const float *disp_dev,
                           void *const *rho_dev, void *const *p_dev, void *const *cs_dev);
 
+/* Lanes of a wavefront that share one destination in the passes over the SoA
+ * fields (FP64, variable-h, periodic and density-rate sums): n destinations,
+ * nsrc sources.  n times the lanes stays below 2^32, the threads of a launch. */
+int32_t sph_pass_lanes(int64_t n, int32_t nsrc, int32_t dim, int32_t periodic);
+
 /* SPHDensityRate over all sources (density_funcs.pyx:89-158, hks off):
  * rate_dev[a] = sum_b m_b (v_a - v_b) . grad_a W(r_a - r_b, (h_a+h_b)/2),
  * the continuity-equation density derivative.  Reads x,y,z,h,u,v,w of the

@@ -205,6 +205,8 @@ _SIGS = {
     "sph_batch_density": (ctypes.c_int32, [_vp, _vp, ctypes.c_int32, ctypes.c_int32,
                                            _P(SphBatchSched)]),
     "sph_batch_stage": (ctypes.c_int32, [_vp, _vp, ctypes.c_int32, _P(SphBatchSched)]),
+    "sph_pass_lanes": (ctypes.c_int32, [ctypes.c_int64, ctypes.c_int32, ctypes.c_int32,
+                                        ctypes.c_int32]),
     "sph_mlp_param_count": (ctypes.c_int64, []),
     "sph_mlp_create": (ctypes.c_int32, [_P(_vp)]),
     "sph_mlp_destroy": (ctypes.c_int32, [_vp]),

@@ -899,8 +899,8 @@ static int nbr_log2(const Grid& G, const NbrArgs<T>& a, bool fill) {
   if (n < (1 << 14)) return 4;
   if (!fill && a.rmax_sym <= 0 && (flat ? n >= (1 << 17) : sizeof(T) == 4 && n >= (1 << 19)))
     return 0;
-  if (flat) return n >= (1 << 17) ? 2 : 3;
-  return !fill && a.rmax_sym <= 0 && n >= (1 << 19) ? 2 : 3;
+  if (flat) return fit_log2(n, n >= (1 << 17) ? 2 : 3);
+  return fit_log2(n, !fill && a.rmax_sym <= 0 && n >= (1 << 19) ? 2 : 3);
 }
 
 template <bool FILL, typename T>

@@ -23,6 +23,13 @@
 
 namespace sph {
 
+// k, or the largest smaller number of lanes (log2) with which n destinations
+// fit in one launch: a grid holds less than 2^32 threads.
+inline int fit_log2(int64_t n, int k) {
+  while (k > 0 && (n << k) > (int64_t(1) << 32) - kBlock) --k;
+  return k;
+}
+
 // Lanes per destination (log2); 0: the plain loops of one lane (for_each_row).
 // Eight is the best split from 16k particles on (FP64 momentum of 40k
 // particles in 2D: 82 / 68 / 77 us with 4 / 8 / 16 lanes, FP32 periodic in 3D,
@@ -44,7 +51,7 @@ namespace sph {
 inline int group_log2(int64_t n, int nsrc, bool flat, bool periodic) {
   if (n < (1 << 14)) return 4;
   const bool few = nsrc >= 2 && n >= (1 << 15);
-  if (!flat) return few || n >= (1 << 20) ? 2 : 3;
+  if (!flat) return fit_log2(n, few || n >= (1 << 20) ? 2 : 3);
   if (n >= (periodic ? 1 << 19 : (nsrc >= 2 ? 1 << 17 : 1 << 18))) return 0;
   return few || n >= (1 << 17) ? 2 : 3;
 }

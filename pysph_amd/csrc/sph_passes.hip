@@ -683,6 +683,10 @@ using namespace sph;
 
 extern "C" {
 
+int32_t sph_pass_lanes(int64_t n, int32_t nsrc, int32_t dim, int32_t periodic) {
+  return 1 << group_log2(n, nsrc, dim < 3, periodic != 0);
+}
+
 int32_t sph_density_rate(void* stream, const sph_grid* g, const sph_params* prm,
                          const sph_view* dst, int32_t nsrc, const sph_view* srcs, double rmax,
                          const float* disp_dev, void* rate_dev) {

@@ -190,3 +190,26 @@ def test_compute_without_gpu_fails_loudly():
     from pysph_amd._device import GPURequired
     with pytest.raises(GPURequired):
         particles.cell_manager.update()
+
+
+def test_pass_lanes_fit_a_launch():
+    """Lanes per destination of the SoA passes: a launch of n destinations
+    stays below 2^32 threads up to the largest array (2^31 - 1)."""
+    lanes = _abi.load().sph_pass_lanes
+    for nsrc in (1, 2):
+        for dim in (1, 2, 3):
+            for periodic in (0, 1):
+                last = 16
+                for e in range(0, 32):
+                    for n in (2 ** e - 1, 2 ** e, 2 ** e + 1):
+                        if not 0 < n < 2 ** 31:
+                            continue
+                        k = lanes(n, nsrc, dim, periodic)
+                        assert k in (1, 2, 4, 8, 16) and k <= last
+                        last = k
+                        block = 256 // k
+                        assert (n + block - 1) // block * 256 < 2 ** 32
+    assert [lanes(n, 1, 3, 0) for n in (100, 1 << 14, 1 << 20)] == [16, 8, 4]
+    assert [lanes(n, 1, 2, 0) for n in ((1 << 18) - 1, 1 << 18)] == [4, 1]
+    assert [lanes(n, 2, 2, 0) for n in ((1 << 17) - 1, 1 << 17)] == [4, 1]
+    assert [lanes(n, 1, 2, 1) for n in ((1 << 19) - 1, 1 << 19)] == [4, 1]
