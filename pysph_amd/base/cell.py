@@ -55,6 +55,13 @@ def construct_immediate_neighbor_list(cell_id, include_self=True, distance=1):
     return out
 
 
+# limits of a grid: cell coordinates of its lower corner, cells along an axis,
+# cells in all
+GRID_MAX_OFFSET = 2**30
+GRID_MAX_DIM = 2**20
+GRID_MAX_CELLS = 2**31 - 2
+
+
 def grid_for_domain(lo, hi, cell_size, slack=2):
     """Cell grid covering [lo, hi] with `slack` spare cells on each side.
     An axis on which the domain has no extent (z of a 2D set) gets a single
@@ -66,10 +73,10 @@ def grid_for_domain(lo, hi, cell_size, slack=2):
         s = 0 if lo[d] == hi[d] else slack
         c0 = math.floor(lo[d] / cs) - s
         c1 = math.floor(hi[d] / cs) + s
-        g.lo[d] = int(max(min(c0, 2**30), -2**30))
-        g.dims[d] = int(max(1, min(c1 - c0 + 1, 2**20)))
+        g.lo[d] = int(max(min(c0, GRID_MAX_OFFSET), -GRID_MAX_OFFSET))
+        g.dims[d] = int(max(1, min(c1 - c0 + 1, GRID_MAX_DIM)))
     ncells = g.dims[0] * g.dims[1] * g.dims[2]
-    if ncells > 2**31 - 2:
+    if ncells > GRID_MAX_CELLS:
         raise MemoryError("cell grid of %d cells is too large" % ncells)
     return g
 
@@ -216,18 +223,25 @@ class CellManager:
         """Bins per reference cell of a grid over [lo, hi]: two, unless that
         makes more than AUTO_BINS_PER_PARTICLE bins per particle (sparse
         domains, where counting and scanning the bins would cost more than
-        the candidates they save).  Bins of half the search radius leave 1.6
-        candidates per neighbour, bins of the radius 3 to 6 (density of 4.2M
-        random points: 864 against 700 us)."""
+        the candidates they save) or a grid beyond grid_for_domain's limits,
+        whose border bins would collect the particles past them.  Bins of
+        half the search radius leave 1.6 candidates per neighbour, bins of
+        the radius 3 to 6 (density of 4.2M random points: 864 against 780
+        us)."""
         if self._bins_fixed:
             return self.bins_per_cell
         cs = (self.cell_size or 1.0) / 2
         bins = 1.0
         for d in range(3):
+            if max(abs(lo[d]), abs(hi[d])) / cs >= GRID_MAX_OFFSET - 4 * self.grid_slack:
+                return 1
             if hi[d] > lo[d]:
-                bins *= (hi[d] - lo[d]) / cs + 4 * self.grid_slack + 2
+                along = (hi[d] - lo[d]) / cs + 4 * self.grid_slack + 2
+                if along > GRID_MAX_DIM:
+                    return 1
+                bins *= along
         n = self.get_number_of_particles()
-        return 2 if bins <= self.AUTO_BINS_PER_PARTICLE * n + 32768 else 1
+        return 2 if bins <= min(self.AUTO_BINS_PER_PARTICLE * n + 32768, GRID_MAX_CELLS) else 1
 
     @property
     def bin_size(self):
