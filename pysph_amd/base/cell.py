@@ -218,6 +218,8 @@ class CellManager:
 
     # bins per particle up to which auto_bins halves the cells
     AUTO_BINS_PER_PARTICLE = 8
+    # how far past that line the present grid's choice holds
+    AUTO_BINS_KEEP = 1.5
 
     def auto_bins(self, lo, hi):
         """Bins per reference cell of a grid over [lo, hi]: two, unless that
@@ -227,7 +229,9 @@ class CellManager:
         whose border bins would collect the particles past them.  Bins of
         half the search radius leave 1.6 candidates per neighbour, bins of
         the radius 3 to 6 (density of 4.2M random points: 864 against 780
-        us)."""
+        us).  The present grid's bins are kept while their number is within
+        a factor of that line (AUTO_BINS_KEEP), so that bounds that come and
+        go around it do not make a new grid each time."""
         if self._bins_fixed:
             return self.bins_per_cell
         cs = (self.cell_size or 1.0) / 2
@@ -241,7 +245,11 @@ class CellManager:
                     return 1
                 bins *= along
         n = self.get_number_of_particles()
-        return 2 if bins <= min(self.AUTO_BINS_PER_PARTICLE * n + 32768, GRID_MAX_CELLS) else 1
+        line = self.AUTO_BINS_PER_PARTICLE * n + 32768
+        if self.grid is not None and self.grid.bins_per_cell in (1, 2):
+            line *= self.AUTO_BINS_KEEP if self.grid.bins_per_cell == 2 else \
+                1.0 / self.AUTO_BINS_KEEP
+        return 2 if bins <= min(line, GRID_MAX_CELLS) else 1
 
     @property
     def bin_size(self):

@@ -50,3 +50,28 @@ def test_cells_far_from_the_origin(at):
     assert g.bins_per_cell == 1
     assert g.lo[0] <= at and at + 100 < g.lo[0] + g.dims[0]
     assert cell.GRID_MAX_OFFSET > abs(at) > cell.GRID_MAX_OFFSET / 2
+
+
+def test_bounds_around_the_line_keep_the_grid():
+    """A sparse set whose bounds swing around the line between one and two
+    bins a cell: the grid made first still covers them, with either choice,
+    until they are well past the line."""
+    n = 1000
+    line = cell.CellManager.AUTO_BINS_PER_PARTICLE * n + 32768
+    edge = 0.5 * (math.sqrt(line) - 10)          # 2D, 2 (edge + 5) bins an axis
+    near, far = 0.97 * edge, 1.03 * edge
+    for first, k in ((near, 2), (far, 1)):
+        cm = _manager(n)
+        cm.grid = cm.make_grid((0, 0, 0), (first, first, 0))
+        assert cm.grid.bins_per_cell == k
+        for hi in (far, near, far, near):
+            # (grown bounds need a larger grid, but not other bins)
+            g = cm.make_grid((0, 0, 0), (hi, hi, 0))
+            assert g.bins_per_cell == k
+            assert cm._covers(cm.grid, g) or hi > first + 1
+    cm = _manager(n)
+    cm.grid = cm.make_grid((0, 0, 0), (near, near, 0))
+    assert cm.make_grid((0, 0, 0), (1.3 * edge, 1.3 * edge, 0)).bins_per_cell == 1
+    cm.grid = cm.make_grid((0, 0, 0), (far, far, 0))
+    cm.grid.bins_per_cell = 1
+    assert cm.make_grid((0, 0, 0), (0.75 * edge, 0.75 * edge, 0)).bins_per_cell == 2
