@@ -106,9 +106,10 @@ class WCSPHPlan:
         self.list_skin = 0.0
         # stage2_rebin: re-bin the moving array by X1 before stage 2 (the
         # reference rebuilds its caches after the predictor).  Off, stage 2
-        # keeps the stage-1 binning and the passes widen their stencil by the predictor's largest displacement (measured on the
-        # device by the stage-1 kernel), which skips one binning and
-        # permutation per step; the neighbour sets are the same.
+        # keeps the stage-1 binning and the passes widen their stencil by the
+        # predictor's largest displacement (measured on the device by the
+        # stage-1 kernel), which skips one binning and permutation per step;
+        # the neighbour sets are the same.
         self.stage2_rebin = False
         # cache_static (opt-in): the density of a non-moving array keeps the
         # partial sums of its non-moving sources (boundary from boundary)
@@ -136,8 +137,8 @@ class WCSPHPlan:
         # the packed passes bin on a grid DEFAULT_CELLS_PER_RADIUS times
         # finer than the reference's cells (cell_size, cell ids and the jump
         # tolerance keep the reference's cell): fewer candidates per
-        # neighbour, the same neighbour sets
-        self.cells_per_radius = self.cm.bins_per_cell
+        # neighbour, the same neighbour sets; others leave it to the cell
+        # manager (CellManager.auto_bins)
         if self.use_packed:
             self.set_cells_per_radius(self.DEFAULT_CELLS_PER_RADIUS)
         # use_graph: step() replays captured HIP graphs where the step allows
@@ -169,7 +170,12 @@ class WCSPHPlan:
         """Bins of the shared CellManager's grid per reference cell (k = 1:
         the reference's cells)."""
         self.cm.set_cells_per_radius(k)
-        self.cells_per_radius = k
+
+    @property
+    def cells_per_radius(self):
+        """Bins per reference cell of the present grid (before the first
+        binning, where nothing set them: 1)."""
+        return self.cm.bins_per_cell
 
     # ----------------------------------------------------------------- match
     @classmethod

@@ -213,3 +213,19 @@ def test_pass_lanes_fit_a_launch():
     assert [lanes(n, 1, 2, 0) for n in ((1 << 18) - 1, 1 << 18)] == [4, 1]
     assert [lanes(n, 2, 2, 0) for n in ((1 << 17) - 1, 1 << 17)] == [4, 1]
     assert [lanes(n, 1, 2, 1) for n in ((1 << 19) - 1, 1 << 19)] == [4, 1]
+
+
+@pytest.mark.parametrize("precision,first", [("double", 1), ("single", 2)])
+def test_plan_reports_the_present_grids_bins(precision, first):
+    f, b, info = solver.generators.dam_break_2d(width=0.05, height=0.05, dx=0.01,
+                                                precision=precision)
+    particles = base.Particles([f, b])
+    s = solver.wcsph_solver(2, co=info["co"], ro=1000.0, alpha=0.1)
+    s.setup_integrator(particles)
+    plan = s.integrator.plan
+    assert plan.cells_per_radius == first
+    # what a binning on a grid of other bins leaves
+    particles.cell_manager.bins_per_cell = 3 - first
+    assert plan.cells_per_radius == 3 - first
+    plan.set_cells_per_radius(4)
+    assert plan.cells_per_radius == 4 == particles.cell_manager.bins_per_cell
