@@ -147,6 +147,9 @@ class CellManager:
         self.async_bounds = True
         self._jump_read = None
         self._jump_seen = 0
+        # the largest move of a step that reached the host with the jump
+        # count (move_word)
+        self.last_move = None
         self._bounds_read = None
         # buffers of the read-backs of replayed steps, used again once a read
         # was taken (others return theirs: most managers bin a few times)
@@ -557,7 +560,7 @@ class CellManager:
             # accumulated on the device; "deferred" reads it in
             # verify_jumps(), True also asynchronously after every binning
             if self._jump_acc is None or self._jump_acc.device != dev:
-                self._jump_acc = torch.zeros(1, dtype=torch.int32, device=dev)
+                self._jump_acc = torch.zeros(2, dtype=torch.int32, device=dev)
             _abi.call("sph_jump_check", stream, v, float(self.cell_size or 1.0), ref.data_ptr(),
                       self._jump_acc.data_ptr())
             if self.check_jumps is True and self._jump_read is None and not self.capturing:
@@ -593,6 +596,16 @@ class CellManager:
         _abi.call("sph_jump_check", require_gpu(pos[0]), v, float(self.cell_size or 1.0),
                   pa.__dict__["_refcell"].data_ptr(), self._jump_acc.data_ptr())
 
+    def move_word(self):
+        """An FP32 word beside the device jump count, read back with it: a
+        fused step records its largest displacement there, which arrives in
+        last_move.  None where no count is read back (check_jumps is not
+        True, periodic axes, nothing binned yet)."""
+        if self.check_jumps is not True or self.periodic_domain is not None or \
+                self._jump_acc is None:
+            return None
+        return self._jump_acc[1:].view(torch.float32)
+
     def _poll_jumps(self, wait):
         """Raise when the device jump count (read back asynchronously, or
         waited for) has grown since it was last seen."""
@@ -602,6 +615,7 @@ class CellManager:
         if v is None:
             return
         self._jump_read = None
+        self.last_move = float(v[1:].view(np.float32)[0])
         nj = int(v[0])
         if nj > self._jump_seen:
             self._jump_seen = nj
@@ -615,7 +629,7 @@ class CellManager:
         one cell between two binnings (waits for the device count)."""
         self._jump_read = None
         if self._jump_acc is not None and self.check_jumps:
-            nj = int(self._jump_acc.item())
+            nj = int(self._jump_acc[0].item())
             if nj > self._jump_seen:
                 self._jump_seen = nj
                 raise _abi.JumpToleranceError(

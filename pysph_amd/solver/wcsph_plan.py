@@ -109,8 +109,10 @@ class WCSPHPlan:
         # keeps the stage-1 binning and the passes widen their stencil by the
         # predictor's largest displacement (measured on the device by the
         # stage-1 kernel), which skips one binning and permutation per step;
-        # the neighbour sets are the same.
+        # the neighbour sets are the same.  FP64 steps re-bin all the same
+        # while particles move far (_note_moves).
         self.stage2_rebin = False
+        self._far_steps = 0
         # cache_static (opt-in): the density of a non-moving array keeps the
         # partial sums of its non-moving sources (boundary from boundary)
         # between calls while neither is re-binned (same bits, fewer pairs
@@ -276,7 +278,46 @@ class WCSPHPlan:
                 "alt": [mk() for _ in range(12)],
                 "disp": torch.zeros(1, dtype=torch.float32, device=pa.device),
             }
+            self._bufs["own_disp"] = self._bufs["disp"]
+        if not self.use_packed:
+            # recorded where it is read back (_note_moves)
+            word = self.cm.move_word()
+            if word is None:
+                word = self._bufs["own_disp"]
+            if word.data_ptr() != self._bufs["disp"].data_ptr():
+                self._bufs["disp"] = word
         return self._bufs
+
+    # FP64 steps keep the stage-1 binning in stage 2 while the largest move
+    # of a step is below this share of the reference's cell.  Widening every
+    # stencil by it costs what one binning saves: a step of the 3D dam break of
+    # 60k + 15k particles takes 638 us re-binned and 615 / 636 / 686 / 811 /
+    # 1091 us kept at moves of 0 / 0.1 / 0.25 / 0.5 / 1 cell, in 2D (30k) 212 and
+    # 187 / 188 / 192 / 198 / 210.  Steps of the CFL condition stay near 0.02.
+    KEEP_MOVE = 0.1
+    # steps that re-bin after one that moved farther: a new mode captures the
+    # step anew
+    FAR_STEPS = 64
+
+    def _note_moves(self):
+        """Decide from the last move that reached the host (with the jump
+        count, a few steps late) whether the next FP64 steps re-bin."""
+        move = self.cm.last_move
+        if self._far_steps:
+            self._far_steps -= 1
+        if move is not None and not move <= self.KEEP_MOVE * self.cm.cell_size:
+            self._far_steps = self.FAR_STEPS
+
+    def _keeps_binning(self):
+        """Whether stage 2 runs on the stage-1 binning."""
+        if self.use_list:
+            # lists built anew in stage 2 need the X1 binning (their validity
+            # check reads the same displacement as the widened stencil)
+            return self.list_reuse
+        if self.stage2_rebin or self.cm.periodic_domain is not None:
+            # periodic positions are wrapped at a binning, so X1 gets one
+            return False
+        return self.use_packed or (self.cm.check_jumps is True and self._far_steps == 0)
 
     # ------------------------------------------------------ packed copies
     # FP32 storage: every array carries float4 copies (x,y,z,h), (u,v,w,m),
@@ -497,13 +538,7 @@ class WCSPHPlan:
         b = self._buffers()
         self._pack_all()
         ov = self._override()
-        # lists built anew in stage 2 need the X1 binning (their validity
-        # check reads the same displacement as the widened stencil); periodic
-        # positions are wrapped at a binning, so X1 gets one there
-        keep_binning = (self.use_list and self.list_reuse) or (
-            not self.stage2_rebin and not self.use_list and
-            self.cm.periodic_domain is None)
-        if keep_binning:
+        if self._keeps_binning():
             # stage 2 keeps the binning: the stage-1 kernel records the
             # predictor's largest displacement on the device, and the stage-2
             # passes widen their stencil by it; with reused lists, stage 1
@@ -535,7 +570,12 @@ class WCSPHPlan:
             # of each stage records the neighbours its momentum pass reads
             self._density(override=ov, list_mode=0)
             probe("density1", b, ov)
-            self._stage(1, dt, b, override=ov)
+            disp = None
+            if self._far_steps:
+                # still recorded: it tells when the binning can be kept again
+                disp = b["disp"]
+                _abi.call("sph_fill_i32", require_gpu(disp), disp.data_ptr(), 1, 0)
+            self._stage(1, dt, b, override=ov, disp_out=disp)
             probe("stage1", b, ov)
             self.rebin_stage(b)
             s1 = self._s1_fields(b)
@@ -596,7 +636,8 @@ class WCSPHPlan:
         """What a captured step bakes in besides buffers and the grid: the
         time step, the parameters and the plan's switches."""
         return (float(dt), bytes(self.prm), bytes(self.flags), self.fused_density,
-                self.concurrent_density, self.use_packed, self.stage2_rebin)
+                self.concurrent_density, self.use_packed, self._keeps_binning(),
+                self._far_steps > 0)
 
     def _eager_step(self, dt, euler=False):
         if euler:
@@ -613,6 +654,7 @@ class WCSPHPlan:
         steps, after a grid change or any change of the arrays' buffers)."""
         cm = self.cm
         n0 = self.steps
+        self._note_moves()
         if not self.graph_applies():
             self._sg.drop()
             self._eager_step(dt, euler)

@@ -153,6 +153,59 @@ def test_fp64_stage_2_on_the_stage_1_binning_counts_jumps_at_the_predictor():
         assert rel_norm(a, b) < 1e-12
 
 
+@pytest.mark.parametrize("use_graph", [False, True])
+def test_fp64_steps_with_a_fast_particle_rebin_in_stage_2(use_graph):
+    """A particle that moves 0.3 cells a step, alone above the others: the
+    steps re-bin in stage 2 instead of widening every stencil by its move,
+    keep the stage-1 binning again some steps after it has slowed down, and
+    agree with steps that always re-bin (other order of the sums: 1e-12)."""
+    from pysph_amd.solver import generators as gen
+    out = []
+    for rebin in (False, True):
+        f, _, info = gen.elliptical_drop_2d(2000, precision="double")
+        particles = base.Particles([f])
+        cm = particles.cell_manager
+        s = solver.wcsph_solver(2, co=info["co"], ro=1.0, alpha=0.1, with_solid=False)
+        s.setup_integrator(particles)
+        plan = s.integrator.plan
+        plan.stage2_rebin, plan.use_graph = rebin, use_graph
+
+        def steps(k):
+            n0, r0 = cm.num_binnings, plan.graph_replays
+            for _ in range(k):
+                s.integrator.integrate(info["dt"])
+                torch.cuda.synchronize()
+            return (cm.num_binnings - n0) / k, plan.graph_replays - r0
+
+        steps(4)
+        x, y, u, v = (f.get(c) for c in ("x", "y", "u", "v"))
+        x[7], y[7], u[7], v[7] = 0.0, y.max() + 50 * cm.cell_size, \
+            0.3 * cm.cell_size / info["dt"], 0.0
+        f.set(x=x, y=y, u=u, v=v)
+        cm.verify_jumps = lambda: 0
+        cm._jump_seen = 1 << 30  # the particle was put there
+        steps(6)
+        per, replays = steps(20)
+        if not rebin:
+            assert not plan._keeps_binning() and cm.last_move > 0.25 * cm.cell_size
+        if use_graph:
+            assert replays > 0 and plan.graph_error is None
+        else:
+            assert per == 2
+        u = f.get("u")
+        u[7] = 0.0
+        f.set(u=u)
+        steps(plan.FAR_STEPS + 12)
+        per, _ = steps(4)
+        if not rebin:
+            assert plan._keeps_binning() and cm.last_move < 0.1 * cm.cell_size
+        if not use_graph:
+            assert per == (2 if rebin else 1)
+        out.append([f.get(c) for c in ("x", "y", "u", "v", "rho", "p")])
+    for a, b in zip(*out):
+        assert rel_norm(a, b) < 1e-12
+
+
 @pytest.mark.parametrize("n,dim,h", [(1, 2, 0.1), (65, 3, 0.2), (3000, 2, 0.15), (3000, 3, 0.25),
                                      (17000, 2, 0.06), (17000, 3, 0.03)])
 @pytest.mark.parametrize("shuffled", [False, True])
