@@ -317,3 +317,48 @@ def test_2d_sets_match_reference_cpp_nnps(precision):
     for a, b in zip(csr_sorted_rows(off, nb), ref):
         assert np.array_equal(a, b)
     assert off[-1] > 5 * len(x)
+
+
+@pytest.mark.parametrize("piece", [8, 8 * 4096, 8 * 50001, 1 << 20])
+def test_lists_above_the_limit_are_ordinary_memory(monkeypatch, piece):
+    """Neighbour lists up to a size are page-locked, larger ones ordinary
+    arrays copied in pieces (whole and partial last ones, fewer than two), and
+    where no memory can be locked the lists come all the same."""
+    import torch
+    from pysph_amd.base import nnps
+    rng = np.random.Generator(np.random.PCG64(4))
+    n = 500 if piece == 8 else 3000
+    a = base.get_particle_array(name="a", x=rng.random(n), y=rng.random(n), h=np.full(n, 0.04))
+    particles = base.Particles([a])
+    cm = particles.cell_manager
+    off, nb = nnps.neighbor_csr(cm, a, a, 2.0)
+    assert torch.from_numpy(nb).is_pinned() and torch.from_numpy(off).is_pinned()
+    monkeypatch.setattr(nnps._HostCopy, "PINNED_MAX", 8 * n)
+    monkeypatch.setattr(nnps._HostCopy, "PIECE", piece)
+    off2, nb2 = nnps.neighbor_csr(cm, a, a, 2.0)
+    assert not torch.from_numpy(nb2).is_pinned() and not torch.from_numpy(off2).is_pinned()
+    assert np.array_equal(off, off2) and np.array_equal(nb, nb2)
+    monkeypatch.setattr(nnps, "_pinned", lambda n, dtype: None)
+    for limit in (8 * n, 1 << 30):
+        monkeypatch.setattr(nnps._HostCopy, "PINNED_MAX", limit)
+        off3, nb3 = nnps.neighbor_csr(cm, a, a, 2.0)
+        assert np.array_equal(off, off3) and np.array_equal(nb, nb3)
+
+
+def test_a_locator_lets_go_of_its_lists_before_the_next(monkeypatch):
+    from pysph_amd.base import nnps
+    a = base.get_particle_array(name="a", x=[0.0, 0.1], h=[0.2, 0.2])
+    particles = base.Particles([a])
+    loc = particles.nnps_manager.get_neighbor_particle_locator(a, a, 2.0)
+    off, nb = loc.get_csr()
+    real, seen = nnps.neighbor_csr, []
+
+    def csr(*args, **kw):
+        seen.append((loc._off, loc._nbr))
+        return real(*args, **kw)
+    monkeypatch.setattr(nnps, "neighbor_csr", csr)
+    a.set_dirty(True)
+    off2, nb2 = loc.get_csr()
+    assert seen == [(None, None)]
+    # lists a caller holds stay what they were
+    assert off.tolist() == off2.tolist() == [0, 2, 4] and nb.tolist() == nb2.tolist()
