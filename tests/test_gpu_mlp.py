@@ -196,7 +196,7 @@ def test_adam_steps_reduce_the_loss():
 @pytest.mark.parametrize("width,height", [(0.01, 0.01), (0.02, 0.03), (0.05, 0.07), (0.3, 0.43)])
 def test_gradients_at_chunk_remainders(width, height):
     """Weight and bias gradients where the node count leaves remainders of
-    the 32-row steps, the 64-row bias blocks and the 256-row chunks (one
+    the 32-row steps, the 64-row bias blocks and the chunks of up to 256 rows (one
     chunk of a few rows up to several chunks), each tensor against the
     BF16-rounded oracle.  Biases and non-negative H x H weights keep every ReLU
     active, so that no unit near zero is masked on one side only (one such unit of one node is worth
@@ -232,13 +232,23 @@ def test_gradients_at_chunk_remainders(width, height):
 
 DEGREES = [[0], [1], [0, 0, 0, 0, 0], [32], [0, 33, 0], [1, 0, 31, 32, 33, 0, 64, 65, 2, 96, 0],
            [21] * 9, [65, 1] * 20, [40] * 3 + [0] + [7] * 4099]
+# more than two nodes for each of the forward kernel's 4096 waves (the backward
+# kernel's 2048), counts mixed so that waves pass from every kind of node to
+# every other
+DEGREES.append(np.random.Generator(np.random.PCG64(8)).choice(
+    [0, 1, 2, 31, 32, 33, 64, 65], 9500).tolist())
+
+
+def _graph_for(degrees):
+    """A graph with at least as many nodes as there are degrees."""
+    return _graph(*((0.2, 0.3) if len(degrees) < 1000 else (0.8, 1.2)))[0]
 
 
 def _set_edges(g, degrees):
     """Give the graph's first nodes these edge counts, with nearby nodes as
     neighbours (repeated ones are edges of their own)."""
-    degrees = degrees[:g.n]
     n = len(degrees)
+    assert n <= g.n
     rng = np.random.Generator(np.random.PCG64(n))
     dst = np.repeat(np.arange(n), degrees)
     nbr = np.clip(dst + rng.integers(-9, 10, len(dst)), 0, n - 1)
@@ -254,11 +264,11 @@ def _set_edges(g, degrees):
 def test_edge_blocks_and_node_runs(degrees):
     """The matrix-core edge aggregation on given edge counts (none, whole and
     partial blocks of 32, several blocks; fewer nodes than waves up to several
-    nodes per wave) against the FP32 vector-unit one on the same graph.  What
+    nodes per wave, which a wave passes between in every combination) against the FP32 vector-unit one on the same graph.  What
     differs is the split-BF16 products (2^-16) and BF16 copies of the
     aggregate that round the other way (2^-8 of a value, on a share of about
     2^-7 of them): below 1e-3, as in the test above."""
-    g, _ = _graph()
+    g = _graph_for(degrees)
     keep = _set_edges(g, degrees)
     model = EdgeMLP(params=_params(5))
     y = model.forward(g)[:g.n].double().cpu().numpy()
@@ -277,7 +287,7 @@ def test_edge_backward_blocks_and_node_runs(degrees):
     copies of dP and dQ round the other way; feature and mask products are
     exact: below 1e-3."""
     from pysph_amd import _abi
-    g, _ = _graph()
+    g = _graph_for(degrees)
     keep = _set_edges(g, degrees)
     model = EdgeMLP(params=_params(6))
     rng = np.random.Generator(np.random.PCG64(len(degrees)))
