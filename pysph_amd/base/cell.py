@@ -12,6 +12,7 @@ The cell of a particle is the reference's floor(x/cell_size)
 The cell size follows compute_cell_size (cell.pyx:893-925).
 """
 import math
+import struct
 
 import numpy as np
 import torch
@@ -147,9 +148,7 @@ class CellManager:
         self.async_bounds = True
         self._jump_read = None
         self._jump_seen = 0
-        # the largest move of a step that reached the host with the jump
-        # count (move_word)
-        self.last_move = None
+        self._move_bits = None
         self._bounds_read = None
         # buffers of the read-backs of replayed steps, used again once a read
         # was taken (others return theirs: most managers bin a few times)
@@ -237,22 +236,23 @@ class CellManager:
         go around it do not make a new grid each time."""
         if self._bins_fixed:
             return self.bins_per_cell
-        cs = (self.cell_size or 1.0) / 2
+        per_cs = 2.0 / (self.cell_size or 1.0)
+        spare = 4 * self.grid_slack
         bins = 1.0
-        for d in range(3):
-            if max(abs(lo[d]), abs(hi[d])) / cs >= GRID_MAX_OFFSET - 4 * self.grid_slack:
+        for a, b in zip(lo, hi):
+            if b * per_cs >= GRID_MAX_OFFSET - spare or a * per_cs <= spare - GRID_MAX_OFFSET:
                 return 1
-            if hi[d] > lo[d]:
-                along = (hi[d] - lo[d]) / cs + 4 * self.grid_slack + 2
+            if b > a:
+                along = (b - a) * per_cs + spare + 2
                 if along > GRID_MAX_DIM:
                     return 1
                 bins *= along
-        n = self.get_number_of_particles()
-        line = self.AUTO_BINS_PER_PARTICLE * n + 32768
-        if self.grid is not None and self.grid.bins_per_cell in (1, 2):
-            line *= self.AUTO_BINS_KEEP if self.grid.bins_per_cell == 2 else \
-                1.0 / self.AUTO_BINS_KEEP
-        return 2 if bins <= min(line, GRID_MAX_CELLS) else 1
+        line = self.AUTO_BINS_PER_PARTICLE * self.get_number_of_particles() + 32768
+        if bins > line / self.AUTO_BINS_KEEP:
+            now = 0 if self.grid is None else self.grid.bins_per_cell
+            if now == 1 or bins > (line * self.AUTO_BINS_KEEP if now == 2 else line):
+                return 1
+        return 2 if bins <= GRID_MAX_CELLS else 1
 
     @property
     def bin_size(self):
@@ -606,6 +606,14 @@ class CellManager:
             return None
         return self._jump_acc[1:].view(torch.float32)
 
+    @property
+    def last_move(self):
+        """The move_word of the last read-back that reached the host (None:
+        none has)."""
+        if self._move_bits is None:
+            return None
+        return struct.unpack("f", struct.pack("i", self._move_bits))[0]
+
     def _poll_jumps(self, wait):
         """Raise when the device jump count (read back asynchronously, or
         waited for) has grown since it was last seen."""
@@ -615,8 +623,7 @@ class CellManager:
         if v is None:
             return
         self._jump_read = None
-        self.last_move = float(v[1:].view(np.float32)[0])
-        nj = int(v[0])
+        nj, self._move_bits = v.tolist()
         if nj > self._jump_seen:
             self._jump_seen = nj
             raise _abi.JumpToleranceError(

@@ -302,6 +302,8 @@ class WCSPHPlan:
     def _note_moves(self):
         """Decide from the last move that reached the host (with the jump
         count, a few steps late) whether the next FP64 steps re-bin."""
+        if self.use_packed:
+            return
         move = self.cm.last_move
         if self._far_steps:
             self._far_steps -= 1
@@ -636,8 +638,8 @@ class WCSPHPlan:
         """What a captured step bakes in besides buffers and the grid: the
         time step, the parameters and the plan's switches."""
         return (float(dt), bytes(self.prm), bytes(self.flags), self.fused_density,
-                self.concurrent_density, self.use_packed, self._keeps_binning(),
-                self._far_steps > 0)
+                self.concurrent_density, self.use_packed, self.stage2_rebin,
+                self._keeps_binning(), self._far_steps > 0)
 
     def _eager_step(self, dt, euler=False):
         if euler:
