@@ -1399,7 +1399,7 @@ static int32_t ensure(Buf& b, size_t bytes) {
 static int nblk(int64_t n) { return (int)((n + 255) / 256); }
 
 // Persistent edge aggregation: up to SPH_EDGE_WAVES waves per SIMD of the
-// 256 CUs, each wave then walking nodes with stride gridDim.x * 4.
+// 256 CUs; a block's four waves take the nodes of its run (node_run) in turn.
 static int edge_fwd_blocks(int64_t n) {
   const int64_t waves = std::min<int64_t>(n, 256 * 4 * SPH_EDGE_WAVES);
   return (int)std::max<int64_t>(1, (waves + 3) / 4);
@@ -1435,9 +1435,10 @@ static GemmArgs gargs(int M, int N, int K, const __bf16* A, int64_t lda, const _
   return a;
 }
 
-// Row chunks of a weight gradient: enough blocks for the 256 CUs (four tiles
-// of 128 x 64 per matrix), each with at least 256 rows so that a slab's
-// 128 KB of output stays small against the rows it reads.
+// Row chunks of a weight gradient: at most 256 rows each while that makes up
+// to 64 of them, enough blocks for the 256 CUs (four tiles of 128 x 64 per
+// matrix), longer ones after that: a slab's 128 KB of output stays small
+// against the rows it reads.
 static int grad_splits(int rows) { return std::max(1, std::min(64, (rows + 255) / 256)); }
 
 // Weight gradient G[kdim x ncols] += X^T D with X [rows x kdim] (ldx), D
@@ -1728,7 +1729,7 @@ int32_t sph_mlp_forward(void* model, void* stream, const sph_mlp_graph* gr, floa
     e.A = HA + kH;
     e.lda = 2 * kH;
     T.begin(2);
-    // the MFMA kernel indexes Q rows with 32-bit offsets (n * 2 * kH < 2^31)
+    // the MFMA kernel addresses Q rows by 32-bit byte offsets (n * 8 kH < 2^32)
     if (SPH_EDGE_MFMA && !(gr->flags & SPH_MLP_EDGE_FP32) && n < (int64_t(1) << 22))
       hipLaunchKernelGGL(edge_fwd_mfma_kernel, dim3(edge_fwd_blocks(n)), dim3(256), 0, st, e, e.off);
     else
