@@ -58,10 +58,9 @@ __device__ __forceinline__ void axis_span(float v, float r, int c, int n, int lo
   b = min((int)fb - c, ring);
 }
 
-// Particle range of the cells of grid row (y, z) within the stencil ring of
-// cell column cx whose extent can hold a point within the cull radius.
-// The cell-start indices [k0, k1] (read cstart[k0] and cstart[k1]) of that
-// range; false when the row holds no candidate cell.
+// Cells of grid row (y, z) within the stencil ring of cell column cx whose
+// extent can hold a point within the cull radius, as cell-start indices
+// [k0, k1] (read cstart[k0] and cstart[k1]); false when there is none.
 __device__ __forceinline__ bool row_cells_cull(const Grid& g, int cx, int y, int z, int ring,
                                                const Cull& cu, int& k0, int& k1) {
   if (y < 0 || y >= g.dims[1] || z < 0 || z >= g.dims[2]) return false;
@@ -69,7 +68,10 @@ __device__ __forceinline__ bool row_cells_cull(const Grid& g, int cx, int y, int
   const float gz = axis_gap(cu.zd, z, g.dims[2], g.lo[2], g.cs_f);
   const float w2 = cu.rc2 - gy * gy - gz * gz;
   if (!(w2 >= 0.f)) return false;
+  // 1-ulp hardware square root: the cull radius carries a 1e-5 margin
   const float w = __builtin_amdgcn_sqrtf(w2);
+  // cells of [x - w, x + w]; the border cells reach to infinity (particles
+  // outside the grid are clamped into them), so clamp the range into the grid
   const float last = (float)(g.dims[0] - 1);
   const float fa = fminf(fmaxf(floorf((cu.xd - w) * g.inv_cs_f) - (float)g.lo[0], 0.f), last);
   const float fb = fminf(fmaxf(floorf((cu.xd + w) * g.inv_cs_f) - (float)g.lo[0], 0.f), last);
@@ -83,29 +85,15 @@ __device__ __forceinline__ bool row_cells_cull(const Grid& g, int cx, int y, int
   return true;
 }
 
+// The particle range [j0, j1) of those cells (empty when there is none).
 __device__ __forceinline__ void row_range_cull(const Grid& g, const int* __restrict__ cstart,
                                                int cx, int y, int z, int ring, const Cull& cu,
                                                int& j0, int& j1) {
   j0 = j1 = 0;
-  if (y < 0 || y >= g.dims[1] || z < 0 || z >= g.dims[2]) return;
-  const float gy = axis_gap(cu.yd, y, g.dims[1], g.lo[1], g.cs_f);
-  const float gz = axis_gap(cu.zd, z, g.dims[2], g.lo[2], g.cs_f);
-  const float w2 = cu.rc2 - gy * gy - gz * gz;
-  if (!(w2 >= 0.f)) return;
-  // 1-ulp hardware square root: the cull radius carries a 1e-5 margin
-  const float w = __builtin_amdgcn_sqrtf(w2);
-  // cells of [x - w, x + w]; the border cells reach to infinity (particles
-  // outside the grid are clamped into them), so clamp the range into the grid
-  const float last = (float)(g.dims[0] - 1);
-  const float fa = fminf(fmaxf(floorf((cu.xd - w) * g.inv_cs_f) - (float)g.lo[0], 0.f), last);
-  const float fb = fminf(fmaxf(floorf((cu.xd + w) * g.inv_cs_f) - (float)g.lo[0], 0.f), last);
-  int x0 = max(cx - ring, 0), x1 = min(cx + ring, g.dims[0] - 1);
-  if (fa > (float)x1 || fb < (float)x0) return;  // NaN positions keep the ring
-  if (fa > (float)x0) x0 = (int)fa;
-  if (fb < (float)x1) x1 = (int)fb;
-  const int base = (z * g.dims[1] + y) * g.dims[0];
-  j0 = cstart[base + x0];
-  j1 = cstart[base + x1 + 1];
+  int k0, k1;
+  if (!row_cells_cull(g, cx, y, z, ring, cu, k0, k1)) return;
+  j0 = cstart[k0];
+  j1 = cstart[k1];
 }
 
 }  // namespace sph

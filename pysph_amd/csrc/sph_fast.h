@@ -1259,17 +1259,7 @@ __device__ __forceinline__ void momentum_small_body(const Grid& g, const PassArg
   }
   float disp = 0.f;
   if (valid && gr.rank == 0) disp = mom_epilogue<float, MODE>(a, i, local, acc, dv, D.vd);
-  if (MODE != 0 && a.disp_out != nullptr) {
-    // one atomic per block at most
-    for (int off = 32; off > 0; off >>= 1) disp = fmaxf(disp, __shfl_xor(disp, off, 64));
-    __shared__ float bmax[kBlock / 64];
-    if ((threadIdx.x & 63) == 0) bmax[threadIdx.x >> 6] = disp;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int k = 1; k < kBlock / 64; ++k) disp = fmaxf(disp, bmax[k]);
-      raise_max(a.disp_out, disp);
-    }
-  }
+  if (MODE != 0 && a.disp_out != nullptr) block_raise_max(a.disp_out, disp);
 }
 
 }  // namespace sph

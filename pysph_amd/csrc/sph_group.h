@@ -102,6 +102,20 @@ struct Group {
   }
 };
 
+// The largest of a block's move bounds (all lanes of all waves) into *disp_out
+// by one atomic at most: the atomics go to one address, and one per wave made
+// the FP64 stage of 5k particles 24 us instead of 12.
+__device__ __forceinline__ void block_raise_max(float* disp_out, float disp) {
+  __shared__ float bmax[kBlock / 64];
+  for (int o = 32; o > 0; o >>= 1) disp = fmaxf(disp, __shfl_xor(disp, o, 64));
+  if ((threadIdx.x & 63) == 0) bmax[threadIdx.x >> 6] = disp;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < kBlock / 64; ++k) disp = fmaxf(disp, bmax[k]);
+    raise_max(disp_out, disp);
+  }
+}
+
 // Shift of image code c along the three axes: digits 0, 1, 2 (base 3) stand
 // for 0, +1 and -1 periods.
 __device__ __forceinline__ double image_shift(int digit, double period) {

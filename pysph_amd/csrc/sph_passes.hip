@@ -389,20 +389,7 @@ __global__ __launch_bounds__(kBlock) void momentum_kernel(Grid g, PassArgs<T> a,
     const double mv = (double)xn - (double)x0;
     mv2 += mv * mv;
   }
-  // block maximum, then at most one atomic per block (the atomics go to one
-  // address: one per wave made this launch 24 us instead of 12 on 5k
-  // particles with 16 lanes each)
-  if (a.disp_out != nullptr) {
-    float disp = move_bound(mv2);
-    for (int off = 32; off > 0; off >>= 1) disp = fmaxf(disp, __shfl_xor(disp, off, 64));
-    __shared__ float bmax[kBlock / 64];
-    if ((threadIdx.x & 63) == 0) bmax[threadIdx.x >> 6] = disp;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int k = 1; k < kBlock / 64; ++k) disp = fmaxf(disp, bmax[k]);
-      raise_max(a.disp_out, disp);
-    }
-  }
+  if (a.disp_out != nullptr) block_raise_max(a.disp_out, move_bound(mv2));
 }
 
 template <typename T>
