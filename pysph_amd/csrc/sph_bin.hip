@@ -420,12 +420,14 @@ __global__ __launch_bounds__(kBlock) void bin_rank(int n, const int* __restrict_
 }
 
 // The whole binning of a small set in one block: counts and cell starts in
-// LDS, the members of a cell ranked by their slots.  The general path's eight
-// launches (two fills, count, three scans, scatter, rank) take 26 us and as
-// many gaps on 2k to 5k particles, this one 6 to 11.  Each thread keeps its (at
-// most kTinyPer) particles' cells in registers; cell c's count is at
-// c + c / 32, so that threads scanning 32 consecutive cells each use
-// different banks.
+// LDS, the members of a cell ranked by their slots among those of the same
+// 1024 particles (among all of them, 8192 particles in one cell took 3.1 ms
+// and in 16 cells 222 us; the general path 624 and 96 us; now 415 and 44).
+// The general path's eight launches (two fills, count, three scans, scatter,
+// rank) take 26 us and as many gaps on 2k to 5k particles, this one 6 to 11.
+// Each thread keeps its (at most kTinyPer) particles' cells in registers;
+// cell c's count is at c + c / 32, so that threads scanning 32 consecutive
+// cells each use different banks.
 constexpr int kTinyBlock = 1024;
 constexpr int kTinyPer = 8;
 constexpr int kTinyN = kTinyBlock * kTinyPer;   // 8192 particles
@@ -448,7 +450,7 @@ __global__ __launch_bounds__(kTinyBlock) void bin_tiny(View<T> a, BinGrid g, int
   const int chunks = (ncells + kTinyChunk) / kTinyChunk;  // covers ncells + 1 entries
   for (int c = t; c < chunks * kTinyChunk; c += kTinyBlock) count[tiny_at(c)] = 0;
   __syncthreads();
-  int cell[kTinyPer], pos[kTinyPer];
+  int cell[kTinyPer], pos[kTinyPer], base[kTinyPer], upto[kTinyPer];
 #pragma unroll
   for (int k = 0; k < kTinyPer; ++k) {
     const int i = t + k * kTinyBlock;
@@ -458,9 +460,20 @@ __global__ __launch_bounds__(kTinyBlock) void bin_tiny(View<T> a, BinGrid g, int
       const int cy = grid_coord((double)a.y[i], g.cs, g.lo[1], g.dims[1]);
       const int cz = grid_coord((double)a.z[i], g.cs, g.lo[2], g.dims[2]);
       cell[k] = (cz * g.dims[1] + cy) * g.dims[0] + cx;
-      pos[k] = atomicAdd(&count[tiny_at(cell[k])], 1);
       if (prev_cell != nullptr && bin_jumped(g, prev_cell[i], cx, cy, cz)) atomicAdd(jumps, 1);
     }
+  }
+  // turn after turn, so that a cell's members of a turn (1024 consecutive
+  // particles) have the places base .. upto - 1, in any order
+#pragma unroll
+  for (int k = 0; k < kTinyPer; ++k) {
+    if (k * kTinyBlock >= a.n) break;
+    int* p = &count[tiny_at(cell[k] < 0 ? 0 : cell[k])];
+    base[k] = *p;
+    __syncthreads();
+    if (cell[k] >= 0) pos[k] = atomicAdd(p, 1);
+    __syncthreads();
+    upto[k] = *p;
   }
   __syncthreads();
   // exclusive scan: 32 consecutive cells per thread
@@ -490,9 +503,9 @@ __global__ __launch_bounds__(kTinyBlock) void bin_tiny(View<T> a, BinGrid g, int
   for (int k = 0; k < kTinyPer; ++k) {
     if (cell[k] < 0) continue;
     const int me = t + k * kTinyBlock;
-    const int s = count[tiny_at(cell[k])], e = count[tiny_at(cell[k] + 1)];
-    int rank = 0;
-    for (int q = s; q < e; ++q) rank += bucket[q] < me ? 1 : 0;
+    const int s = count[tiny_at(cell[k])];
+    int rank = base[k];
+    for (int q = base[k]; q < upto[k]; ++q) rank += bucket[s + q] < me ? 1 : 0;
     perm[s + rank] = me;
     cell_out[s + rank] = cell[k];
   }
