@@ -895,8 +895,10 @@ __global__ __launch_bounds__(kBlock) void nbr_count_kernel(Grid g, NbrArgs<T> a)
 
 // Lanes per destination (log2) of the groups, 0: nbr_count_kernel.  Counting
 // costs little beside a group's rows and ballots, so one lane pays from 2^17
-// particles on in flat sets (one layer of bins) and, in FP32, whose pairs are
-// half the bytes, from 2^19 in 3D.  In us, 1 / 4 / 8 lanes:
+// particles on in flat sets (one layer of bins; 2^15 with one row of them)
+// and, in FP32, whose pairs are half the bytes, from 2^19 in 3D.  In us, 1 / 4
+// / 8 lanes:
+//   1D FP64  20k: 5 / - / 6   50k: 5 / - / 8   100k: 6 / - / 11
 //   2D FP32  100k: 18 / 16 / 16   200k: 23 / 24 / 27   1M: 73 / 90 / 112
 //            4M: 257 / 342 / 431   (FP64: 381 / 395 / 504)
 //   3D FP32  200k: 99 / 102 / 91   400k: 164 / 175 / 168   1M: 351 / 406 / 400
@@ -910,8 +912,9 @@ static int nbr_log2(const Grid& G, const NbrArgs<T>& a, bool fill) {
   const int64_t n = a.dst.n;
   const bool flat = G.dims[2] == 1;
   if (n < (1 << 14)) return 4;
-  if (!fill && a.rmax_sym <= 0 && (flat ? n >= (1 << 17) : sizeof(T) == 4 && n >= (1 << 19)))
-    return 0;
+  const int64_t alone = flat ? (G.dims[1] == 1 ? 1 << 15 : 1 << 17)
+                             : (sizeof(T) == 4 ? 1 << 19 : INT64_MAX);
+  if (!fill && a.rmax_sym <= 0 && n >= alone) return 0;
   if (flat) return fit_log2(n, n >= (1 << 17) ? 2 : 3);
   return fit_log2(n, !fill && a.rmax_sym <= 0 && n >= (1 << 19) ? 2 : 3);
 }

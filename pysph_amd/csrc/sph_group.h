@@ -38,20 +38,22 @@ inline int fit_log2(int64_t n, int k) {
 // Two sources cull every row twice, which fewer groups per wave make dearer: 4
 // lanes once the waves suffice (dam break of 60k + 15k, FP64 momentum: 146 /
 // 171 / 213 us; density 66 / 68 / 76).  Once the waves fill the GPU without
-// groups, their rows, queues and ballots cost more than they save, sooner on
-// `flat` sets (1D and 2D: few rows and pairs a destination) and with two
-// sources, later on periodic ones, whose images the groups share out.
+// groups, their rows, queues and ballots cost more than they save, sooner in
+// 1D and 2D (few rows and pairs a destination) and with two sources, later on
+// periodic sets, whose images the groups share out.
 // Density + rate + momentum in FP64, 1 (plain loops) / 4 / 8 lanes, in us:
+//   1D  20k: 58 / - / 52   50k: 63 / - / 66   100k: 68 / - / 98
 //   2D  100k: 218 / 159 / 169   200k: 289 / 275   300k: 374 / 395 / 457
 //       1M: 961 / 1257 / 1511   4M: 3438 / 5562 / 6644
 //   2D periodic  300k: 519 / 461 / 534   1M (FP32): 922 / 1018 / 1230
 //   2D dam break, a step  150k: 415 / 446   300k: 590 / 742   2M: 2416 (8: 4390)
 //   3D  300k: 1343 / 1016 / 1034   1M: 3782 / 3364 / 3568   4M: 15877 / 14477 / 15467
 //       (clustered 1M: 6365 / 5444 / 5014, so 8 lanes up to there)
-inline int group_log2(int64_t n, int nsrc, bool flat, bool periodic) {
+inline int group_log2(int64_t n, int nsrc, int dim, bool periodic) {
   if (n < (1 << 14)) return 4;
+  if (dim == 1) return n >= (1 << 15) ? 0 : 3;
   const bool few = nsrc >= 2 && n >= (1 << 15);
-  if (!flat) return fit_log2(n, few || n >= (1 << 20) ? 2 : 3);
+  if (dim == 3) return fit_log2(n, few || n >= (1 << 20) ? 2 : 3);
   if (n >= (periodic ? 1 << 19 : (nsrc >= 2 ? 1 << 17 : 1 << 18))) return 0;
   return few || n >= (1 << 17) ? 2 : 3;
 }

@@ -446,7 +446,7 @@ static void launch_density_s(hipStream_t st, const Grid& G, const PassArgs<T>& a
 
 template <typename T, typename CT, bool TAIT>
 static void launch_density_t(hipStream_t st, const Grid& G, const PassArgs<T>& a) {
-  const int k = group_log2(a.dst.n, a.nsrc, a.dim < 3, G.periodic);
+  const int k = group_log2(a.dst.n, a.nsrc, a.dim, G.periodic);
   if (k == 0)
     launch_density_s<T, CT, TAIT, kAlone>(st, G, a, k);
   else if (a.disp != nullptr || a.cache_src >= 0)
@@ -474,7 +474,7 @@ static void launch_rate_s(hipStream_t st, const Grid& G, const PassArgs<T>& a, i
 
 template <typename T, typename CT>
 static void launch_rate(hipStream_t st, const Grid& G, const PassArgs<T>& a) {
-  const int k = group_log2(a.dst.n, a.nsrc, a.dim < 3, G.periodic);
+  const int k = group_log2(a.dst.n, a.nsrc, a.dim, G.periodic);
   if (k == 0)
     launch_rate_s<T, CT, kAlone>(st, G, a, k);
   else
@@ -503,7 +503,7 @@ static void launch_momentum_s(hipStream_t st, const Grid& G, const PassArgs<T>& 
 
 template <typename T, typename CT>
 static void launch_momentum(hipStream_t st, const Grid& G, const PassArgs<T>& a, int mode) {
-  const int k = group_log2(a.dst.n, a.nsrc, a.dim < 3, G.periodic);
+  const int k = group_log2(a.dst.n, a.nsrc, a.dim, G.periodic);
   if (G.periodic) {
     if (k == 0) launch_momentum_s<T, CT, true, kAlone>(st, G, a, mode, k);
     else launch_momentum_s<T, CT, true, kQueued>(st, G, a, mode, k);
@@ -671,7 +671,7 @@ using namespace sph;
 extern "C" {
 
 int32_t sph_pass_lanes(int64_t n, int32_t nsrc, int32_t dim, int32_t periodic) {
-  return 1 << group_log2(n, nsrc, dim < 3, periodic != 0);
+  return 1 << group_log2(n, nsrc, dim, periodic != 0);
 }
 
 int32_t sph_density_rate(void* stream, const sph_grid* g, const sph_params* prm,

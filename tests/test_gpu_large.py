@@ -1,6 +1,6 @@
 """The SoA passes and neighbour counts where large sets leave the groups of lanes: one lane per
-destination from 2^18 particles on in 1D and 2D (2^17 with two sources, 2^19
-with periodic axes), fewer lanes from 2^17 (2D) and 2^20 (3D) on, against the FP64 oracle on the same stored bits; plain,
+destination from 2^15 particles on in 1D and 2^18 in 2D (2^17 with two
+sources, 2^19 with periodic axes), fewer lanes from 2^17 (2D) and 2^20 (3D) on, against the FP64 oracle on the same stored bits; plain,
 periodic and symmetric variable-h sets.  FP64 within 1e-12 (sums of at most
 1e3 terms, as in test_gpu_group.py)."""
 import numpy as np
@@ -26,7 +26,7 @@ def _set(n, dim, nbrs, seed, vary=0.0, precision="double"):
     vel = rng.normal(size=(3, n))
     pos[dim:] = 0.0
     vel[dim:] = 0.0
-    vol = np.pi if dim == 2 else 4.0 / 3.0 * np.pi
+    vol = {1: 2.0, 2: np.pi, 3: 4.0 / 3.0 * np.pi}[dim]
     h = 0.5 * (nbrs / (vol * n)) ** (1.0 / dim)
     return base.get_particle_array(
         name="s", type=Fluid, cl_precision=precision, x=pos[0], y=pos[1], z=pos[2], u=vel[0], v=vel[1], w=vel[2],
@@ -44,13 +44,15 @@ def _oracle_threads():
 @pytest.mark.parametrize("n,dim,kind", [
     ((1 << 17) - 1, 2, "plain"), (1 << 17, 2, "plain"), ((1 << 18) - 1, 2, "plain"),
     (1 << 18, 2, "plain"), (1 << 18, 2, "periodic"), (1 << 18, 2, "varh"),
-    ((1 << 17) - 1, 2, "two"), (1 << 17, 2, "two"), (1 << 19, 2, "periodic"),
+    ((1 << 15) - 1, 1, "plain"), (1 << 15, 1, "plain"), (1 << 15, 1, "periodic"),
+    (1 << 15, 1, "varh"), ((1 << 17) - 1, 2, "two"), (1 << 17, 2, "two"), (1 << 19, 2, "periodic"),
     (1 << 20, 3, "plain")])
 def test_sums_where_the_lanes_change(n, dim, kind):
     a = _set(n, dim, 15, 3, 0.5 if kind == "varh" else 0.0)
     dom = None
     if kind == "periodic":
-        dom = base.PeriodicDomain(xmin=0.0, xmax=1.0, ymin=0.0, ymax=1.0)
+        dom = base.PeriodicDomain(xmin=0.0, xmax=1.0,
+                                  **({} if dim == 1 else dict(ymin=0.0, ymax=1.0)))
     b = [_set(n // 3, dim, 15, 4)] if kind == "two" else []
     for pa in b:
         pa.set(h=np.full(n // 3, a.get("h")[0]))
@@ -63,7 +65,8 @@ def test_sums_where_the_lanes_change(n, dim, kind):
     ao = to_oracle(a)
     src = [ao] + [to_oracle(pa, 1) for pa in b]
     if kind == "periodic":
-        src[0], _ = O.with_ghosts(ao, (1.0, 1.0, 0.0), (0.0, 0.0, 0.0), cs, cs)
+        src[0], _ = O.with_ghosts(ao, (1.0, 1.0 if dim > 1 else 0.0, 0.0), (0.0, 0.0, 0.0), cs,
+                                  cs)
     kw = dict(cell_size=cs, varh=kind == "varh")
     F, G = [Fluid], [Solid] if b else []
     op = solver.SPHOperation(sph.SPHRho.withargs(), on_types=F, from_types=F + G, updates=["rho"],
@@ -86,7 +89,8 @@ def test_sums_where_the_lanes_change(n, dim, kind):
 @pytest.mark.parametrize("n,dim,kind,precision", [
     ((1 << 17) - 1, 2, "plain", "single"), (1 << 17, 2, "plain", "single"),
     (1 << 17, 2, "plain", "double"), (1 << 17, 2, "periodic", "single"),
-    (1 << 17, 2, "varh", "double"), ((1 << 19) - 1, 3, "plain", "single"),
+    (1 << 17, 2, "varh", "double"), ((1 << 15) - 1, 1, "plain", "double"),
+    (1 << 15, 1, "plain", "double"), (1 << 15, 1, "periodic", "double"), ((1 << 19) - 1, 3, "plain", "single"),
     (1 << 19, 3, "plain", "single"), (1 << 19, 3, "plain", "double")])
 @pytest.mark.parametrize("bins", [1, 2])
 def test_counts_where_the_lanes_change(n, dim, kind, precision, bins):
@@ -94,7 +98,8 @@ def test_counts_where_the_lanes_change(n, dim, kind, precision, bins):
     a = _set(n, dim, 15, 5, 0.5 if kind == "varh" else 0.0, precision)
     dom = None
     if kind == "periodic":
-        dom = base.PeriodicDomain(xmin=0.0, xmax=1.0, ymin=0.0, ymax=1.0)
+        dom = base.PeriodicDomain(xmin=0.0, xmax=1.0,
+                                  **({} if dim == 1 else dict(ymin=0.0, ymax=1.0)))
     particles = base.Particles([a], variable_h=kind == "varh", periodic_domain=dom)
     cm = particles.cell_manager
     cm.set_cells_per_radius(bins)
@@ -102,7 +107,8 @@ def test_counts_where_the_lanes_change(n, dim, kind, precision, bins):
     ao = to_oracle(a)
     src = ao
     if kind == "periodic":
-        src, _ = O.with_ghosts(ao, (1.0, 1.0, 0.0), (0.0, 0.0, 0.0), cm.cell_size, cm.cell_size)
+        src, _ = O.with_ghosts(ao, (1.0, 1.0 if dim > 1 else 0.0, 0.0), (0.0, 0.0, 0.0),
+                               cm.cell_size, cm.cell_size)
     off, _ = O.nnps_csr(ao, src, cell_size=cm.cell_size, varh=kind == "varh")
     v = a.view()
     counts = torch.empty(n, dtype=torch.int64, device=a.device)

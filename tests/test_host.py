@@ -210,6 +210,7 @@ def test_pass_lanes_fit_a_launch():
                         block = 256 // k
                         assert (n + block - 1) // block * 256 < 2 ** 32
     assert [lanes(n, 1, 3, 0) for n in (100, 1 << 14, 1 << 20)] == [16, 8, 4]
+    assert [lanes(n, 1, 1, 0) for n in ((1 << 15) - 1, 1 << 15)] == [8, 1]
     assert [lanes(n, 1, 2, 0) for n in ((1 << 18) - 1, 1 << 18)] == [4, 1]
     assert [lanes(n, 2, 2, 0) for n in ((1 << 17) - 1, 1 << 17)] == [4, 1]
     assert [lanes(n, 1, 2, 1) for n in ((1 << 19) - 1, 1 << 19)] == [4, 1]
