@@ -152,14 +152,18 @@ __device__ __forceinline__ float fsqrt<float>(float x) {
   return __builtin_amdgcn_sqrtf(x);
 }
 
-// Branch-free cubic spline shape W(q) (kernels.pyx:367-374).
+// Branch-free cubic spline shape W(q) (kernels.pyx:367-374); t = 2 - q.
 template <typename CT>
-__device__ __forceinline__ CT w_sel(CT q) {
+__device__ __forceinline__ CT w_sel(CT q, CT t) {
 #pragma clang fp contract(off)
-  const CT t = CT(2) - q;
   const CT outer = CT(0.25) * t * t * t;
   const CT inner = fma_(CT(-1.5) * (q * q), fma_(CT(-0.5), q, CT(1)), CT(1));
   return q > CT(2) ? CT(0) : (q > CT(1) ? outer : inner);
+}
+
+template <typename CT>
+__device__ __forceinline__ CT w_sel(CT q) {
+  return w_sel<CT>(q, CT(2) - q);
 }
 
 // Branch-free gradient factor (kernels.pyx:403-412): grad W = r_ab * g.
@@ -837,6 +841,8 @@ __device__ __forceinline__ PairTerms<float> mom_terms_u(const MomDst<float>& D, 
   const float rs = __builtin_amdgcn_rsqf(d2);
   const float rr = d2 > 0.f ? d2 * rs : 0.f;  // the self pair: r = 0, not 0 * inf
   const float qq = rr * U.inv;
+  // 2 - r / h_ab: one rounding where both sums share it
+  const float t = DM && DX ? fma_(-U.inv, rr, 2.f) : 2.f - qq;
   const float mb = vs.w;
   const float rhob = as.x;
   const float irhoab = frcp<float>(0.5f * (D.rhoa + rhob));
@@ -850,13 +856,12 @@ __device__ __forceinline__ PairTerms<float> mom_terms_u(const MomDst<float>& D, 
     const float mu = U.hab * dot * frcp<float>(d2 + U.eta2hh);
     const float piab = fma_(D.beta * mu, mu, -D.alpha * cab * mu) * irhoab;
     const float tmp = D.Aa + Ab + (dot < 0.f ? piab : 0.f);
-    const float t = 2.f - qq;
     const float outer = U.kout * (t * t) * rs;
     const float inner = U.kin * fma_(0.75f, qq, -1.f);
     const float gfac = qq > 2.f ? 0.f : (qq >= 1.f ? outer : (qq > 1e-14f ? inner : 0.f));
     T.gf = -mb * tmp * gfac;
   }
-  if (DX) T.temp = mb * (w_sel<float>(qq) * U.fac) * irhoab;
+  if (DX) T.temp = mb * (w_sel<float>(qq, t) * U.fac) * irhoab;
   return T;
 }
 
@@ -1224,8 +1229,15 @@ __device__ __forceinline__ void momentum_small_body(const Grid& g, const PassArg
         if (k < count) {
           const int j = q[k];
           const float4 ps = ld4(S.pos4, j), vs = ld4(S.vel4, j), as = ld4(S.aux4, j);
-          T = uni ? mom_terms_u<true, true>(D, U, ps, vs, as)
-                  : mom_terms_r<float, true, true>(D, ps, vs, as);
+          // a source's roles are part of a pair's rounding (mom_terms_u)
+          if (!uni)
+            T = mom_terms_r<float, true, true>(D, ps, vs, as);
+          else if (do_m && do_x)
+            T = mom_terms_u<true, true>(D, U, ps, vs, as);
+          else if (do_m)
+            T = mom_terms_u<true, false>(D, U, ps, vs, as);
+          else
+            T = mom_terms_u<false, true>(D, U, ps, vs, as);
         }
         float* tp = terms + gr.rank * kTermPitch;
         tp[0] = T.gf;

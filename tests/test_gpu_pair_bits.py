@@ -1,8 +1,9 @@
 """The rounding of the packed FP32 pair arithmetic, pinned bit for bit.
 
 |r|^2 is fma(z, z, fma(x, x, y * y)) and (v . r) is fma(vz, z, fma(vx, x,
-vy * y)) in every packed kernel: results stay what they were to the last bit
-when a kernel is rewritten.  The hardware's square root and reciprocals have
+vy * y)) in every packed kernel, and 2 - r / h is one fma where a source of
+uniform h feeds both the momentum and the XSPH sum: results stay what they
+were to the last bit when a kernel is rewritten.  The hardware's square root and reciprocals have
 no host equivalent, so a pair is compared with another pair that gives the
 same rounded |r|^2 (or v . r) from one component alone: everything after it
 is the same arithmetic on the same bits."""
@@ -71,12 +72,12 @@ def _first(pa, t):
     return a[0] if o is None else a[np.flatnonzero(o == 0)[0]]
 
 
-def _pass(kind, src, uniform, pad):
+def _pass(kind, src, uniform, pad, flags=_abi.SPH_SRC_MOMENTUM, h=1.0):
     """The first output(s) of a destination at the origin at rest, with the
-    source particle src = (x, y, u, v)."""
-    D = _array("d", 0.0, 0.0, 0.0, 0.0, pad, (1.0, 1.0))
+    source particle src = (x, y, u, v) of roles `flags`."""
+    D = _array("d", 0.0, 0.0, 0.0, 0.0, pad, (h, h))
     # one far source of another h: the source's h is not uniform then
-    S = _array("s", *src, 0 if uniform else 1, (1.0, 1.0 if uniform else 0.9))
+    S = _array("s", *src, 0 if uniform else 1, (h, h if uniform else 0.9 * h))
     cm = base.CellManager(arrays_to_bin=[D, S])
     cm.check_jumps = False
     cm.update()
@@ -94,8 +95,8 @@ def _pass(kind, src, uniform, pad):
         aux[:] = torch.tensor([1000.0, 10.0, 3e-6, 3.0], device=pa.device)
         ov[id(pa)]["aux4"] = aux
     acc, dv = [mk() for _ in range(3)], [mk() for _ in range(3)]
-    _ops.momentum_xsph(cm, prm, D, [S], [_abi.SPH_SRC_MOMENTUM], acc=acc, dv=dv, override=ov)
-    return [_first(D, t) for t in acc]
+    _ops.momentum_xsph(cm, prm, D, [S], [flags], acc=acc, dv=dv, override=ov)
+    return [_first(D, t) for t in acc + dv]
 
 
 def _square_of(v):
@@ -138,6 +139,36 @@ def test_velocity_product(groups, uniform):
     for x, y, u, v, p, q in _samples(16, make):
         got = _pass("momentum", (x, y, -u, -v), uniform, pad)
         want = _pass("momentum", (x, y, -p, 0), uniform, pad)
-        assert got[0] != 0 and got == want, (x, y, u, v, got, want)
-        told += want != _pass("momentum", (x, y, -q, 0), uniform, pad)
+        assert got[0] != 0 and got[:3] == want[:3], (x, y, u, v, got, want)
+        told += want[:3] != _pass("momentum", (x, y, -q, 0), uniform, pad)[:3]
     assert told >= 4
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+def test_roles_and_groups(uniform):
+    """A pair's momentum and XSPH terms for a source of both roles, of one
+    role, from groups of lanes and from one lane per destination.  Groups and
+    scans agree bit for bit in every role.  With a uniform h that is no power
+    of two, 2 - r / h of the outer gradient branch is one fma for a source of
+    both roles and a rounded quotient for one of momentum alone: apart in some
+    pairs, by what a half last bit of r / h below 2 is of (2 - r / h)^3 at the
+    largest r / h, 3 * 2^-24 / (2 - 1.93) = 2.6e-6, and twice that of the other
+    roundings beside it."""
+    M, X = _abi.SPH_SRC_MOMENTUM, _abi.SPH_SRC_XSPH
+    rng = np.random.Generator(np.random.PCG64(5))
+    apart = 0
+    for _ in range(24):
+        a = rng.uniform(0, 2 * np.pi)
+        r = rng.uniform(0.75, 1.35)  # q from 1.07 to 1.93
+        src = (F(r * np.cos(a)), F(r * np.sin(a)), F(rng.uniform(-1, 1)), F(rng.uniform(-1, 1)))
+        out = {}
+        for flags in (M, X, M | X):
+            out[flags] = _pass("momentum", src, uniform, 0, flags, 0.7)
+            scan = _pass("momentum", src, uniform, SCAN_MIN["momentum"], flags, 0.7)
+            assert out[flags] == scan, (flags, src)
+        both, mom, xs = np.array(out[M | X]), np.array(out[M]), np.array(out[X])
+        assert np.all(mom[3:] == 0) and np.all(xs[:3] == 0) and both[0] != 0 and both[3] != 0
+        assert np.allclose(both[:3], mom[:3], rtol=5e-6, atol=0)
+        assert np.allclose(both[3:], xs[3:], rtol=5e-6, atol=0)
+        apart += np.any(both[:3] != mom[:3])
+    assert apart >= 4 if uniform else apart == 0
